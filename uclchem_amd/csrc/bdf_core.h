@@ -34,6 +34,19 @@
 #define BDF_HD inline
 #include <cmath>
 #endif
+// The control state is the same in every lane.  On the GPU its values are produced by FP64
+// vector instructions; uni() moves them to scalar registers, so that the state costs no vector
+// registers across the phases of a step and its branches are scalar.
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __forceinline__ double bdf_uni(double v)
+{
+    const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
+    const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
+    return __hiloint2double(hi, lo);
+}
+#else
+BDF_HD double bdf_uni(double v) { return v; }
+#endif
 
 namespace bdf {
 
@@ -86,64 +99,90 @@ BDF_HD double powi(double x, int k)
     return r;
 }
 
+// by-value select: with the operands loaded first, two loads are not merged into one from a
+// computed address, which would put the array into scratch memory
+BDF_HD double sel(bool c, double a, double b) { return c ? a : b; }
+// a[i] with a run-time index but compile-time storage (the arrays stay in registers)
+BDF_HD double pick(const double *a, int n, int i)
+{
+    double v = a[0];
+#pragma unroll
+    for (int k = 1; k < n; k++) v = sel(i == k, a[k], v);
+    return v;
+}
+
 // BDF coefficients l[] and test constants tq[] for order q with step history tau[].
 BDF_HD void set_bdf(State &s)
 {
     const int q = s.q;
     double alpha0, alpha0_hat, xi_inv, xistar_inv, hsum;
-    for (int i = 0; i <= QMAX; i++) s.l[i] = 0.0;
-    s.l[0] = s.l[1] = xi_inv = xistar_inv = 1.0;
+    double l[QMAX + 1];
+#pragma unroll
+    for (int i = 0; i <= QMAX; i++) l[i] = 0.0;
+    l[0] = l[1] = xi_inv = xistar_inv = 1.0;
     alpha0 = alpha0_hat = -1.0;
     hsum = s.h;
     if (q > 1) {
-        for (int j = 2; j < q; j++) {
-            hsum += s.tau[j - 1];
-            xi_inv = s.h / hsum;
-            alpha0 -= 1.0 / j;
-            for (int i = j; i >= 1; i--) s.l[i] += s.l[i - 1] * xi_inv;
+#pragma unroll
+        for (int j = 2; j < QMAX; j++) {
+            if (j < q) {
+                hsum += s.tau[j - 1];
+                xi_inv = s.h / hsum;
+                alpha0 -= 1.0 / j;
+#pragma unroll
+                for (int i = j; i >= 1; i--) l[i] += l[i - 1] * xi_inv;
+            }
         }
         alpha0 -= 1.0 / q;
-        xistar_inv = -s.l[1] - alpha0;
-        hsum += s.tau[q - 1];
+        xistar_inv = -l[1] - alpha0;
+        hsum += pick(s.tau, QMAX + 2, q - 1);
         xi_inv = s.h / hsum;
-        alpha0_hat = -s.l[1] - xi_inv;
-        for (int i = q; i >= 1; i--) s.l[i] += s.l[i - 1] * xistar_inv;
+        alpha0_hat = -l[1] - xi_inv;
+#pragma unroll
+        for (int i = QMAX; i >= 1; i--)
+            if (i <= q) l[i] += l[i - 1] * xistar_inv;
     }
     // error and convergence test constants
+    const double lq = pick(l, QMAX + 1, q);
     double A1 = 1.0 - alpha0_hat + alpha0;
     double A2 = 1.0 + q * A1;
-    s.tq[2] = dabs(A1 / (alpha0 * A2));
-    s.tq[5] = dabs(A2 * xistar_inv / (s.l[q] * xi_inv));
+    s.tq[2] = bdf_uni(dabs(A1 / (alpha0 * A2)));
+    s.tq[5] = bdf_uni(dabs(A2 * xistar_inv / (lq * xi_inv)));
     if (q > 1) {
-        double C = xistar_inv / s.l[q];
+        double C = xistar_inv / lq;
         double A3 = alpha0 + 1.0 / q;
         double A4 = alpha0_hat + xi_inv;
         double Cpinv = (1.0 - A4 + A3) / A3;
-        s.tq[1] = dabs(C * Cpinv);
-        hsum += s.tau[q];
+        s.tq[1] = bdf_uni(dabs(C * Cpinv));
+        hsum += pick(s.tau, QMAX + 2, q);
         xi_inv = s.h / hsum;
         double A5 = alpha0 - 1.0 / (q + 1);
         double A6 = alpha0_hat - xi_inv;
         double Cppinv = (1.0 - A6 + A5) / A2;
-        s.tq[3] = dabs(Cppinv / (xi_inv * (q + 2) * A5));
+        s.tq[3] = bdf_uni(dabs(Cppinv / (xi_inv * (q + 2) * A5)));
     }
-    s.tq[4] = NLSCOEF / s.tq[2];
+    s.tq[4] = bdf_uni(NLSCOEF / s.tq[2]);
+#pragma unroll
+    for (int i = 0; i <= QMAX; i++) s.l[i] = bdf_uni(l[i]);
 }
 
 // Nordsieck-array correction coefficients for an order change by +1 / -1.
 BDF_HD void increase_coeffs(const State &s, double *lc, double &A1)
 {
     const int q = s.q;
+#pragma unroll
     for (int i = 0; i <= QMAX; i++) lc[i] = 0.0;
     lc[2] = 1.0;
     double alpha1 = 1.0, prod = 1.0, xiold = 1.0, alpha0 = -1.0, hsum = s.hscale;
-    if (q > 1) {
-        for (int j = 1; j < q; j++) {
+#pragma unroll
+    for (int j = 1; j < QMAX - 1; j++) {   // an increase starts from order QMAX - 1 at most
+        if (j < q) {
             hsum += s.tau[j + 1];
             double xi = hsum / s.hscale;
             prod *= xi;
             alpha0 -= 1.0 / (j + 1);
             alpha1 += 1.0 / xi;
+#pragma unroll
             for (int i = j + 2; i >= 2; i--) lc[i] = lc[i] * xiold + lc[i - 1];
             xiold = xi;
         }
@@ -154,15 +193,27 @@ BDF_HD void increase_coeffs(const State &s, double *lc, double &A1)
 BDF_HD void decrease_coeffs(const State &s, double *lc)
 {
     const int q = s.q;
+#pragma unroll
     for (int i = 0; i <= QMAX; i++) lc[i] = 0.0;
     lc[2] = 1.0;
     double hsum = 0.0;
-    for (int j = 1; j <= q - 2; j++) {
-        hsum += s.tau[j];
-        double xi = hsum / s.hscale;
-        for (int i = j + 2; i >= 2; i--) lc[i] = lc[i] * xi + lc[i - 1];
+#pragma unroll
+    for (int j = 1; j <= QMAX - 2; j++) {
+        if (j <= q - 2) {
+            hsum += s.tau[j];
+            double xi = hsum / s.hscale;
+#pragma unroll
+            for (int i = j + 2; i >= 2; i--) lc[i] = lc[i] * xi + lc[i - 1];
+        }
     }
 }
+
+// one out-of-line power function for the step-size formulas
+#if defined(__HIP_DEVICE_COMPILE__)
+__device__ __attribute__((noinline)) double bdf_pow(double x, double y) { return pow(x, y); }
+#else
+BDF_HD double bdf_pow(double x, double y) { return pow(x, y); }
+#endif
 
 template <class Ops>
 BDF_HD void adjust_order(Ops &o, State &s, int dq)
@@ -173,10 +224,14 @@ BDF_HD void adjust_order(Ops &o, State &s, int dq)
         increase_coeffs(s, lc, A1);
         // zn[q+1] = A1 * saved acor (kept in zn[QMAX]); zn[j] += lc[j] * zn[q+1]
         o.scale_into_z(s.q + 1, A1, QMAX);
-        for (int j = 2; j <= s.q; j++) o.axpy_zz(j, lc[j], s.q + 1);
+#pragma unroll
+        for (int j = 2; j < QMAX; j++)
+            if (j <= s.q) o.axpy_zz(j, lc[j], s.q + 1);
     } else if (dq == -1) {
         decrease_coeffs(s, lc);
-        for (int j = 2; j < s.q; j++) o.axpy_zz(j, -lc[j], s.q);
+#pragma unroll
+        for (int j = 2; j < QMAX; j++)
+            if (j < s.q) o.axpy_zz(j, -lc[j], s.q);
     }
 }
 
@@ -184,7 +239,7 @@ template <class Ops>
 BDF_HD void rescale(Ops &o, State &s)
 {
     o.rescale_z(s.q, s.eta);
-    s.h = s.hscale * s.eta;
+    s.h = bdf_uni(s.hscale * s.eta);
     s.hscale = s.h;
 }
 
@@ -243,7 +298,7 @@ BDF_HD int nls(Ops &o, State &s, Stats &st, int nflag)
                 if (!s.jcur) { retry = true; break; }
                 return 1;
             }
-            if (m > 0) s.crate = dmax(CRDOWN * s.crate, del / delp);
+            if (m > 0) s.crate = bdf_uni(dmax(CRDOWN * s.crate, del / delp));
             double dcon = del * dmin(1.0, s.crate) / s.tq[4];
             if (dcon <= 1.0) {
                 s.acnrm = (m == 0) ? del : o.wrms(ACOR);
@@ -286,13 +341,13 @@ BDF_HD int step(Ops &o, State &s, Stats &st)
     }
     for (;;) {
         // predict
-        s.tn += s.h;
+        s.tn = bdf_uni(s.tn + s.h);
         o.predict(s.q);
         set_bdf(s);
-        s.rl1 = 1.0 / s.l[1];
-        s.gamma = s.h * s.rl1;
+        s.rl1 = bdf_uni(1.0 / s.l[1]);
+        s.gamma = bdf_uni(s.h * s.rl1);
         if (st.nst == 0) s.gammap = s.gamma;
-        s.gamrat = (st.nst > 0) ? s.gamma / s.gammap : 1.0;
+        s.gamrat = bdf_uni((st.nst > 0) ? s.gamma / s.gammap : 1.0);
 
         int r = nls(o, s, st, nflag);
         if (r < 0) {
@@ -320,7 +375,7 @@ BDF_HD int step(Ops &o, State &s, Stats &st)
         if (nef == MXNEF) return -4;
         s.etamax = 1.0;
         if (nef < MXNEF1) {
-            s.eta = 1.0 / (pow(BIAS2 * dsm, 1.0 / s.L) + ADDON);
+            s.eta = bdf_uni(1.0 / (bdf_pow(BIAS2 * dsm, 1.0 / s.L) + ADDON));
             s.eta = dmax(ETAMIN, s.eta);
             if (nef >= SMALL_NEF) s.eta = dmin(s.eta, ETAMXF);
             rescale(o, s);
@@ -337,7 +392,7 @@ BDF_HD int step(Ops &o, State &s, Stats &st)
         }
         // order 1 after repeated failures: shrink and restart the history from f
         s.eta = ETAMIN;
-        s.h *= s.eta;
+        s.h = bdf_uni(s.h * s.eta);
         s.hscale = s.h;
         s.qwait = LONG_WAIT;
         o.start_corrector();
@@ -348,7 +403,9 @@ BDF_HD int step(Ops &o, State &s, Stats &st)
     // complete the step
     st.nst++;
     s.nst_call++;
-    for (int i = s.q; i >= 2; i--) s.tau[i] = s.tau[i - 1];
+#pragma unroll
+    for (int i = QMAX; i >= 2; i--)
+        if (i <= s.q) s.tau[i] = s.tau[i - 1];
     if (s.q == 1 && st.nst > 1) s.tau[2] = s.tau[1];
     s.tau[1] = s.h;
     o.complete(s.q, s.l);
@@ -366,7 +423,7 @@ BDF_HD int step(Ops &o, State &s, Stats &st)
         s.etamax = (st.nst <= SMALL_NST) ? ETAMX2 : ETAMX3;
         return 0;
     }
-    s.etaq = 1.0 / (pow(BIAS2 * dsm, 1.0 / s.L) + ADDON);
+    s.etaq = bdf_uni(1.0 / (bdf_pow(BIAS2 * dsm, 1.0 / s.L) + ADDON));
     if (s.qwait != 0) {
         s.eta = s.etaq;
         s.qprime = s.q;
@@ -375,13 +432,13 @@ BDF_HD int step(Ops &o, State &s, Stats &st)
         s.etaqm1 = 0.0;
         if (s.q > 1) {
             double ddn = o.wrms(s.q) * s.tq[1];
-            s.etaqm1 = 1.0 / (pow(BIAS1 * ddn, 1.0 / s.q) + ADDON);
+            s.etaqm1 = bdf_uni(1.0 / (bdf_pow(BIAS1 * ddn, 1.0 / s.q) + ADDON));
         }
         s.etaqp1 = 0.0;
         if (s.q != QMAX) {
             double cquot = (s.tq[5] / s.saved_tq5) * powi(s.h / s.tau[2], s.L);
             double dup = o.wrms_acor_minus(cquot, QMAX) * s.tq[3];
-            s.etaqp1 = 1.0 / (pow(BIAS3 * dup, 1.0 / (s.L + 1)) + ADDON);
+            s.etaqp1 = bdf_uni(1.0 / (bdf_pow(BIAS3 * dup, 1.0 / (s.L + 1)) + ADDON));
         }
         double etam = dmax(s.etaqm1, dmax(s.etaq, s.etaqp1));
         if (etam < THRESH) {
@@ -404,8 +461,8 @@ BDF_HD int step(Ops &o, State &s, Stats &st)
         s.hprime = s.h;
         s.qprime = s.q;
     } else {
-        s.eta = dmin(s.eta, s.etamax);
-        s.hprime = s.h * s.eta;
+        s.eta = bdf_uni(dmin(s.eta, s.etamax));
+        s.hprime = bdf_uni(s.h * s.eta);
     }
     s.etamax = (st.nst <= SMALL_NST) ? ETAMX2 : ETAMX3;
     return 0;

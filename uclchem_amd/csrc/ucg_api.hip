@@ -189,7 +189,7 @@ size_t lds_bytes(const ucg::DevNet &N)
 {
     const int npad = (N.neq + 7) & ~7;
     const int region = ucg::flux_region_len(N);
-    return sizeof(double) * ((size_t)region + 4 * npad + 16 + ucg::S_NSCAL + ucg::P_NPARAM);
+    return sizeof(double) * ((size_t)region + 4 * npad + ucg::RED_LEN + ucg::S_NSCAL + ucg::P_NPARAM);
 }
 
 int ensure_ws(NetHandle &h, size_t bytes)

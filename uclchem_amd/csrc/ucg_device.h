@@ -20,6 +20,8 @@ namespace ucg {
 #define GLB __attribute__((address_space(1)))
 template <class T> __device__ __forceinline__ const GLB T *glb(const T *p) { return (const GLB T *)p; }
 template <class T> __device__ __forceinline__ GLB T *glbw(T *p) { return (GLB T *)p; }
+// constant-memory view of the network descriptor: its fields are always scalar loads
+#define CST __attribute__((address_space(4)))
 __device__ __forceinline__ int2 ld_int2(const GLB int *p, int i)
 {
     int2 r;
@@ -37,8 +39,12 @@ __device__ __forceinline__ int4 ld_int4(const GLB int *p, int i)
     return r;
 }
 
-constexpr int NT = 256;          // threads per workgroup (one workgroup solves one grid point)
-constexpr int EPT = 2;           // state elements owned per thread => NEQ <= 512
+// One workgroup solves one grid point.  Its phases are chains of dependent LDS and L2 accesses, so
+// a second wave on every SIMD hides what one wave waits for: 512 threads with one equation each
+// against 256 with two (default network, FP64, 8 grid points alone on the chip): RHS 26.3 -> 17.5
+// us a call, Jacobian 105 -> 68, factorisation 190 -> 157, solve 46 -> 33.
+constexpr int NT = 512;          // threads per workgroup
+constexpr int EPT = 1;           // state elements owned per thread => NEQ <= 512
 constexpr int JZ_LONG = 16;      // Jacobian entries with more contributions than this...
 constexpr int JZ_GROUP = 16;     // ...are summed by a group of this many lanes
 constexpr int MAXOPS = 6;
@@ -131,10 +137,23 @@ struct DevNet {
     const int8_t *nw_unscaled;   // [nval] 1 where the Newton matrix takes the J-form value without gamma
 };
 
+using NetRef = const CST DevNet &;
+// The descriptor with its address hidden from the optimiser.  Each phase of a step reads its
+// table pointers through its own copy: loads hoisted out of the integration loop would keep some
+// hundred pointers and per-lane addresses alive across every phase, and spill.
+__device__ __forceinline__ NetRef fresh(NetRef N)
+{
+    const uint64_t p = (uint64_t)(const CST void *)&N;
+    int lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)p), hi = __builtin_amdgcn_readfirstlane((int)(p >> 32));
+    asm volatile("" : "+s"(lo), "+s"(hi));
+    return *(const CST DevNet *)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+
 // LDS bytes the sparse solve stages: factors (lut bytes each; FP32 all of them, FP64 the
 // sparse part), column indices, row records, permutation, work vector and the dense-tail
 // product's scratch (16-byte aligned parts)
-__host__ __device__ inline int solve_stage_bytes(const DevNet &N, int lut)
+template <class Net>
+__host__ __device__ inline int solve_stage_bytes(const Net &N, int lut)
 {
     const int nst = lut == 4 ? N.nw_nval : N.nw_nsp;
     auto al = [](int x) { return (x + 15) & ~15; };
@@ -147,14 +166,15 @@ __host__ __device__ inline int solve_stage_bytes(const DevNet &N, int lut)
 // (all of them in FP32, the dense tail in FP64) plus the permuted work vector.  Plans too
 // large to stage (strongly coupled networks with a wide dense tail) keep their factors in
 // the workspace and need only the work vector here.
-__host__ __device__ inline int flux_region_len(const DevNet &N)
+template <class Net>
+__host__ __device__ inline int flux_region_len(const Net &N)
 {
     const int npad = (N.neq + 7) & ~7, Npad = (N.nw_N + 7) & ~7;
     const int a = N.npart_pad + 2 * npad;
     const int g = N.gt_off + N.ngt;                  // fluxes + chunk partial sums
     const int b0 = N.nreac > a ? N.nreac : a;
     const int b1 = b0 > g ? b0 : g;
-    const int b = b1 > 256 ? b1 : 256;               // >= one value per thread (ordered_sum)
+    const int b = b1 > NT ? b1 : NT;                 // >= one value per thread (ordered_sum)
     if (!N.nw_stage) return b > Npad ? b : Npad;               // unstaged plan: the work vector only
     const int t64 = N.nw_T * N.nw_T + ((N.nlp_src + 7) & ~7) + Npad;   // FP64: staged tail + Schur sources
     const int s32 = (solve_stage_bytes(N, 4) + 7) / 8, s64 = (solve_stage_bytes(N, 8) + 7) / 8;

@@ -1,6 +1,6 @@
 // Batched stiff chemistry solve for MI355X (gfx950).
 //
-// One workgroup (256 threads, 4 wave64) integrates one grid point at a time and then
+// One workgroup (512 threads, 8 wave64) integrates one grid point at a time and then
 // takes the next point from a device work counter, so uneven points (step counts vary
 // by >30x) never stall a whole batch: this is the persistent "retire and refill"
 // kernel.  Per point it reproduces UCLCHEM's per-interval semantics
@@ -21,7 +21,7 @@ __constant__ PhotoTables c_photo;
 
 // LDS scalar slots
 enum { S_SM, S_SBK, S_BLR, S_TS, S_SPRE, S_SCAT, S_H2COL, S_COCOL, S_CCOL, S_PHI, S_DENS, S_TGAS, S_TDUST,
-       S_AV, S_CS, S_COLDENS, S_ABSFAC, S_FLAG, S_H2CRP, S_RAD, S_MASS, S_NSCAL = 24 };
+       S_AV, S_CS, S_COLDENS, S_ABSFAC, S_FLAG, S_H2CRP, S_RAD, S_MASS, S_TIMERS = 24, S_NSCAL = 40 };
 
 // Large collective routines can be kept out of line to bound the kernel's register
 // allocation (UCG_BIG=__attribute__((noinline))); inlined by default.
@@ -38,64 +38,162 @@ enum { S_SM, S_SBK, S_BLR, S_TS, S_SPRE, S_SCAT, S_H2COL, S_COCOL, S_CCOL, S_PHI
 struct Lds {
     double *rate;                                   // workspace (global memory)
     LDS double *flux, *y, *f, *b, *g, *red, *sc, *prm;
+    int timed;                                      // per-phase clocks wanted (ucg_solve_batch_profiled)
 };
 
 __device__ __forceinline__ int tid() { return (int)threadIdx.x; }
 
-__device__ inline double block_sum(double v, LDS double *red)
+// The phases of a step (RHS, Newton-matrix set-up, Newton solve) are functions of their own:
+// the integrator's state stays in callee-saved registers across them and each phase is
+// allocated by itself, in a single copy of its code.  With everything inlined the history and the
+// control state lived in scratch memory: the work of a step outside these phases took 35 us, 13
+// like this (default network, FP64).  Arguments arrive in vector registers; these move the
+// uniform ones back to scalar registers.
+#define PHASE __device__ __attribute__((noinline))
+__device__ __forceinline__ uint64_t uniform64(uint64_t p)
 {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    __syncthreads();
-    if ((tid() & 63) == 0) red[tid() >> 6] = v;
+    const int lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)p), hi = __builtin_amdgcn_readfirstlane((int)(p >> 32));
+    return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
+}
+template <class T> __device__ __forceinline__ T *uniform_ptr(T *p) { return (T *)uniform64((uint64_t)p); }
+__device__ __forceinline__ LDS double *uniform_ptr(LDS double *p)
+{
+    return (LDS double *)(uintptr_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)p);
+}
+__device__ __forceinline__ Lds uniform_lds(Lds L)
+{
+    L.rate = uniform_ptr(L.rate);
+    L.flux = uniform_ptr(L.flux);
+    L.y = uniform_ptr(L.y);
+    L.f = uniform_ptr(L.f);
+    L.b = uniform_ptr(L.b);
+    L.g = uniform_ptr(L.g);
+    L.red = uniform_ptr(L.red);
+    L.sc = uniform_ptr(L.sc);
+    L.prm = uniform_ptr(L.prm);
+    L.timed = __builtin_amdgcn_readfirstlane(L.timed);
+    return L;
+}
+
+// Per-phase device clock (100 MHz), read only when the launch asks for it: mark(k) adds the time
+// since the last mark to timer k of the point.
+struct PhaseClock {
+    LDS double *tm;
+    bool on;
+    uint64_t c = 0;
+    __device__ __forceinline__ explicit PhaseClock(const Lds &L) : tm(L.sc + S_TIMERS), on(L.timed != 0)
+    {
+        if (on) c = wall_clock64();
+    }
+    __device__ __forceinline__ void mark(int k)
+    {
+        if (on) {
+            const uint64_t t = wall_clock64();
+            if (threadIdx.x == 0) tm[k] += (double)(t - c);
+            c = t;
+        }
+    }
+    __device__ __forceinline__ void mark(int k, uint64_t since) const
+    {
+        if (on && threadIdx.x == 0) tm[k] += (double)(wall_clock64() - since);
+    }
+};
+// timer slots: phases, then parts of them
+enum { TM_RATES, TM_RHS, TM_JAC, TM_LU, TM_SOLVE, TM_LU_SPARSE = 7, TM_LU_TAIL, TM_SOL_SPARSE, TM_SOL_TAIL,
+       TM_RHS_FLUX = 12, TM_RHS_SUMS, TM_RHS_TOTALS, TM_SKIP = 15 };
+
+// Sum over the 64 lanes of a wave with DPP row shifts and row broadcasts (no LDS round trips: six
+// shuffles through the LDS pipe cost about 0.35 us, this 0.06 us); every lane gets the total.
+template <int CTRL, int ROWS> __device__ __forceinline__ double dpp_zero(double v)
+{   // the value DPP brings to this lane, 0 where it brings none
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_lane(double v, int lane)
+{
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_sum(double v)
+{
+    v += dpp_zero<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+    v += dpp_zero<0x112, 0xf>(v);
+    v += dpp_zero<0x114, 0xf>(v);
+    v += dpp_zero<0x118, 0xf>(v);
+    v += dpp_zero<0x142, 0xa>(v);   // row_bcast 15 into rows 1 and 3
+    v += dpp_zero<0x143, 0xc>(v);   // row_bcast 31 into rows 2 and 3
+    return wave_lane(v, 63);
+}
+__device__ __forceinline__ double wave_max0(double v)   // v >= 0
+{
+    v = fmax(v, dpp_zero<0x111, 0xf>(v));
+    v = fmax(v, dpp_zero<0x112, 0xf>(v));
+    v = fmax(v, dpp_zero<0x114, 0xf>(v));
+    v = fmax(v, dpp_zero<0x118, 0xf>(v));
+    v = fmax(v, dpp_zero<0x142, 0xa>(v));
+    v = fmax(v, dpp_zero<0x143, 0xc>(v));
+    return wave_lane(v, 63);
+}
+
+// Workgroup reductions with one barrier: each wave's total goes to its slot of a buffer, every
+// wave adds all of them.  A buffer may be used again once a barrier lies between its last use
+// and the next; the call sites use distinct buffers (RED_*) so that this always holds.
+constexpr int NWAVE = NT / 64;
+enum { RED_TS, RED_S, RED_TOTALS, RED_CHARGE, RED_EWT, RED_ACOR, RED_CORR, RED_HIST, RED_NBUF };
+constexpr int RED_FLAGS = 16;                                   // red[0..15]: flags and small scratch
+constexpr int RED_LEN = RED_FLAGS + RED_NBUF * 2 * NWAVE;
+__device__ __forceinline__ double block_sum(double v, LDS double *red, int id)
+{
+    LDS double *buf = red + RED_FLAGS + id * 2 * NWAVE;
+    v = wave_sum(v);
+    if ((tid() & 63) == 0) buf[tid() >> 6] = v;
     __syncthreads();
     double r = 0.0;
 #pragma unroll
-    for (int w = 0; w < NT / 64; w++) r += red[w];
-    return r;
+    for (int w = 0; w < NWAVE; w++) r += buf[w];
+    return bdf_uni(r);
 }
-
-__device__ inline void block_sum2(double &a, double &b, LDS double *red)
+__device__ __forceinline__ void block_sum2(double &a, double &b, LDS double *red, int id)
 {
-    for (int off = 32; off > 0; off >>= 1) {
-        a += __shfl_xor(a, off);
-        b += __shfl_xor(b, off);
-    }
-    __syncthreads();
+    LDS double *buf = red + RED_FLAGS + id * 2 * NWAVE;
+    a = wave_sum(a);
+    b = wave_sum(b);
     if ((tid() & 63) == 0) {
-        red[tid() >> 6] = a;
-        red[NT / 64 + (tid() >> 6)] = b;
+        buf[tid() >> 6] = a;
+        buf[NWAVE + (tid() >> 6)] = b;
     }
     __syncthreads();
     double ra = 0.0, rb = 0.0;
 #pragma unroll
-    for (int w = 0; w < NT / 64; w++) {
-        ra += red[w];
-        rb += red[NT / 64 + w];
+    for (int w = 0; w < NWAVE; w++) {
+        ra += buf[w];
+        rb += buf[NWAVE + w];
     }
-    a = ra;
-    b = rb;
+    a = bdf_uni(ra);
+    b = bdf_uni(rb);
 }
-
-__device__ inline double block_max(double v, LDS double *red)
+__device__ __forceinline__ double block_max0(double v, LDS double *red, int id)   // v >= 0
 {
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off));
+    LDS double *buf = red + RED_FLAGS + id * 2 * NWAVE;
+    v = wave_max0(v);
+    if ((tid() & 63) == 0) buf[tid() >> 6] = v;
     __syncthreads();
-    if ((tid() & 63) == 0) red[tid() >> 6] = v;
-    __syncthreads();
-    double r = red[0];
+    double r = buf[0];
 #pragma unroll
-    for (int w = 1; w < NT / 64; w++) r = fmax(r, red[w]);
-    return r;
+    for (int w = 1; w < NWAVE; w++) r = fmax(r, buf[w]);
+    return bdf_uni(r);
 }
 
-__device__ __forceinline__ bool type_active(const DevNet &N, int t)
+__device__ __forceinline__ bool type_active(NetRef N, int t)
 {
     int a = N.type_ranges[2 * t], b = N.type_ranges[2 * t + 1];
     if (t == T_TWOBODY || t == T_BULKSWAP || t == T_SURFSWAP) return a >= 0;
     return a >= 0 && a != b;   // rates.f90 range blocks are skipped when idx1 == idx2
 }
 
-__device__ inline double freeze_out(const DevNet &N, const LDS double *prm, int j, double T, double Td)
+__device__ inline double freeze_out(NetRef N, const LDS double *prm, int j, double T, double Td)
 {   // rates.f90:354-367
     double f = 1.0 + N.beta[j] * 16.71e-4 / (GRAIN_RADIUS * T);
     if (prm[P_FREEZEFAC] == 0.0 || Td > MAX_GRAIN_TEMP) return 0.0;
@@ -107,7 +205,7 @@ __device__ inline double freeze_out(const DevNet &N, const LDS double *prm, int 
 // Rate coefficients for the current interval attempt (rates.f90:21-343 preceded by the
 // ice bookkeeping of chemistry.f90:167-200).  Reads y (LDS), writes rate (LDS), updates
 // y[BULK], y[SURFACE], the column densities, the ice scalars and phi.
-UCG_BIG __device__ void block_rates(const DevNet &N, const Lds L)
+__device__ __attribute__((noinline)) void block_rates(NetRef N, const Lds L)
 {
     const int neq = N.neq;
     const LDS double *prm = L.prm;
@@ -119,7 +217,7 @@ UCG_BIG __device__ void block_rates(const DevNet &N, const Lds L)
     double sb = 0.0, ss = 0.0;
     for (int i = tid(); i < N.nbulkl; i += NT) sb += y[N.bulk_list[i]];
     for (int i = tid(); i < N.nsurfl; i += NT) ss += y[N.surface_list[i]];
-    block_sum2(sb, ss, L.red);
+    block_sum2(sb, ss, L.red, RED_TOTALS);
     if (tid() == 0) {
         y[N.nbulk] = sb;
         y[N.nsurface] = ss;
@@ -348,7 +446,7 @@ __device__ __forceinline__ double term_from_codes(const int c[8], double r, cons
     return v;
 }
 
-__device__ __forceinline__ double term_value(const DevNet &N, int k, const double *rate, const LDS double *y,
+__device__ __forceinline__ double term_value(NetRef N, int k, const double *rate, const LDS double *y,
                                              double D, double blr, double TS, double sm)
 {
     int c[8];
@@ -358,9 +456,10 @@ __device__ __forceinline__ double term_value(const DevNet &N, int k, const doubl
 
 // RHS f(y) (chemistry.f90:294-352 + the generated GETYDOT, odes.f90).  Input L.y, output
 // L.f; also leaves the pre-transfer surface total in sc[S_SPRE] for the Jacobian.
-UCG_BIG __device__ void block_rhs(const DevNet &N, const Lds L, uint64_t *split = nullptr)
+UCG_BIG __device__ void block_rhs(NetRef N_, const Lds L)
 {
-    const uint64_t c0 = wall_clock64();
+    NetRef N = fresh(N_);
+    PhaseClock clk(L);
     const int neq = N.neq;
     LDS double *y = L.y, *f = L.f, *flux = L.flux, *sc = L.sc;
     double *rate = L.rate;
@@ -372,8 +471,8 @@ UCG_BIG __device__ void block_rhs(const DevNet &N, const Lds L, uint64_t *split 
     const double blr = fmin(1.0, NUM_SITES_PER_GRAIN / (GAS_DUST_DENSITY_RATIO * sbk));
     double ts = 0.0;
     for (int q = tid(); q < N.nswap; q += NT) ts += term_value(N, N.swap_list[q], rate, y, D, blr, 0.0, sm);
-    const double TS = block_sum(ts, L.red);
-    const uint64_t c1 = wall_clock64();
+    const double TS = block_sum(ts, L.red, RED_TS);
+    clk.mark(TM_SKIP);
     // H2 and CO photodissociation depend on the current column densities (chemistry.f90:311-319):
     // the last wave evaluates them (the seven CO row splines, the scattering term and the H2
     // rate in separate lanes) and their two fluxes while the other waves take every other flux.
@@ -426,7 +525,7 @@ UCG_BIG __device__ void block_rhs(const DevNet &N, const Lds L, uint64_t *split 
         }
     }
     __syncthreads();
-    const uint64_t c2 = wall_clock64();
+    clk.mark(TM_RHS_FLUX);
     // production and loss sums in balanced chunks (partial sums in LDS after the fluxes),
     // then per species in chunk order
     LDS double *part = flux + N.gt_off;
@@ -443,7 +542,7 @@ UCG_BIG __device__ void block_rhs(const DevNet &N, const Lds L, uint64_t *split 
         }
     }
     __syncthreads();
-    const uint64_t c3 = wall_clock64();
+    clk.mark(TM_RHS_SUMS);
     double pre[EPT];
     double spre = 0.0;
 #pragma unroll
@@ -460,7 +559,7 @@ UCG_BIG __device__ void block_rhs(const DevNet &N, const Lds L, uint64_t *split 
             if (N.is_surface[i]) spre += pre[e];
         }
     }
-    const double S = block_sum(spre, L.red);
+    const double S = block_sum(spre, L.red, RED_S);
     double tb = 0.0, tsu = 0.0;
     double out[EPT];
 #pragma unroll
@@ -484,7 +583,7 @@ UCG_BIG __device__ void block_rhs(const DevNet &N, const Lds L, uint64_t *split 
             }
         }
     }
-    block_sum2(tb, tsu, L.red);
+    block_sum2(tb, tsu, L.red, RED_TOTALS);
 #pragma unroll
     for (int e = 0; e < EPT; e++) {
         const int i = tid() + e * NT;
@@ -502,16 +601,11 @@ UCG_BIG __device__ void block_rhs(const DevNet &N, const Lds L, uint64_t *split 
         // enforceChargeConservation: ydot(e-) is the sum of the positive-ion rows (chemistry.f90:333-335)
         double e = 0.0;
         for (int q = tid(); q < N.nion; q += NT) e += f[N.ion_list[q]];
-        e = block_sum(e, L.red);
+        e = block_sum(e, L.red, RED_CHARGE);
         if (tid() == 0) f[N.nelec] = e;
         __syncthreads();
     }
-    if (split) {   // totalSwap, photo rates + fluxes, chunked sums, species totals + transfer
-        split[0] += c1 - c0;
-        split[1] += c2 - c1;
-        split[2] += c3 - c2;
-        split[3] += wall_clock64() - c3;
-    }
+    clk.mark(TM_RHS_TOTALS);
 }
 
 // ---------------------------------------------------------------- analytic Jacobian
@@ -537,7 +631,7 @@ __device__ __forceinline__ double fac_deriv(int c, double dblr, double dism, dou
 // Partial derivatives of every reaction term with respect to each of its factors:
 // P[fac_off[k] + m] = rate_k * d(factor m) * prod_{m' != m} factor m'.  One 16-byte
 // record per reaction holds its (up to 8) factor codes as int16, -1 padded.
-__device__ void block_term_partials(const DevNet &N, const double *rate, const LDS double *y, LDS double *P, double D,
+__device__ void block_term_partials(NetRef N, const double *rate, const LDS double *y, LDS double *P, double D,
                                     double blr, double ism, double tsm, double dblr, double dism, double dtsm)
 {
     const GLB int *fp = glb(N.facp);
@@ -565,7 +659,7 @@ __device__ void block_term_partials(const DevNet &N, const double *rate, const L
 }
 
 // Value of structural nonzero n of dJ (generated part): sum of coefficient * partial.
-__device__ __forceinline__ double jac_entry(const DevNet &N, const LDS double *P, int n)
+__device__ __forceinline__ double jac_entry(NetRef N, const LDS double *P, int n)
 {
     double acc = 0.0;
     const GLB int *jp = glb(N.jnz_ptr), *pk_ = glb(N.jc_pk);
@@ -583,7 +677,7 @@ __device__ __forceinline__ double jac_entry(const DevNet &N, const LDS double *P
 // shuffle tree inside the group; all lanes of a group take the same trip count, so the shuffles
 // read active lanes only).  The longest list (hundreds of terms) no longer serialises one lane.
 template <typename Store>
-__device__ __forceinline__ void jac_entries(const DevNet &N, const LDS double *P, Store store)
+__device__ __forceinline__ void jac_entries(NetRef N, const LDS double *P, Store store)
 {
     const GLB int *js = glb(N.jz_short);
     for (int q = tid(); q < N.nj_short; q += NT) {
@@ -611,7 +705,7 @@ __device__ __forceinline__ void jac_entries(const DevNet &N, const LDS double *P
 // BULK/SURFACE totals).  With scale != 0 the matrix is equilibrated by the error weights:
 // M' = W M W^-1, W = diag(ewt) (held in L.g).
 template <typename LUT>
-UCG_BIG __device__ void block_newton_matrix(const DevNet &N, const Lds L, LUT *M, double gamma, bool convert = true,
+UCG_BIG __device__ void block_newton_matrix(NetRef N, const Lds L, LUT *M, double gamma, bool convert = true,
                                     bool scaled = false)
 {
     const int neq = N.neq, ld = N.ld;
@@ -628,7 +722,7 @@ UCG_BIG __device__ void block_newton_matrix(const DevNet &N, const Lds L, LUT *M
     // totalSwap
     double ts = 0.0;
     for (int q = tid(); q < N.nswap; q += NT) ts += term_value(N, N.swap_list[q], rate, y, D, blr, 0.0, sm);
-    const double TS = block_sum(ts, L.red);
+    const double TS = block_sum(ts, L.red, RED_TS);
     const double tsm = TS / sm;
     const double dtsm = (ysur > 1e-30) ? -TS * ism * ism : 0.0;
     // 1. zero J; partial derivatives of every term
@@ -1278,8 +1372,9 @@ UCG_BIG __device__ void block_lu_solve(MP M, int n, int ld, LDS double *b)
 // transfer couplings (columns u1 and w2, rows -g1 and -gsum0, and c1); the BULK and
 // SURFACE rows are replaced by constant rows when the Newton matrix is formed
 // (sparse_form_newton).  Values are written in plan slot order; fill slots start at zero.
-UCG_BIG __device__ void sparse_jacobian(const DevNet &N, const Lds L, double *V)
+UCG_BIG __device__ void sparse_jacobian(NetRef N_, const Lds L, double *V)
 {
+    NetRef N = fresh(N_);
     const int neq = N.neq;
     LDS double *y = L.y, *sc = L.sc;
     double *rate = L.rate;
@@ -1293,7 +1388,7 @@ UCG_BIG __device__ void sparse_jacobian(const DevNet &N, const Lds L, double *V)
     const double dism = (ysur > 1e-30) ? -ism * ism : 0.0;
     double ts = 0.0;
     for (int q = tid(); q < N.nswap; q += NT) ts += term_value(N, N.swap_list[q], rate, y, D, blr, 0.0, sm);
-    const double TS = block_sum(ts, L.red);
+    const double TS = block_sum(ts, L.red, RED_TS);
     const double tsm = TS / sm;
     const double dtsm = (ysur > 1e-30) ? -TS * ism * ism : 0.0;
     {
@@ -1349,7 +1444,7 @@ UCG_BIG __device__ void sparse_jacobian(const DevNet &N, const Lds L, double *V)
     }
     double cs = 0.0;
     for (int q = tid(); q < N.nsurfl; q += NT) cs += scr[N.surface_list[q]];
-    const double c1 = block_sum(cs, L.red);
+    const double c1 = block_sum(cs, L.red, RED_S);
     if (tid() == 0) {
         V[N.nw_misc[2]] = c1;
     }
@@ -1435,8 +1530,9 @@ UCG_BIG __device__ void sparse_jacobian(const DevNet &N, const Lds L, double *V)
 // that carry gamma are scaled, the rank-one column factors and c1 are not; then the
 // identity, the border diagonals and the replaced BULK/SURFACE rows.
 template <typename LUT>
-UCG_BIG __device__ void sparse_form_newton(const DevNet &N, const double *J, LUT *V, double gamma, bool enforce)
+UCG_BIG __device__ void sparse_form_newton(NetRef N_, const double *J, LUT *V, double gamma, bool enforce)
 {
+    NetRef N = fresh(N_);
     for (int q = tid(); q < N.nw_nval; q += NT) V[q] = (LUT)(N.nw_unscaled[q] ? J[q] : gamma * J[q]);
     __syncthreads();
     for (int i = tid(); i < N.neq; i += NT) {
@@ -1469,7 +1565,7 @@ UCG_BIG __device__ void sparse_form_newton(const DevNet &N, const double *J, LUT
 // precision (the FP32 form does its whole factorisation in FP32: the Newton iteration's FP64
 // residuals absorb the difference) and stored back.  stage: 512 doubles of LDS.
 template <typename LUT, typename WP>
-__device__ __forceinline__ void crout_phases(const DevNet &N, WP W, LDS double *red, int nph)
+__device__ __forceinline__ void crout_phases(NetRef N, WP W, LDS double *red, int nph)
 {
     const GLB int *ph = glb(N.nw_ph_ptr), *tgs = glb(N.nw_tg_slot), *tgp = glb(N.nw_tg_ptr), *tgd = glb(N.nw_tg_div);
     const GLB int *pr = glb(N.nw_pr);
@@ -1510,18 +1606,17 @@ __device__ __forceinline__ void crout_phases(const DevNet &N, WP W, LDS double *
 }
 
 template <typename LUT>
-UCG_BIG __device__ int sparse_lu(const DevNet &N, LUT *V, LDS double *region, LDS double *red, LDS double *stage,
-                                 uint64_t *split = nullptr)
+UCG_BIG __device__ int sparse_lu(NetRef N_, const Lds &L, LUT *V, LDS double *region, LDS double *red, LDS double *stage)
 {
+    NetRef N = fresh(N_);
     const int nval = N.nw_nval, nsp = N.nw_nsp, T = N.nw_T;
     if (tid() == 0) red[9] = 0.0;
     int r = 0;
-    const uint64_t c0 = wall_clock64();
-    uint64_t c1;
+    PhaseClock clk(L);
     if (!N.nw_stage) {                    // factors too large to stage: everything in the workspace
         __syncthreads();
         crout_phases<LUT>(N, glbw(V), red, N.nw_nph);
-        c1 = wall_clock64();
+        clk.mark(TM_LU_SPARSE);
         if (red[9] != 0.0) return 1;
         if (T > 0) r = block_lu_tiled<LUT>(V + nsp, T, T, red, stage);
     } else {
@@ -1572,16 +1667,13 @@ UCG_BIG __device__ int sparse_lu(const DevNet &N, LUT *V, LDS double *region, LD
                 tl[e] = (a0 + a1) + (a2 + a3);
             }
         }
-        c1 = wall_clock64();
+        clk.mark(TM_LU_SPARSE);
         __syncthreads();
         if (T > 0) r = block_gj_inverse<LUT>(tl, T, T, red, stage);
         for (int q = tid(); q < T * T; q += NT) V[nsp + q] = tl[q];
     }
     __syncthreads();
-    if (split) {
-        split[0] += c1 - c0;
-        split[1] += wall_clock64() - c1;
-    }
+    clk.mark(TM_LU_TAIL);
     return r;
 }
 
@@ -1621,9 +1713,8 @@ __device__ __forceinline__ double group_sum(double v, int G)
 // backward by level.  V, the column indices and the row records are LDS or workspace
 // pointers (staged or unstaged plan); b (length neq, LDS) is overwritten by x.
 template <typename LUT, typename VP, typename IP, typename TP>
-__device__ __forceinline__ void solve_program(const DevNet &N, VP V, IP cols, IP recs, IP inv, IP lev, TP tail,
-                                              LDS double *w, LDS double *b, double sb, double ss, uint64_t *split,
-                                              uint64_t c0, uint64_t cs)
+__device__ __forceinline__ void solve_program(NetRef N, VP V, IP cols, IP recs, IP inv, IP lev, TP tail,
+                                              LDS double *w, LDS double *b, double sb, double ss, PhaseClock &clk)
 {
     const int neq = N.neq, NN = N.nw_N, ns = N.nw_ns, T = N.nw_T;
     for (int i = tid(); i < NN; i += NT) {
@@ -1636,7 +1727,6 @@ __device__ __forceinline__ void solve_program(const DevNet &N, VP V, IP cols, IP
         w[inv[i]] = v;
     }
     __syncthreads();
-    const uint64_t cf0 = wall_clock64();
     for (int l = 0; l < N.nw_nlev; l++) {   // forward, sparse rows by level
         const int q0 = lev[l];
         const int R = lev[l + 1] - q0;
@@ -1671,12 +1761,12 @@ __device__ __forceinline__ void solve_program(const DevNet &N, VP V, IP cols, IP
         }
     }
     __syncthreads();
-    const uint64_t c1 = wall_clock64();
+    clk.mark(TM_SOL_SPARSE);
     if (T > 0) {
         if (N.nw_stage) tail_matvec(tail, T, w + ns, w + NN);   // staged plans hold the block's inverse
         else block_lu_solve<LUT>(tail, T, T, w + ns);          // unstaged plans hold its LU factors
     }
-    const uint64_t c2 = wall_clock64();
+    clk.mark(TM_SOL_TAIL);
     for (int l = N.nw_nlev - 1; l >= 0; l--) {   // backward, sparse rows by level
         const int q0 = lev[l];
         const int R = lev[l + 1] - q0;
@@ -1698,12 +1788,7 @@ __device__ __forceinline__ void solve_program(const DevNet &N, VP V, IP cols, IP
     }
     for (int i = tid(); i < neq; i += NT) b[i] = w[inv[i]];
     __syncthreads();
-    if (split) {
-        split[0] += (c1 - c0) + (wall_clock64() - c2);   // staging, sparse rows, permutations
-        split[1] += c2 - c1;                             // dense tail
-        split[2] += cs - c0;                             // staging + right-hand-side sums
-        split[3] += c1 - cf0;                            // forward levels + tail rows
-    }
+    clk.mark(TM_SOL_SPARSE);
 }
 
 // Solve M x = b with the factors of sparse_lu: b (length neq, in LDS) is overwritten by x.
@@ -1713,15 +1798,15 @@ __device__ __forceinline__ void solve_program(const DevNet &N, VP V, IP cols, IP
 // too, FP64 tails are read from the workspace by the dense triangular solves.  An unstaged
 // plan reads all of it from the workspace and keeps only the work vector in region.
 template <typename LUT>
-UCG_BIG __device__ void sparse_lu_solve(const DevNet &N, const Lds L, const LUT *Vg, LDS double *b, LDS double *region,
-                                       uint64_t *split = nullptr)
+UCG_BIG __device__ void sparse_lu_solve(NetRef N_, const Lds L, const LUT *Vg, LDS double *b, LDS double *region)
 {
-    const uint64_t c0 = wall_clock64();
+    NetRef N = fresh(N_);
+    PhaseClock clk(L);
     const int NN = N.nw_N, nsp = N.nw_nsp;
     if (L.prm[P_ENFORCECHARGE] != 0.0 && N.nelec < N.nspec) {   // right-hand side of the charge row
         double se = 0.0;
         for (int q = tid(); q < N.nion; q += NT) se += b[N.ion_list[q]];
-        se = block_sum(se, L.red);
+        se = block_sum(se, L.red, RED_CHARGE);
         if (tid() == 0) b[N.nelec] -= se;
         __syncthreads();
     }
@@ -1729,9 +1814,8 @@ UCG_BIG __device__ void sparse_lu_solve(const DevNet &N, const Lds L, const LUT 
     for (int q = tid(); q < N.nbulkl; q += NT) sb += b[N.bulk_list[q]];
     for (int q = tid(); q < N.nsurfl; q += NT) ss += b[N.surface_list[q]];
     if (!N.nw_stage) {
-        block_sum2(sb, ss, L.red);
-        solve_program<LUT>(N, Vg, N.nw_sp_col, N.sv_rec, N.nw_inv, N.nw_lev_ptr, Vg + nsp, region, b, sb, ss, split, c0,
-                           wall_clock64());
+        block_sum2(sb, ss, L.red, RED_TOTALS);
+        solve_program<LUT>(N, Vg, N.nw_sp_col, N.sv_rec, N.nw_inv, N.nw_lev_ptr, Vg + nsp, region, b, sb, ss, clk);
         return;
     }
     constexpr bool STAGE_TAIL = sizeof(LUT) == 4;
@@ -1767,15 +1851,14 @@ UCG_BIG __device__ void sparse_lu_solve(const DevNet &N, const Lds L, const LUT 
     for (int q = tid(); q < NN; q += NT) inv[q] = glb(N.nw_inv)[q];
     LDS int *lev = inv + NN;   // level pointers (nlev + 1), after the permutation
     for (int q = tid(); q <= N.nw_nlev; q += NT) lev[q] = glb(N.nw_lev_ptr)[q];
-    block_sum2(sb, ss, L.red);   // its barriers also publish the staged program
-    const uint64_t cs = wall_clock64();
+    block_sum2(sb, ss, L.red, RED_TOTALS);   // its barriers also publish the staged program
     const LDS LUT *V = Vs;
     if constexpr (STAGE_TAIL)
         solve_program<LUT>(N, V, (const LDS int *)cols, (const LDS int *)recs, (const LDS int *)inv,
-                           (const LDS int *)lev, V + nsp, w, b, sb, ss, split, c0, cs);
+                           (const LDS int *)lev, V + nsp, w, b, sb, ss, clk);
     else
         solve_program<LUT>(N, V, (const LDS int *)cols, (const LDS int *)recs, (const LDS int *)inv,
-                           (const LDS int *)lev, Vg + nsp, w, b, sb, ss, split, c0, cs);
+                           (const LDS int *)lev, Vg + nsp, w, b, sb, ss, clk);
 }
 
 // ---------------------------------------------------------------- BDF ops policy
@@ -1788,64 +1871,117 @@ __device__ __forceinline__ bool cancel_requested(const int *cancel, int gen)
     return cancel && __hip_atomic_load(cancel, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) >= gen;
 }
 
+PHASE void rhs_phase(const DevNet *Np, Lds L_)
+{
+    const Lds L = uniform_lds(L_);
+    PhaseClock clk(L);
+    block_rhs(*(const CST DevNet *)uniform_ptr(Np), L);
+    clk.mark(TM_RHS);
+}
+
+template <typename LUT>
+PHASE void sparse_solve_phase(const DevNet *Np, Lds L_, const LUT *M)
+{
+    const Lds L = uniform_lds(L_);
+    PhaseClock clk(L);
+    sparse_lu_solve<LUT>(*(const CST DevNet *)uniform_ptr(Np), L, uniform_ptr(M), L.b, L.flux);
+    clk.mark(TM_SOLVE);
+}
+
+template <typename LUT>
+PHASE void dense_solve_phase(const DevNet *Np, Lds L_, const LUT *M)
+{
+    const Lds L = uniform_lds(L_);
+    PhaseClock clk(L);
+    NetRef N = *(const CST DevNet *)uniform_ptr(Np);
+    block_lu_solve<LUT>(uniform_ptr(M), N.neq, N.ld, L.b);
+    clk.mark(TM_SOLVE);
+}
+
+template <typename LUT>
+PHASE int sparse_setup_phase(const DevNet *Np, Lds L_, LUT *M, double *J, double gamma, bool new_jacobian)
+{
+    const Lds L = uniform_lds(L_);
+    NetRef N = *(const CST DevNet *)uniform_ptr(Np);
+    M = uniform_ptr(M);
+    J = uniform_ptr(J);
+    PhaseClock clk(L);
+    if (new_jacobian) sparse_jacobian(N, L, J);
+    sparse_form_newton<LUT>(N, J, M, gamma, L.prm[P_ENFORCECHARGE] != 0.0);
+    clk.mark(TM_JAC);
+    const int r = sparse_lu<LUT>(N, L, M, L.flux, L.red, L.b);
+    clk.mark(TM_LU);
+    return r;
+}
+
+template <typename LUT>
+PHASE int dense_setup_phase(const DevNet *Np, Lds L_, LUT *M, double gamma, bool equilibrate)
+{
+    const Lds L = uniform_lds(L_);
+    NetRef N = *(const CST DevNet *)uniform_ptr(Np);
+    M = uniform_ptr(M);
+    PhaseClock clk(L);
+    block_newton_matrix<LUT>(N, L, M, gamma, true, equilibrate);
+    clk.mark(TM_JAC);
+    const int r = block_lu<LUT>(M, N.neq, N.ld, L.red, L.flux);
+    clk.mark(TM_LU);
+    return r;
+}
+
 template <typename LUT>
 struct GpuOps {
-    const DevNet &N;
+    NetRef N;
+    const DevNet *Np;
     const Lds L;   // by value: the LDS and workspace pointers live in registers
     LUT *M;
     int neq;
     double z[6][EPT], acor[EPT], ewt[EPT], atol[EPT], f0[EPT];
-    uint64_t t_rhs = 0, t_jac = 0, t_lu = 0, t_sol = 0;   // device wall-clock ticks per phase
-    uint64_t t_lu_split[2] = {0, 0}, t_sol_split[4] = {0, 0, 0, 0};   // sparse part, dense tail, ...
-    uint64_t t_rhs_split[4] = {0, 0, 0, 0};
+    double z0_norm = 0.0;   // WRMS norm of z[0] in the weights of the last set_ewt
     bool equilibrate = false;   // factor W M W^-1 (W = diag(ewt)) instead of M (dense form only)
     bool sparse = true;         // static-pattern sparse plan (else dense LU of the full matrix)
     double *Jsave = nullptr;    // saved J-form values of the sparse plan (workspace)
     const int *cancel = nullptr;  // highest cancelled launch generation, raised by the host while kernels run
     int gen = 0;                  // this launch's generation
-    __device__ bool cancelled() const { return cancel_requested(cancel, gen); }
+    int polls = 0;
+    // the cancel word is in memory shared with the host (a load from it takes microseconds):
+    // read it at every 16th step
+    __device__ __forceinline__ bool cancelled() { return (polls++ & 15) == 0 && cancel_requested(cancel, gen); }
 
-    __device__ GpuOps(const DevNet &n_, Lds &l_, LUT *m_) : N(n_), L(l_), M(m_), neq(n_.neq) {}
+    __device__ GpuOps(const DevNet *np_, Lds &l_, LUT *m_)
+        : N(*(const CST DevNet *)np_), Np(np_), L(l_), M(m_), neq(((const CST DevNet *)np_)->neq) {}
 
     __device__ __forceinline__ bool own(int e) const { return tid() + e * NT < neq; }
     __device__ __forceinline__ int idx(int e) const { return tid() + e * NT; }
 
-    // z[j][e] with a run-time j but compile-time storage indices (keeps z in VGPRs)
+    // z[j][e] with a run-time j but compile-time storage indices: selects between values, since a
+    // switch over the elements is merged into one access with a computed address, which puts the
+    // whole history into scratch memory
     __device__ __forceinline__ double zget(int j, int e) const
     {
-        switch (j) {
-        case 0: return z[0][e];
-        case 1: return z[1][e];
-        case 2: return z[2][e];
-        case 3: return z[3][e];
-        case 4: return z[4][e];
-        default: return z[5][e];
-        }
+        double v = z[0][e];
+#pragma unroll
+        for (int k = 1; k <= bdf::QMAX; k++) v = bdf::sel(j == k, z[k][e], v);
+        return v;
     }
     __device__ __forceinline__ void zset(int j, int e, double v)
     {
-        switch (j) {
-        case 0: z[0][e] = v; break;
-        case 1: z[1][e] = v; break;
-        case 2: z[2][e] = v; break;
-        case 3: z[3][e] = v; break;
-        case 4: z[4][e] = v; break;
-        default: z[5][e] = v; break;
-        }
+#pragma unroll
+        for (int k = 0; k <= bdf::QMAX; k++) z[k][e] = bdf::sel(j == k, v, z[k][e]);
     }
-    __device__ double wrms(int v)
+    __device__ __forceinline__ double wrms(int v)
     {
+        if (v == bdf::Z0) return z0_norm;   // set_ewt has it
         double acc = 0.0;
 #pragma unroll
         for (int e = 0; e < EPT; e++)
             if (own(e)) {
-                double x = (v == bdf::ACOR) ? acor[e] : zget(v, e);
+                double x = bdf::sel(v == bdf::ACOR, acor[e], zget(v, e));
                 double t = x * ewt[e];
                 acc += t * t;
             }
-        return sqrt(block_sum(acc, L.red) / neq);
+        return bdf_uni(sqrt(block_sum(acc, L.red, v == bdf::ACOR ? RED_ACOR : RED_HIST) / neq));
     }
-    __device__ double wrms_acor_minus(double c, int zj)
+    __device__ __forceinline__ double wrms_acor_minus(double c, int zj)
     {
         double acc = 0.0;
 #pragma unroll
@@ -1854,21 +1990,26 @@ struct GpuOps {
                 double t = (acor[e] - c * zget(zj, e)) * ewt[e];
                 acc += t * t;
             }
-        return sqrt(block_sum(acc, L.red) / neq);
+        return bdf_uni(sqrt(block_sum(acc, L.red, RED_CORR) / neq));
     }
-    __device__ bool set_ewt(double rtol)
+    // error weights of z[0], their check and z[0]'s norm in them, one reduction
+    __device__ __forceinline__ bool set_ewt(double rtol)
     {
-        double bad = 0.0;
+        double bad = 0.0, acc = 0.0;
 #pragma unroll
         for (int e = 0; e < EPT; e++)
             if (own(e)) {
                 double d = rtol * fabs(z[0][e]) + atol[e];
                 if (!(d > 0.0)) bad = 1.0;
                 ewt[e] = 1.0 / d;
+                double t = z[0][e] * ewt[e];
+                acc += t * t;
             }
-        return block_max(bad, L.red) == 0.0;
+        block_sum2(acc, bad, L.red, RED_EWT);
+        z0_norm = bdf_uni(sqrt(acc / neq));
+        return bad == 0.0;
     }
-    __device__ void start_corrector()
+    __device__ __forceinline__ void start_corrector()
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++)
@@ -1878,35 +2019,33 @@ struct GpuOps {
             }
         __syncthreads();
     }
-    __device__ void rhs()
+    __device__ __forceinline__ void rhs()
     {
-        uint64_t t0 = wall_clock64();
-        block_rhs(N, L, t_rhs_split);
-        t_rhs += wall_clock64() - t0;
+        rhs_phase(Np, L);
     }
-    __device__ void save_f0()
+    __device__ __forceinline__ void save_f0()
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++)
             if (own(e)) f0[e] = L.f[idx(e)];
     }
-    __device__ void scale_into_z_from(int j, double a, int src)
+    __device__ __forceinline__ void scale_into_z_from(int j, double a, int src)
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++)
-            if (own(e)) zset(j, e, a * ((src == bdf::F0) ? f0[e] : L.f[idx(e)]));
+            if (own(e)) zset(j, e, a * bdf::sel(src == bdf::F0, f0[e], L.f[idx(e)]));
     }
-    __device__ void scale_into_z(int j, double a, int src)
+    __device__ __forceinline__ void scale_into_z(int j, double a, int src)
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++) zset(j, e, a * zget(src, e));
     }
-    __device__ void axpy_zz(int j, double a, int src)
+    __device__ __forceinline__ void axpy_zz(int j, double a, int src)
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++) zset(j, e, zget(j, e) + a * zget(src, e));
     }
-    __device__ void rescale_z(int q, double eta)
+    __device__ __forceinline__ void rescale_z(int q, double eta)
     {
         double f = eta;
 #pragma unroll
@@ -1918,7 +2057,7 @@ struct GpuOps {
             }
         }
     }
-    __device__ void predict(int q)
+    __device__ __forceinline__ void predict(int q)
     {
 #pragma unroll
         for (int k = 1; k <= bdf::QMAX; k++)
@@ -1928,7 +2067,7 @@ struct GpuOps {
 #pragma unroll
                     for (int e = 0; e < EPT; e++) z[j - 1][e] += z[j][e];
     }
-    __device__ void unpredict(int q)
+    __device__ __forceinline__ void unpredict(int q)
     {
 #pragma unroll
         for (int k = 1; k <= bdf::QMAX; k++)
@@ -1938,7 +2077,7 @@ struct GpuOps {
 #pragma unroll
                     for (int e = 0; e < EPT; e++) z[j - 1][e] -= z[j][e];
     }
-    __device__ void complete(int q, const double *l)
+    __device__ __forceinline__ void complete(int q, const double *l)
     {
 #pragma unroll
         for (int j = 0; j <= bdf::QMAX; j++)
@@ -1946,12 +2085,12 @@ struct GpuOps {
 #pragma unroll
                 for (int e = 0; e < EPT; e++) z[j][e] += l[j] * acor[e];
     }
-    __device__ void copy_acor_to_z(int j)
+    __device__ __forceinline__ void copy_acor_to_z(int j)
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++) zset(j, e, acor[e]);
     }
-    __device__ void form_residual(double gamma, double rl1)
+    __device__ __forceinline__ void form_residual(double gamma, double rl1)
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++)
@@ -1962,14 +2101,12 @@ struct GpuOps {
             }
         __syncthreads();
     }
-    __device__ void solve()
+    __device__ __forceinline__ void solve()
     {
-        uint64_t t0 = wall_clock64();
-        if (sparse) sparse_lu_solve<LUT>(N, L, M, L.b, L.flux, t_sol_split);
-        else block_lu_solve<LUT>(M, neq, N.ld, L.b);
-        t_sol += wall_clock64() - t0;
+        if (sparse) sparse_solve_phase<LUT>(Np, L, M);
+        else dense_solve_phase<LUT>(Np, L, M);
     }
-    __device__ double apply_correction(double scale)
+    __device__ __forceinline__ double apply_correction(double scale)
     {
         double acc = 0.0;
 #pragma unroll
@@ -1983,7 +2120,7 @@ struct GpuOps {
                 acor[e] += d;
                 L.y[i] = z[0][e] + acor[e];
             }
-        double r = sqrt(block_sum(acc, L.red) / neq);
+        double r = bdf_uni(sqrt(block_sum(acc, L.red, RED_CORR) / neq));
         return r;
     }
     // Reusing a saved J between Newton-matrix setups (DVODE's JSV=1) was measured on the
@@ -1991,45 +2128,31 @@ struct GpuOps {
     // a net loss since an analytic J costs under half a factorisation here; kept off.
     bool reuse_jacobian = false;
     __device__ bool can_reuse_jacobian() const { return sparse && reuse_jacobian; }
-    __device__ int setup(double gamma, bool new_jacobian)
+    __device__ __forceinline__ int setup(double gamma, bool new_jacobian)
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++)
             if (own(e)) L.g[idx(e)] = equilibrate ? ewt[e] : 1.0;
         __syncthreads();
-        uint64_t t0 = wall_clock64();
-        int r;
-        uint64_t t1;
-        if (sparse) {
-            if (new_jacobian) sparse_jacobian(N, L, Jsave);
-            sparse_form_newton<LUT>(N, Jsave, M, gamma, L.prm[P_ENFORCECHARGE] != 0.0);
-            t1 = wall_clock64();
-            r = sparse_lu<LUT>(N, M, L.flux, L.red, L.b, t_lu_split);
-        } else {
-            block_newton_matrix<LUT>(N, L, M, gamma, true, equilibrate);
-            t1 = wall_clock64();
-            r = block_lu<LUT>(M, neq, N.ld, L.red, L.flux);
-        }
-        uint64_t t2 = wall_clock64();
-        t_jac += t1 - t0;
-        t_lu += t2 - t1;
-        return r;
+        const int r = sparse ? sparse_setup_phase<LUT>(Np, L, M, Jsave, gamma, new_jacobian)
+                             : dense_setup_phase<LUT>(Np, L, M, gamma, equilibrate);
+        return __builtin_amdgcn_readfirstlane(r);
     }
-    __device__ double hub_inverse(double fac)
+    __device__ __forceinline__ double hub_inverse(double fac)
     {
         double m = 0.0;
 #pragma unroll
         for (int e = 0; e < EPT; e++)
             if (own(e)) m = fmax(m, fabs(f0[e]) / (fac * fabs(z[0][e]) + atol[e]));
-        return block_max(m, L.red);
+        return block_max0(m, L.red, RED_HIST);
     }
-    __device__ double ydd_norm(double t0, double hg)
+    __device__ __forceinline__ double ydd_norm(double t0, double hg)
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++)
             if (own(e)) L.y[idx(e)] = z[0][e] + hg * f0[e];
         __syncthreads();
-        block_rhs(N, L);
+        rhs_phase(Np, L);
         double acc = 0.0;
 #pragma unroll
         for (int e = 0; e < EPT; e++)
@@ -2037,10 +2160,10 @@ struct GpuOps {
                 double t = (L.f[idx(e)] - f0[e]) / hg * ewt[e];
                 acc += t * t;
             }
-        return sqrt(block_sum(acc, L.red) / neq);
+        return bdf_uni(sqrt(block_sum(acc, L.red, RED_CORR) / neq));
     }
     __device__ void finish_at_tn() {}
-    __device__ void interpolate(double s, int q)
+    __device__ __forceinline__ void interpolate(double s, int q)
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++) {
@@ -2100,7 +2223,7 @@ struct SolveArgs {
     int y_stride;             // y_out row stride, 0: the network's NEQ
 };
 
-__device__ void elemental_start(const DevNet &N, const LDS double *prm, LDS double *y, double density)
+__device__ void elemental_start(NetRef N, const LDS double *prm, LDS double *y, double density)
 {   // chemistry.f90:58-105: elemental abundances from the point's parameters, in the
     // reference's order (species a network lacks share the density slot, restored last)
     const int neq = N.neq;
@@ -2168,7 +2291,7 @@ __device__ inline double h2_crp_rate_dev(double coldens, double zeta, bool high)
     return pow(10.0, sum) * zeta;
 }
 
-__device__ void record_row(const DevNet &N, const Lds L, const SolveArgs &A, int pidx, int row, double tyears)
+__device__ void record_row(NetRef N, const Lds L, const SolveArgs &A, int pidx, int row, double tyears)
 {
     if (A.max_rec <= 0 || row >= A.max_rec) return;
     const int ns = N.nspec;
@@ -2191,7 +2314,7 @@ __device__ void record_row(const DevNet &N, const Lds L, const SolveArgs &A, int
 
 // LDS layout shared by all kernels; the rate coefficients live in the workspace slot
 // (read coalesced, written once per interval attempt).
-__device__ void lds_layout(const DevNet &N, Lds &L, double *lds_raw, double *rate)
+__device__ void lds_layout(NetRef N, Lds &L, double *lds_raw, double *rate)
 {
     const int npad = (N.neq + 7) & ~7;
     L.rate = rate;
@@ -2201,8 +2324,9 @@ __device__ void lds_layout(const DevNet &N, Lds &L, double *lds_raw, double *rat
     L.b = L.f + npad;
     L.g = L.b + npad;
     L.red = L.g + npad;
-    L.sc = L.red + 16;
+    L.sc = L.red + RED_LEN;
     L.prm = L.sc + S_NSCAL;
+    L.timed = 0;
 }
 
 // Resets the work counter and the cancel flag and marks every point "not run" before a
@@ -2380,11 +2504,14 @@ __global__ __launch_bounds__(NT, UCG_WAVES_PER_EU) void solve_points_kernel(cons
         if (pidx >= A.n_points) break;   // every wave of the workgroup leaves here
         // the point's network: tables in global memory (field loads stay scalar, nothing copied
         // to scratch); its LDS layout fits the launch's LDS, sized for the largest network
-        const DevNet &N = A.q_nets ? *A.q_nets[inet] : *Np;
+        const DevNet *Nq = uniform_ptr(A.q_nets ? A.q_nets[inet] : Np);
+        NetRef N = *(const CST DevNet *)Nq;
         const int neq = N.neq;
         const size_t ystride = A.y_stride ? (size_t)A.y_stride : (size_t)neq;
         Lds L;
         lds_layout(N, L, lds_raw, (double *)(slot + A.ws_mat_bytes + A.ws_jac_bytes));
+        L.timed = A.timers != nullptr;
+        if (tid() < 16) L.sc[S_TIMERS + tid()] = 0.0;
 
         if (A.t_start && tid() == 0) A.t_start[pidx] = (double)wall_clock64();
         // ---- point set-up: parameters, physics (physics-core.f90:42-73, cloud.f90:20-31)
@@ -2431,7 +2558,7 @@ __global__ __launch_bounds__(NT, UCG_WAVES_PER_EU) void solve_points_kernel(cons
         } else {
             elemental_start(N, prm, L.y, L.sc[S_DENS]);
         }
-        GpuOps<LUT> o(N, L, M);
+        GpuOps<LUT> o(Nq, L, M);
         o.sparse = A.sparse != 0;
         o.Jsave = (double *)(slot + A.ws_mat_bytes);
         o.cancel = A.cancel;
@@ -2456,7 +2583,6 @@ __global__ __launch_bounds__(NT, UCG_WAVES_PER_EU) void solve_points_kernel(cons
         // integrator cannot advance t at all; here such a point stops with
         // INT_TOO_MANY_FAILS_ERROR after 10 intervals without progress.
         int stuck = 0;
-        uint64_t t_rates = 0;
         const uint64_t t_point0 = wall_clock64();
         const uint64_t c_point0 = clock64();   // shader clock, for the effective frequency
         while (!flag && (interval_mode ? nint == 0
@@ -2481,9 +2607,9 @@ __global__ __launch_bounds__(NT, UCG_WAVES_PER_EU) void solve_points_kernel(cons
                 // the density the physics set, unless it is integrated (chemistry.f90:166)
                 if (!freefall && tid() == 0) L.y[neq - 1] = L.sc[S_DENS];
                 __syncthreads();
-                const uint64_t tr0 = wall_clock64();
+                PhaseClock clk(L);
                 block_rates(N, L);
-                t_rates += wall_clock64() - tr0;
+                clk.mark(TM_RATES);
                 const double absfac = L.sc[S_ABSFAC];
 #pragma unroll
                 for (int e = 0; e < EPT; e++)
@@ -2511,7 +2637,7 @@ __global__ __launch_bounds__(NT, UCG_WAVES_PER_EU) void solve_points_kernel(cons
                     __syncthreads();
                     double ions = 0.0;
                     for (int q = tid(); q < N.nion; q += NT) ions += L.y[N.ion_list[q]];
-                    ions = block_sum(ions, L.red);
+                    ions = block_sum(ions, L.red, RED_CHARGE);
 #pragma unroll
                     for (int e = 0; e < EPT; e++)
                         if (o.own(e) && o.idx(e) == N.nelec) o.z[0][e] = ions;
@@ -2582,15 +2708,10 @@ __global__ __launch_bounds__(NT, UCG_WAVES_PER_EU) void solve_points_kernel(cons
             if (A.timers) {
                 const double tick = 1.0e-8;   // wall_clock64 runs at 100 MHz
                 double *tm = A.timers + (size_t)pidx * 16;
-                tm[0] = t_rates * tick; tm[1] = o.t_rhs * tick; tm[2] = o.t_jac * tick; tm[3] = o.t_lu * tick;
+                for (int k = 0; k < 16; k++) tm[k] = L.sc[S_TIMERS + k] * tick;
                 const uint64_t dw = wall_clock64() - t_point0, dc = clock64() - c_point0;
-                tm[4] = o.t_sol * tick; tm[5] = dw * tick;
+                tm[5] = dw * tick;
                 tm[6] = dw ? (double)dc / ((double)dw * tick) * 1e-6 : 0.0;   // mean shader clock, MHz
-                tm[7] = o.t_lu_split[0] * tick; tm[8] = o.t_lu_split[1] * tick;
-                tm[9] = o.t_sol_split[0] * tick; tm[10] = o.t_sol_split[1] * tick;
-                tm[11] = o.t_sol_split[2] * tick;   // solve: staging + right-hand-side sums
-                for (int k = 1; k < 4; k++) tm[11 + k] = o.t_rhs_split[k] * tick;
-                tm[15] = o.t_sol_split[3] * tick;   // solve: forward levels (staging in [9])
             }
         }
         __syncthreads();
@@ -2623,7 +2744,7 @@ struct PieceArgs {
     size_t ws_jac_bytes;
 };
 
-__device__ void piece_setup(const DevNet &N, Lds &L, const PieceArgs &A, int p)
+__device__ void piece_setup(NetRef N, Lds &L, const PieceArgs &A, int p)
 {
     for (int i = tid(); i < P_NPARAM; i += NT) L.prm[i] = A.params[(size_t)p * P_NPARAM + i];
     for (int i = tid(); i < N.neq; i += NT) L.y[i] = A.y[(size_t)p * N.neq + i];
@@ -2651,7 +2772,7 @@ __device__ void piece_setup(const DevNet &N, Lds &L, const PieceArgs &A, int p)
 
 __global__ __launch_bounds__(NT) void rates_kernel(const DevNet *__restrict__ Np, PieceArgs A)
 {
-    const DevNet &N = *Np;   // tables in global memory: field loads stay scalar, nothing copied to scratch
+    NetRef N = *(const CST DevNet *)Np;   // tables in global memory: field loads stay scalar
     extern __shared__ double lds_raw[];
     Lds L;
     lds_layout(N, L, lds_raw, (double *)((char *)A.ws + (size_t)blockIdx.x * A.ws_stride + A.ws_mat_bytes + A.ws_jac_bytes));
@@ -2670,7 +2791,7 @@ __global__ __launch_bounds__(NT) void rates_kernel(const DevNet *__restrict__ Np
 
 __global__ __launch_bounds__(NT) void rhs_kernel(const DevNet *__restrict__ Np, PieceArgs A)
 {
-    const DevNet &N = *Np;   // tables in global memory: field loads stay scalar, nothing copied to scratch
+    NetRef N = *(const CST DevNet *)Np;   // tables in global memory: field loads stay scalar
     extern __shared__ double lds_raw[];
     Lds L;
     lds_layout(N, L, lds_raw, (double *)((char *)A.ws + (size_t)blockIdx.x * A.ws_stride + A.ws_mat_bytes + A.ws_jac_bytes));
@@ -2687,7 +2808,7 @@ __global__ __launch_bounds__(NT) void rhs_kernel(const DevNet *__restrict__ Np, 
 
 __global__ __launch_bounds__(NT) void jac_kernel(const DevNet *__restrict__ Np, PieceArgs A)
 {
-    const DevNet &N = *Np;   // tables in global memory: field loads stay scalar, nothing copied to scratch
+    NetRef N = *(const CST DevNet *)Np;   // tables in global memory: field loads stay scalar
     extern __shared__ double lds_raw[];
     Lds L;
     lds_layout(N, L, lds_raw, (double *)((char *)A.ws + (size_t)blockIdx.x * A.ws_stride + A.ws_mat_bytes + A.ws_jac_bytes));
@@ -2708,7 +2829,7 @@ __global__ __launch_bounds__(NT) void jac_kernel(const DevNet *__restrict__ Np, 
 template <typename LUT>
 __global__ __launch_bounds__(NT) void newton_solve_kernel(const DevNet *__restrict__ Np, PieceArgs A)
 {
-    const DevNet &N = *Np;   // tables in global memory: field loads stay scalar, nothing copied to scratch
+    NetRef N = *(const CST DevNet *)Np;   // tables in global memory: field loads stay scalar
     extern __shared__ double lds_raw[];
     Lds L;
     lds_layout(N, L, lds_raw, (double *)((char *)A.ws + (size_t)blockIdx.x * A.ws_stride + A.ws_mat_bytes + A.ws_jac_bytes));
@@ -2726,7 +2847,7 @@ __global__ __launch_bounds__(NT) void newton_solve_kernel(const DevNet *__restri
         double *J = (double *)((char *)A.ws + (size_t)blockIdx.x * A.ws_stride + A.ws_mat_bytes);
         sparse_jacobian(N, L, J);
         sparse_form_newton<LUT>(N, J, M, A.gamma, L.prm[P_ENFORCECHARGE] != 0.0);
-        bad = sparse_lu<LUT>(N, M, L.flux, L.red, L.b);
+        bad = sparse_lu<LUT>(N, L, M, L.flux, L.red, L.b);
     } else {
         block_newton_matrix<LUT>(N, L, M, A.gamma);
         bad = block_lu<LUT>(M, N.neq, N.ld, L.red, L.flux);

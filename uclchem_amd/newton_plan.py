@@ -331,7 +331,7 @@ def lds_bytes(tables, staged: bool = True) -> int:
     else:
         c = Npad
     from .params import NPARAM
-    return 8 * (max(b, c) + 4 * npad + 16 + 24 + NPARAM)   # + reduction slots, scalars, parameters
+    return 8 * (max(b, c) + 4 * npad + 144 + 40 + NPARAM)   # + reduction slots, scalars, parameters
 
 
 def schur_sources(tables) -> int:
