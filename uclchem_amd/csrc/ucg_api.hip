@@ -510,8 +510,8 @@ static int check_plan(const ucg_network_desc *d)
         nph < 1 || nphs < 0 || ngs < 0)
         return bad("inconsistent sizes");
     if (T > 0 && NN - ns > ucg::NT * ucg::EPT) return bad("tail too large");
-    // the tail's Gauss-Jordan keeps its 8x8 pivot-block inverse in the right-hand-side vector
-    if (T > 0 && ((d->neq + 7) & ~7) < ucg::GJ_B * ucg::GJ_B) return bad("network too small for the dense tail");
+    // the unstaged tail's blocked LU keeps its 16x16 block factors in the NEQ-long work vectors
+    if (T > 0 && ((d->neq + 7) & ~7) < 64) return bad("network too small for the dense tail");
     auto in = [](const int *a, long n, long lo, long hi) {   // every a[i] in [lo, hi)
         if (n > 0 && !a) return false;
         for (long i = 0; i < n; i++)
@@ -958,7 +958,8 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
     HIPCHK(hipMemset(h.cancel, 0, sizeof(int)));
     hipDeviceProp_t prop;
     HIPCHK(hipGetDeviceProperties(&prop, g_device));
-    if (lds_bytes(N) > (size_t)prop.sharedMemPerBlock) N.nw_stage = 0;   // factors stay in the workspace
+    if (lds_bytes(N) > (size_t)prop.sharedMemPerBlock || N.nw_T > ucg::GJ_MAX)
+        N.nw_stage = 0;   // factors stay in the workspace
     size_t lds = lds_bytes(N);
     if (lds > (size_t)prop.sharedMemPerBlock)
         return fail(UCG_E_ARG, "network needs " + std::to_string(lds) + " B of LDS per workgroup, device allows " +

@@ -176,7 +176,10 @@ __host__ __device__ inline int flux_region_len(const Net &N)
     const int b1 = b0 > g ? b0 : g;
     const int b = b1 > NT ? b1 : NT;                 // >= one value per thread (ordered_sum)
     if (!N.nw_stage) return b > Npad ? b : Npad;               // unstaged plan: the work vector only
-    const int t64 = N.nw_T * N.nw_T + ((N.nlp_src + 7) & ~7) + Npad;   // FP64: staged tail + Schur sources
+    // staged tail beside the Schur sources, then beside the exchange buffers of its inversion
+    const int gj = 2 * ((N.nw_T + 15) / 16 + 1) * 16 * 17;
+    const int beside = ((N.nlp_src + 7) & ~7) + Npad > gj ? ((N.nlp_src + 7) & ~7) + Npad : gj;
+    const int t64 = N.nw_T * N.nw_T + beside;
     const int s32 = (solve_stage_bytes(N, 4) + 7) / 8, s64 = (solve_stage_bytes(N, 8) + 7) / 8;
     const int f = s32 > s64 ? s32 : s64;
     const int c = t64 > f ? t64 : f;

@@ -1148,107 +1148,162 @@ UCG_BIG __device__ int block_lu_tiled(MP M, int n, int ld, LDS double *red, LDS 
     return 0;
 }
 
-// In-place inverse of the dense n x n block M (column-major, leading dimension ld) by
-// blocked Gauss-Jordan elimination without pivoting, GJ_B = 8 pivots per sweep: the 8x8 pivot
-// block is inverted by wave 0, one element per lane (eight elimination steps whose pivot row
-// and column travel by shuffles), its row panel is multiplied by that inverse (one column per
-// thread), every entry outside the pivot rows and columns takes the rank-8 update in 4x4
-// register tiles, then the pivot column panel becomes -A_IK inv(A_KK).  Eight pivots per sweep
-// halve the sweeps and barriers of a four-pivot sweep and load each 4x4 tile once per eight
-// rank-one terms.  The pivots are those of the unpivoted LU and are checked the same way; it
-// is used for the trailing block of the sparse plan so that each Newton solve applies the
-// block as one matrix-vector product instead of two dependent triangular sweeps.  stage: >= 64
-// doubles of LDS.  Returns nonzero (uniformly) on a zero or non-finite pivot.
-constexpr int GJ_B = 8;
-template <typename LUT, typename MP>
-__device__ __attribute__((always_inline)) int block_gj_inverse(MP M, int n, int ld, LDS double *red, LDS double *stage)
+// ---------------------------------------------------------------- inverse of the dense tail
+// The tail (n <= 128 rows, padded with the identity to nb = ceil(n/16) blocks of 16) is inverted
+// by block Gauss-Jordan elimination without pivoting, 16 pivots per sweep, in the accumulator
+// layout of v_mfma_f64_16x16x4: wave w holds block column w as nb tiles of four doubles per lane
+// (lane 16g + c, register i: row 4i + g, column c) from the first sweep to the last.  In that
+// layout a tile is also a B operand (register i = k-step i), so a sweep only exchanges the pivot
+// column: its owner inverts the pivot block in registers and publishes the inverse and the
+// negated column panel through LDS (double-buffered: one barrier a sweep); every wave then forms
+// P = inv(A_KK) A_KJ and A_IJ += (-A_IK) P with 4 MFMAs a tile.  The owner's own column takes the
+// same update with P = inv(A_KK) and zero tiles, which leaves -A_IK inv(A_KK).
+//
+// The register-blocked sweeps over LDS that this replaces (8 pivots a sweep) took 105 us for the
+// default network's 104 rows, bound by LDS round trips and three barriers a sweep; this form takes
+// 35 us.  Its floor is the matrix cores' 10 us for 2 n^3 FLOP at FP64 on one CU; the pivot
+// blocks' serial inversions (16 dependent steps each) are most of the rest.
+constexpr int GJ_MAX = 16 * NWAVE;        // rows one workgroup's waves can hold
+constexpr int GJ_TILE = 16 * 17;          // LDS tile, column-major, column stride 17 (bank spread)
+using f64x4 = __attribute__((ext_vector_type(4))) double;
+
+// LDS doubles of the exchange buffers: two generations of inverse + panel
+__host__ __device__ inline int gj_stage_len(int n) { return 2 * ((n + 15) / 16 + 1) * GJ_TILE; }
+
+template <int K> __device__ __forceinline__ double row16_bcast(double v)
+{   // lane k of each row of 16 lanes, to the whole row
+    return __longlong_as_double(__builtin_amdgcn_update_dpp(__double_as_longlong(v), __double_as_longlong(v), 0x150 + K,
+                                                            0xf, 0xf, true));
+}
+template <int R> __device__ __forceinline__ unsigned rows_bcast32(unsigned v)
+{   // row R of 16 lanes, to all four rows
+    const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    const unsigned x = a[R & 1];
+    const auto b = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return b[R >> 1];
+}
+template <int R> __device__ __forceinline__ double rows_bcast(double v)
 {
-    using AT = LUT;          // arithmetic in the storage precision
-    constexpr int B = GJ_B;
-    LDS AT *P = (LDS AT *)stage;   // P[l*B+m] = inv(A_KK)(l, m)
-    for (int kb = 0; kb < n; kb += B) {
-        const int nb = min(B, n - kb);
-        __syncthreads();
-        if (tid() < 64) {   // wave 0: lane r*B + c holds element (r, c) of the pivot block
-            const int r = tid() / B, c = tid() % B;
-            AT a = (r < nb && c < nb) ? (AT)M[(size_t)(kb + c) * ld + kb + r] : (r == c ? (AT)1 : (AT)0);
+    return __hiloint2double((int)rows_bcast32<R>((unsigned)__double2hiint(v)),
+                            (int)rows_bcast32<R>((unsigned)__double2loint(v)));
+}
+// 1/x by the hardware estimate and two Newton steps
+__device__ __forceinline__ double fast_rcp(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+    r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
+    return r;
+}
+// one Gauss-Jordan step on a 16x16 block in the tile layout
+template <int K> __device__ __forceinline__ void gj16_steps(f64x4 &d, int g, int c, bool &bad)
+{
+    if constexpr (K < 16) {
+        const double rowk = rows_bcast<K & 3>(d[K >> 2]);   // a(K, c)
+        const double piv = row16_bcast<K>(rowk);
+        bad |= !(piv == piv) || piv == 0.0 || isinf(piv);
+        const double q = fast_rcp(piv);
+        const double rq = (c == K) ? q : rowk * q;          // row K of the result
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const double colk = row16_bcast<K>(d[i]);       // a(4i + g, K)
+            const double base = (c == K) ? 0.0 : d[i];
+            const double v = __builtin_fma(-colk, rq, base);
+            d[i] = (i == (K >> 2) && g == (K & 3)) ? rq : v;
+        }
+        gj16_steps<K + 1>(d, g, c, bad);
+    }
+}
+
+// A: n x n, column-major, leading dimension n, in LDS; overwritten by its inverse.  `stage`: LDS
+// scratch of gj_stage_len(n) doubles outside A.  Returns nonzero (uniformly) on a zero or
+// non-finite pivot.
+template <typename LUT>
+__device__ __forceinline__ int block_gj_inverse(LDS LUT *A, int n, LDS double *red, LDS double *stage)
+{
+    const int w = __builtin_amdgcn_readfirstlane(tid() >> 6), lane = tid() & 63, g = lane >> 4, c = lane & 15;
+    const int nb = (n + 15) >> 4, gen = (nb + 1) * GJ_TILE;
+    const int col = 16 * w + c;
+    f64x4 t[NWAVE];
+    if (tid() == 0) red[8] = 0.0;
+#pragma unroll
+    for (int I = 0; I < NWAVE; I++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = 16 * I + 4 * i + g;
+            t[I][i] = (row < n && col < n) ? (double)A[col * n + row] : (row == col ? 1.0 : 0.0);
+        }
+    __syncthreads();
+    f64x4 mine = {0.0, 0.0, 0.0, 0.0};   // the owner's inverted pivot block
+    for (int K = -1; K < nb; K++) {
+        const LDS double *inv = stage + (K & 1) * gen, *panel = inv + GJ_TILE;
+        f64x4 P = mine;
+        if (K >= 0) {
+            __syncthreads();
+            if (red[8] != 0.0) return 1;
+            if (w != K && w < nb) {
+                f64x4 b = t[0];
+#pragma unroll
+                for (int I = 1; I < NWAVE; I++)
+                    if (I == K) b = t[I];
+                P = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+                    P = __builtin_amdgcn_mfma_f64_16x16x4f64(inv[17 * (4 * s + g) + c], b[s], P, 0, 0, 0);
+            }
+        }
+        // the next pivot block's owner updates that block first and inverts it while the other
+        // waves' matrix instructions of this sweep run
+        const bool next = w == K + 1 && w < nb;
+        LDS double *ninv = stage + ((K + 1) & 1) * gen, *npanel = ninv + GJ_TILE;
+        if (next) {
+            mine = t[0];
+#pragma unroll
+            for (int I = 1; I < NWAVE; I++)
+                if (I == w) mine = t[I];
+            if (K >= 0) {
+                const LDS double *pw = panel + w * GJ_TILE;
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+                    mine = __builtin_amdgcn_mfma_f64_16x16x4f64(pw[17 * (4 * s + g) + c], P[s], mine, 0, 0, 0);
+            }
             bool bad = false;
+            gj16_steps<0>(mine, g, c, bad);
+            if (bad) red[8] = 1.0;
 #pragma unroll
-            for (int k = 0; k < B; k++) {
-                const AT piv = __shfl(a, k * B + k);
-                const AT rowk = __shfl(a, k * B + c);   // a(k, c)
-                const AT colk = __shfl(a, r * B + k);   // a(r, k)
-                if (!(piv == piv) || piv == (AT)0 || isinf(piv)) bad = true;
-                const AT q = (AT)1 / piv;
-                if (r == k) a = (c == k) ? q : a * q;
-                else a = (c == k) ? -colk * q : a - colk * (rowk * q);
-            }
-            P[r * B + c] = a;
-            if (r < nb && c < nb) M[(size_t)(kb + c) * ld + kb + r] = (LUT)a;
-            if (tid() == 0) red[8] = bad ? 1.0 : 0.0;
+            for (int i = 0; i < 4; i++) ninv[17 * c + 4 * i + g] = mine[i];
         }
-        __syncthreads();
-        if (red[8] != 0.0) return 1;
-        for (int j = tid(); j < n; j += NT) {   // row panel: A_KJ <- inv(A_KK) A_KJ
-            if (j >= kb && j < kb + nb) continue;
-            AT v[B];
+        if (K >= 0 && w < nb) {
 #pragma unroll
-            for (int m = 0; m < B; m++) v[m] = m < nb ? (AT)M[(size_t)j * ld + kb + m] : (AT)0;
+            for (int I = 0; I < NWAVE; I++) {
+                if (I == K) t[I] = P;
+                else if (I < nb && !(next && I == w)) {
 #pragma unroll
-            for (int l = 0; l < B; l++) {
-                AT acc = 0;
-#pragma unroll
-                for (int m = 0; m < B; m++) acc += P[l * B + m] * v[m];
-                if (l < nb) M[(size_t)j * ld + kb + l] = (LUT)acc;
-            }
-        }
-        __syncthreads();
-        const int nt = (n + 3) >> 2;
-        for (int tt = tid(); tt < nt * nt; tt += NT) {   // A_IJ -= A_IK A_KJ outside the pivot block
-            const int ti = tt % nt, tj = tt / nt;
-            const int i0 = 4 * ti, j0 = 4 * tj;
-            if ((i0 < kb + nb && i0 + 4 > kb) || (j0 < kb + nb && j0 + 4 > kb)) continue;
-            AT acc[4][4];
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-#pragma unroll
-                for (int r = 0; r < 4; r++)
-                    acc[r][c] = (i0 + r < n && j0 + c < n) ? (AT)M[(size_t)(j0 + c) * ld + i0 + r] : (AT)0;
-#pragma unroll
-            for (int m = 0; m < B; m++) {
-                if (m < nb) {
-                    AT a[4], b[4];
-#pragma unroll
-                    for (int r = 0; r < 4; r++) a[r] = (i0 + r < n) ? (AT)M[(size_t)(kb + m) * ld + i0 + r] : (AT)0;
-#pragma unroll
-                    for (int c = 0; c < 4; c++) b[c] = (j0 + c < n) ? (AT)M[(size_t)(j0 + c) * ld + kb + m] : (AT)0;
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-#pragma unroll
-                        for (int c = 0; c < 4; c++) acc[r][c] -= a[r] * b[c];
+                    for (int s = 0; s < 4; s++)
+                        t[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(panel[I * GJ_TILE + 17 * (4 * s + g) + c], P[s], t[I],
+                                                                    0, 0, 0);
                 }
             }
-#pragma unroll
-            for (int c = 0; c < 4; c++)
-#pragma unroll
-                for (int r = 0; r < 4; r++)
-                    if (i0 + r < n && j0 + c < n) M[(size_t)(j0 + c) * ld + i0 + r] = (LUT)acc[r][c];
         }
-        __syncthreads();
-        for (int i = tid(); i < n; i += NT) {   // column panel: A_IK <- -A_IK inv(A_KK)
-            if (i >= kb && i < kb + nb) continue;
-            AT c[B];
+        if (next) {
 #pragma unroll
-            for (int l = 0; l < B; l++) c[l] = l < nb ? (AT)M[(size_t)(kb + l) * ld + i] : (AT)0;
+            for (int I = 0; I < NWAVE; I++)
+                if (I < nb && I != w) {
 #pragma unroll
-            for (int m = 0; m < B; m++) {
-                AT acc = 0;
-#pragma unroll
-                for (int l = 0; l < B; l++) acc += c[l] * P[l * B + m];
-                if (m < nb) M[(size_t)(kb + m) * ld + i] = (LUT)(-acc);
-            }
+                    for (int i = 0; i < 4; i++) npanel[I * GJ_TILE + 17 * c + 4 * i + g] = -t[I][i];
+                    t[I] = f64x4{0.0, 0.0, 0.0, 0.0};
+                }
         }
     }
+    // every wave has read A and the last panel
+    __syncthreads();
+#pragma unroll
+    for (int I = 0; I < NWAVE; I++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = 16 * I + 4 * i + g;
+            if (row < n && col < n) A[col * n + row] = (LUT)t[I][i];
+        }
     __syncthreads();
     return 0;
 }
@@ -1669,7 +1724,7 @@ UCG_BIG __device__ int sparse_lu(NetRef N_, const Lds &L, LUT *V, LDS double *re
         }
         clk.mark(TM_LU_SPARSE);
         __syncthreads();
-        if (T > 0) r = block_gj_inverse<LUT>(tl, T, T, red, stage);
+        if (T > 0) r = block_gj_inverse<LUT>(tl, T, red, region + T * T);
         for (int q = tid(); q < T * T; q += NT) V[nsp + q] = tl[q];
     }
     __syncthreads();

@@ -326,7 +326,8 @@ def lds_bytes(tables, staged: bool = True) -> int:
     if staged:
         al = lambda x: (x + 15) & ~15
         stage = lambda nst, lut: al(nst * lut) + al(nsp * 4) + N * 16 + al((N + nlev + 1) * 4) + N * 8 + T * 8
-        c = max(T * T + ((schur_sources(tables) + 7) & ~7) + Npad, (stage(nsp + T * T, 4) + 7) // 8,
+        gj = 2 * ((T + 15) // 16 + 1) * 16 * 17          # exchange buffers of the tail's inversion
+        c = max(T * T + max(((schur_sources(tables) + 7) & ~7) + Npad, gj), (stage(nsp + T * T, 4) + 7) // 8,
                 (stage(nsp, 8) + 7) // 8)
     else:
         c = Npad
@@ -354,5 +355,6 @@ def schur_sources(tables) -> int:
 
 
 def plan_is_staged(tables) -> bool:
-    """Whether the library stages this network's plan in LDS (else it runs it from the workspace)."""
-    return lds_bytes(tables, True) <= LDS_BYTES_PER_CU
+    """Whether the library stages this network's plan in LDS (else it runs it from the workspace):
+    it fits, and the tail fits the waves that invert it in registers (128 rows)."""
+    return lds_bytes(tables, True) <= LDS_BYTES_PER_CU and int(tables.arrays["nw_sizes"][2]) <= 128
