@@ -179,6 +179,18 @@ int upload(NetHandle &h, const T *src, size_t n, const T *&dst)
     return 0;
 }
 
+int upload_program(NetHandle &h, const ucg::Program &P, ucg::DevProg &D)
+{
+    int rc;
+    if ((rc = upload(h, P.slices.data(), P.slices.size(), D.slices)) ||
+        (rc = upload(h, P.wave_ptr.data(), P.wave_ptr.size(), D.wave_ptr)) ||
+        (rc = upload(h, P.hdr.data(), P.hdr.size(), D.hdr)) || (rc = upload(h, P.rec.data(), P.rec.size(), D.rec)))
+        return rc;
+    D.phases = P.phases;
+    D.n_hdr = (int)P.hdr.size();
+    return 0;
+}
+
 NetHandle *get(int handle)
 {
     if (handle < 0 || handle >= (int)g_nets.size() || !g_nets[handle].used) return nullptr;
@@ -187,9 +199,9 @@ NetHandle *get(int handle)
 
 size_t lds_bytes(const ucg::DevNet &N)
 {
-    const int npad = (N.neq + 7) & ~7;
+    const int npad = (N.neq + 7) & ~7, ypad = (N.neq + ucg::YX_N + 7) & ~7;
     const int region = ucg::flux_region_len(N);
-    return sizeof(double) * ((size_t)region + 4 * npad + ucg::RED_LEN + ucg::S_NSCAL + ucg::P_NPARAM);
+    return sizeof(double) * ((size_t)region + ypad + 3 * npad + ucg::RED_LEN + ucg::S_NSCAL + ucg::P_NPARAM);
 }
 
 int ensure_ws(NetHandle &h, size_t bytes)
@@ -781,39 +793,63 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
                 if (idx[q] < 0 || idx[q] >= d->nreac) return fail(UCG_E_ARG, "production/loss reaction index");
         }
     }
-    {   // balanced production/loss sum tasks (chunks of at most GT_CHUNK flux indices)
-        const int GT_CHUNK = 24;
-        struct Task { int start, end, species, kind; };
-        std::vector<Task> tasks;
-        for (int i = 0; i < d->nspec; i++)
-            for (int kind = 0; kind < 2; kind++) {
-                const int *ptr = kind ? d->loss_ptr : d->prod_ptr;
-                for (int a = ptr[i]; a < ptr[i + 1]; a += GT_CHUNK)
-                    tasks.push_back({a, std::min(a + GT_CHUNK, ptr[i + 1]), i, kind});
+    {   // RHS: factor records, the terms with totalSwap, the waves' shares, the species sums
+        int most = 1;
+        for (size_t k = 0; k < R; k++) most = std::max(most, d->nfac[k]);
+        N.rx_w = (most + 3) / 4;
+        std::vector<uint32_t> rx(2 * R * N.rx_w, 0u);
+        std::vector<int> sx;
+        for (size_t k = 0; k < R; k++) {
+            std::vector<unsigned> f;
+            int swaps = 0;
+            for (int m = 0; m < d->nfac[k]; m++) {
+                const int c = d->fac[ucg::MAXFAC * k + m];
+                if (c == ucg::OP_SWAP && !swaps++) continue;
+                f.push_back((unsigned)(c >= 0 ? c
+                                            : d->neq + (c == ucg::OP_BLR ? ucg::YX_BLR : c == ucg::OP_DIVSM ? ucg::YX_ISM : ucg::YX_TSM)));
+                if (c == ucg::FAC_D) f.back() = (unsigned)d->neq - 1;
             }
-        std::vector<int> order(tasks.size());
-        for (size_t t = 0; t < order.size(); t++) order[t] = (int)t;
-        std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-            return tasks[x].end - tasks[x].start > tasks[y].end - tasks[y].start;
-        });
-        std::vector<int> rec(4 * tasks.size()), where(tasks.size());
-        for (size_t t = 0; t < order.size(); t++) {
-            const Task &k = tasks[order[t]];
-            rec[4 * t] = k.start; rec[4 * t + 1] = k.end; rec[4 * t + 2] = k.species; rec[4 * t + 3] = k.kind;
-            where[order[t]] = (int)t;
+            f.resize(4 * N.rx_w, (unsigned)(d->neq + ucg::YX_ONE));
+            if (swaps) {   // last place of the last record, where the RHS looks for it
+                f.back() = (unsigned)(d->neq + ucg::YX_TSM);
+                sx.push_back((int)k);
+            }
+            for (int m = 0; m < 4 * N.rx_w; m++) ucg::put16(&rx[2 * k * N.rx_w], m, f[m]);
         }
-        std::vector<int> sptr(2 * (size_t)d->nspec + 1, 0), stask;
-        for (size_t t = 0; t < tasks.size(); t++) sptr[2 * tasks[t].species + tasks[t].kind + 1]++;
-        for (size_t q = 1; q < sptr.size(); q++) sptr[q] += sptr[q - 1];
-        stask.resize(tasks.size());
-        std::vector<int> fill(sptr.begin(), sptr.end() - 1);
-        for (size_t t = 0; t < tasks.size(); t++)   // tasks were generated in chunk order
-            stask[fill[2 * tasks[t].species + tasks[t].kind]++] = where[t];
-        N.ngt = (int)tasks.size();
-        N.gt_off = (d->nreac + 7) & ~7;
-        if ((rc = upload(h, rec.data(), rec.size(), N.gt_rec))) return rc;
-        if ((rc = upload(h, sptr.data(), sptr.size(), N.gt_sp_ptr))) return rc;
-        if ((rc = upload(h, stask.data(), stask.size(), N.gt_sp_task))) return rc;
+        N.nswt = (int)sx.size();
+        if ((rc = upload(h, rx.data(), rx.size(), N.rx))) return rc;
+        if ((rc = upload(h, sx.data(), sx.size(), N.sx_list))) return rc;
+        // the last wave has the photo rates, the one before it totalSwap and half a share
+        const int rows = (int)(R + 63) / 64;
+        std::vector<int> fx(ucg::NWAVE + 1, rows);
+        const double share = rows / (ucg::NWAVE - 2 + 0.5);
+        for (int w = 0; w < ucg::NWAVE - 1; w++) fx[w] = std::min(rows, (int)std::ceil(share * w));
+        if ((rc = upload(h, fx.data(), fx.size(), N.fx_row))) return rc;
+        std::vector<int> fs, fb;
+        for (int i = 0; i < d->nspec; i++) {
+            if (d->is_surface[i]) fs.insert(fs.end(), {i, d->bulk_partner_of_surface[i]});
+            else if (d->is_bulk[i]) fb.insert(fb.end(), {i, d->surface_partner_of_bulk[i]});
+        }
+        N.nfin_surf = (int)fs.size() / 2;
+        N.nfin_bulk = (int)fb.size() / 2;
+        if ((rc = upload(h, fs.data(), fs.size(), N.fin_surf))) return rc;
+        if ((rc = upload(h, fb.data(), fb.size(), N.fin_bulk))) return rc;
+        if (d->nreac >= 0x8000) return fail(UCG_E_ARG, "more than 32767 reactions");
+        std::vector<std::vector<unsigned>> op(d->nspec);
+        std::vector<int> len;
+        for (int i = 0; i < d->nspec; i++) {   // a reaction's production and loss of one species cancel here
+            std::map<int, int> net;
+            for (int q = d->prod_ptr[i]; q < d->prod_ptr[i + 1]; q++) net[d->prod_idx[q]]++;
+            for (int q = d->loss_ptr[i]; q < d->loss_ptr[i + 1]; q++) net[d->loss_idx[q]]--;
+            for (auto &x : net)
+                for (int k = 0; k < std::abs(x.second); k++) op[i].push_back((unsigned)x.first | (x.second < 0 ? 0x8000u : 0u));
+            len.push_back((int)op[i].size());
+        }
+        ucg::Program P;
+        P.add(ucg::pack_slices(len, ucg::NWAVE), ucg::NWAVE, 1, 2, 4,
+              [&](int it, uint32_t *w) { w[0] = it >= 0 ? (ucg::HDR_VALID | (uint32_t)it) : 0u; },
+              [&](int it, int e, int k, uint32_t *w) { ucg::put16(w, k, e >= 0 ? op[it][e] : (unsigned)d->nreac); }, len);
+        if ((rc = upload_program(h, P, N.pg_sum))) return rc;
     }
     {   // packed term records {n_d, ops[6], nfac}
         std::vector<int> prog(8 * R);

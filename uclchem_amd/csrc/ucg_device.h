@@ -8,6 +8,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "ucg_plan.h"
 
 namespace ucg {
 
@@ -85,6 +86,15 @@ constexpr double NUM_SITES_PER_GRAIN = GRAIN_RADIUS * GRAIN_RADIUS * 1.5e15 * 4.
 constexpr double SURFACE_COVERAGE0 = 0.5 * GAS_DUST_DENSITY_RATIO / NUM_SITES_PER_GRAIN;  // bulkGainFromMantleBuildUp
 constexpr double MIN_ABUND = 1.0e-30;
 
+// A program of the planner (ucg_plan.h) on the device.
+struct DevProg {
+    const int32_t *slices;     // [n][4]
+    const int32_t *wave_ptr;   // [phases][NWAVE + 1]
+    const uint32_t *hdr, *rec;
+    int32_t phases, n_hdr;
+};
+constexpr int NWAVE = NT / 64;
+
 struct DevNet {
     int32_t nspec, neq, nreac, nice, nsurfl, nbulkl, nfp, nswap, nnz, ld;
     const double *alpha, *beta, *gama, *tmin, *tmax, *mass, *rstat;  // rstat [nreac*5]
@@ -93,10 +103,6 @@ struct DevNet {
     const int32_t *facp;   // [nreac*4] factor codes as int16 x 8 (density factors first), -1 padded
     const int32_t *fac_off, *jc_pk;   // partial offsets [nreac+1]; contributions (partial << 4 | coef + 8)
     int32_t npart, npart_pad;         // number of partials; LDS offset of the scratch after them
-    // balanced production/loss sums: tasks {start, end, species, 0 prod | 1 loss} (longest
-    // first), per species the task lists [2i, 2i+1) prod and [2i+1, 2i+2) loss
-    const int32_t *gt_rec, *gt_sp_ptr, *gt_sp_task;
-    int32_t ngt, gt_off;              // task count; LDS offset (after the fluxes) of the partial sums
     const int8_t *extrapolate;
     const int32_t *type_ranges;                                     // [NTYPES*2]
     const int32_t *loss_ptr, *loss_idx, *prod_ptr, *prod_idx, *swap_list;
@@ -120,6 +126,14 @@ struct DevNet {
     const double *gar;
     // static-pattern sparse Newton plan (augmented order of size nw_N = neq + 2)
     int32_t nw_N, nw_ns, nw_T, nw_nsp, nw_nlev, nw_nph, nw_nval;
+    // RHS: factor records (extended-state indices, 4 per 8 bytes, rx_w records a reaction), the
+    // waves' shares of the reactions (64 a row), the terms that carry totalSwap, the
+    // production/loss sums per species, the ice transfer {species, partner}
+    const uint32_t *rx;
+    int32_t rx_w, nswt;
+    const int32_t *fx_row, *sx_list, *fin_surf, *fin_bulk;
+    int32_t nfin_surf, nfin_bulk;
+    DevProg pg_sum;
     int32_t nw_stage;            // 1: factors and solve program are staged in LDS; 0: they stay in the workspace
     const int32_t *nw_perm, *nw_inv, *nw_sp_ptr, *nw_sp_col, *nw_sp_dpos, *nw_lev_ptr, *nw_lev_rows, *nw_ph_ptr;
     const int32_t *nw_tg_slot, *nw_tg_ptr, *nw_tg_div, *nw_pr_l, *nw_pr_u, *nw_jnz_slot, *nw_diag_slot;
@@ -171,9 +185,7 @@ __host__ __device__ inline int flux_region_len(const Net &N)
 {
     const int npad = (N.neq + 7) & ~7, Npad = (N.nw_N + 7) & ~7;
     const int a = N.npart_pad + 2 * npad;
-    const int g = N.gt_off + N.ngt;                  // fluxes + chunk partial sums
-    const int b0 = N.nreac > a ? N.nreac : a;
-    const int b1 = b0 > g ? b0 : g;
+    const int b1 = N.nreac + 1 > a ? N.nreac + 1 : a;     // fluxes and the sums' padding value
     const int b = b1 > NT ? b1 : NT;                 // >= one value per thread (ordered_sum)
     if (!N.nw_stage) return b > Npad ? b : Npad;               // unstaged plan: the work vector only
     // staged tail beside the Schur sources, then beside the exchange buffers of its inversion
@@ -318,6 +330,124 @@ __device__ inline double co_photodiss_dev(double nh2col, double ncocol, double r
     for (int j = 0; j < 7; j++) yy[j] = co_row_spline(j, lognh2);
     const double ssf = co_shielding(yy, lognco);
     return co_rate_from_parts(radfield, ssf, co_scatter(nh2col, ncocol, av));
+}
+
+// Both photodissociation rates at up to four column pairs by one wave: each row of 16 lanes takes
+// the columns its lanes were given (equal within a row) and every lane of the row returns the
+// rates.  The chain of the functions above is cut to one logarithm and one exponential: the lanes
+// of a row evaluate the two columns' logarithms and the H2 optical depth's together, then the
+// scattering terms, the H2 shielding power and the CO shielding power together; the spline knots
+// are one apart (12..18 and 18..23), so intervals come from comparisons and the natural spline's
+// tridiagonal system has constant factors; the dust wavelength is clamped to the first knots.
+static __device__ __constant__ const double c_scat[8][2] = {{1.0, 7.514e-01}, {2.006, 8.490e-01}, {-1.438, 1.013},
+    {7.364e-01, 1.282}, {-5.076e-01, 2.005}, {-5.920e-02, 5.832}, {0.0, 0.0}, {0.0, 0.0}};
+template <int K> __device__ __forceinline__ double row16_bcast(double v)
+{   // lane K of each row of 16 lanes, to the whole row
+    return __longlong_as_double(__builtin_amdgcn_update_dpp(__double_as_longlong(v), __double_as_longlong(v), 0x150 + K,
+                                                            0xf, 0xf, true));
+}
+__device__ __forceinline__ double pick_uniform(double x, double lo, const double *v, int n)
+{   // v[number of knots lo + 1, lo + 2, ... below x], at most n - 1
+    double r = v[0];
+#pragma unroll
+    for (int i = 1; i < n; i++) r = x > lo + i ? v[i] : r;
+    return r;
+}
+__device__ __forceinline__ void photo_rates_wave(double h2col, double cocol, double radfield, double scat1000, double av,
+                                                 double &kh, double &kc)
+{
+    const int l = (int)threadIdx.x & 15, j = l < 7 ? l : 6;
+    double ya[6], yd[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) {
+        ya[k] = c_photo.ya[j][k];
+        yd[k] = c_photo.y2a[j][k];
+    }
+    const double sc_c = c_scat[l & 7][0], sc_k = c_scat[l & 7][1];
+    const double taud = 0.5 * h2col * (double)1.5e-2f * 1.0e-2 / (1.0 / (1000.0 * 1.0e-8));
+    const double larg = l == 0 ? h2col + 1.0 : l == 1 ? cocol + 1.0 : l == 2 ? fabs(h2col) + 1.0
+                      : l == 3 ? fabs(cocol) + 1.0 : taud;
+    const double lg = log10(larg);
+    double lognh2 = row16_bcast<0>(lg), lognco = row16_bcast<1>(lg);
+    const double lw = row16_bcast<2>(lg), lu = row16_bcast<3>(lg), ltau = row16_bcast<4>(lg);
+    if (lognco < 12.0) lognco = 12.0;
+    if (lognh2 < 18.0) lognh2 = 18.0;
+    if (lognco > 18.0) lognco = 18.0;
+    if (lognh2 > 23.0) lognh2 = 23.0;
+    // row j of the 7x6 shielding table at log N(H2) (splin2's first pass)
+    double row;
+    {
+        const double lo = pick_uniform(lognh2, 18.0, ya, 5), hi = pick_uniform(lognh2, 18.0, ya + 1, 5);
+        const double dl = pick_uniform(lognh2, 18.0, yd, 5), dh = pick_uniform(lognh2, 18.0, yd + 1, 5);
+        const double knot[6] = {18.0, 19.0, 20.0, 21.0, 22.0, 23.0};
+        const double b = lognh2 - pick_uniform(lognh2, 18.0, knot, 5), a = pick_uniform(lognh2, 18.0, knot + 1, 5) - lognh2;
+        row = a * lo + b * hi + ((a * a * a - a) * dl + (b * b * b - b) * dh) / 6.0;
+    }
+    double s;   // log10 of the CO shielding (splin2's second pass, along log N(CO))
+    {
+        const double y[7] = {row16_bcast<0>(row), row16_bcast<1>(row), row16_bcast<2>(row), row16_bcast<3>(row),
+                             row16_bcast<4>(row), row16_bcast<5>(row), row16_bcast<6>(row)};
+        // natural spline on unit knots: y2[i] = -0.5/p[i], p[i] = 2 + 0.5 y2[i-1], y2[0] = 0
+        constexpr double c1 = -0.25, c2 = -0.5 / (2.0 + 0.5 * c1), c3 = -0.5 / (2.0 + 0.5 * c2),
+                         c4 = -0.5 / (2.0 + 0.5 * c3), c5 = -0.5 / (2.0 + 0.5 * c4);
+        const double cf[6] = {0.0, c1, c2, c3, c4, c5};
+        double u[7], d2[7];
+        u[0] = 0.0;
+#pragma unroll
+        for (int i = 1; i < 6; i++)   // u = (6 (second difference)/2 - u[i-1]/2)/p, 1/p = -2 cf
+            u[i] = (3.0 * ((y[i + 1] - y[i]) - (y[i] - y[i - 1])) - 0.5 * u[i - 1]) * (-2.0 * cf[i]);
+        d2[6] = 0.0;
+#pragma unroll
+        for (int i = 5; i >= 1; i--) d2[i] = cf[i] * d2[i + 1] + u[i];
+        d2[0] = 0.0;
+        const double knot[7] = {12.0, 13.0, 14.0, 15.0, 16.0, 17.0, 18.0};
+        const double lo = pick_uniform(lognco, 12.0, y, 6), hi = pick_uniform(lognco, 12.0, y + 1, 6);
+        const double dl = pick_uniform(lognco, 12.0, d2, 6), dh = pick_uniform(lognco, 12.0, d2 + 1, 6);
+        const double b = lognco - pick_uniform(lognco, 12.0, knot, 6), a = pick_uniform(lognco, 12.0, knot + 1, 6) - lognco;
+        s = a * lo + b * hi + ((a * a * a - a) * dl + (b * b * b - b) * dh) / 6.0;
+    }
+    // dust optical depth at the mean wavelength, 913.6 to 1076.1 A: knots 910, 950, 1000, 1050, 1110
+    double tl;
+    {
+        double lb = (5675.0 - 200.6 * lw) - (571.6 - 24.09 * lw) * lu + (18.22 - 0.7664 * lw) * (lu * lu);
+        if (lb > 1076.1) lb = 1076.1;
+        if (lb < 913.6) lb = 913.6;
+        double x0 = c_photo.lam[0], x1 = c_photo.lam[1], v0 = c_photo.xl[0], v1 = c_photo.xl[1], e0 = c_photo.xl_d2[0],
+               e1 = c_photo.xl_d2[1];
+#pragma unroll
+        for (int k = 1; k < 4; k++)
+            if (lb > c_photo.lam[k]) {
+                x0 = c_photo.lam[k]; x1 = c_photo.lam[k + 1];
+                v0 = c_photo.xl[k]; v1 = c_photo.xl[k + 1];
+                e0 = c_photo.xl_d2[k]; e1 = c_photo.xl_d2[k + 1];
+            }
+        const double h = x1 - x0, a = (x1 - lb) / h, b = (lb - x0) / h;
+        double xl = a * v0 + b * v1 + ((a * a * a - a) * e0 + (b * b * b - b) * e1) * (h * h) / 6.0;
+        if (xl < 0.0) xl = 0.0;
+        tl = (av / 1.086) * xl;
+    }
+    // one exponential: scattering terms (lanes 0..5), H2 shielding (6), CO shielding (7)
+    constexpr double LN10 = 2.302585092994045684;
+    const double p = taud < 10.0 ? -1.25 : taud < 100.0 ? -1.15 : -1.0667;
+    const double earg = l == 6 ? (taud < 2.0 ? -0.6666667 * taud : p * ltau * LN10) : l == 7 ? s * LN10 : -(sc_k * tl);
+    const double ex = exp(earg);
+    const double term = (l < 6 && -earg >= 100.0) ? 0.0 : (l < 6 ? sc_c * ex : ex);
+    const double t0 = row16_bcast<0>(term);
+    double scat = row16_bcast<1>(term);
+    scat = scat + row16_bcast<2>(term);
+    scat = scat + row16_bcast<3>(term);
+    scat = scat + row16_bcast<4>(term);
+    scat = scat + row16_bcast<5>(term);
+    if (tl < 1.0) scat = t0;
+    double sj = row16_bcast<6>(term);
+    if (taud == 0.0) sj = 1.0;
+    else if (!(taud < 2.0)) sj = (taud < 10.0 ? 0.638 : taud < 100.0 ? 0.505 : 0.344) * sj;
+    const double r = 8.0e7 / (1.7724539 * (1.0 / (1000.0 * 1.0e-8)));
+    const double t = 3.02 * pow(r * 1.0e3, -0.064);   // constants: folded
+    const double uu = sqrt(taud * r) / t;
+    const double sr = r / (t * sqrt(0.78539816 + uu * uu));
+    kh = 5.18e-11 * (radfield / (double)1.7f) * scat1000 * (sj + sr);
+    kc = co_rate_from_parts(radfield, row16_bcast<7>(term), scat);
 }
 
 __device__ inline double c_ionization_dev(double alpha, double gamma, double t, double ncol, double nh2col,

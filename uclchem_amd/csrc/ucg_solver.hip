@@ -140,7 +140,6 @@ __device__ __forceinline__ double wave_max0(double v)   // v >= 0
 // Workgroup reductions with one barrier: each wave's total goes to its slot of a buffer, every
 // wave adds all of them.  A buffer may be used again once a barrier lies between its last use
 // and the next; the call sites use distinct buffers (RED_*) so that this always holds.
-constexpr int NWAVE = NT / 64;
 enum { RED_TS, RED_S, RED_TOTALS, RED_CHARGE, RED_EWT, RED_ACOR, RED_CORR, RED_HIST, RED_NBUF };
 constexpr int RED_FLAGS = 16;                                   // red[0..15]: flags and small scratch
 constexpr int RED_LEN = RED_FLAGS + RED_NBUF * 2 * NWAVE;
@@ -454,155 +453,196 @@ __device__ __forceinline__ double term_value(NetRef N, int k, const double *rate
     return term_from_codes(c, rate[k], y, D, blr, TS, sm);
 }
 
-// RHS f(y) (chemistry.f90:294-352 + the generated GETYDOT, odes.f90).  Input L.y, output
-// L.f; also leaves the pre-transfer surface total in sc[S_SPRE] for the Jacobian.
+// Sum over aligned groups of G lanes (a power of two, uniform); every lane gets its group's sum.
+__device__ __forceinline__ double group_sum(double v, int G)
+{
+    if (G >= 2) v += __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0xB1, 0xf, 0xf, true));
+    if (G >= 4) v += __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x4E, 0xf, 0xf, true));
+    if (G >= 8) v += __shfl_xor(v, 4);
+    if (G >= 16) v += __shfl_xor(v, 8);
+    if (G >= 32) v += __shfl_xor(v, 16);
+    if (G >= 64) v += __shfl_xor(v, 32);
+    return v;
+}
+struct Slice { int row, rows, G, hdr; };
+__device__ __forceinline__ Slice slice_at(const GLB int *slices, int s)
+{
+    return {slices[4 * s], slices[4 * s + 1], slices[4 * s + 2], slices[4 * s + 3]};
+}
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(tid() >> 6); }
+
+// a factor product over the extended state, four factors a record
+__device__ __forceinline__ double term4(uint2 w, double r, const LDS double *y)
+{
+    return r * y[w.x & 0xffff] * (y[w.x >> 16] * (y[w.y & 0xffff] * y[w.y >> 16]));
+}
+__device__ __forceinline__ uint2 ld_uint2(const GLB uint32_t *p, int i)
+{
+    uint2 r;
+    r.x = p[2 * i];
+    r.y = p[2 * i + 1];
+    return r;
+}
+__device__ __forceinline__ double term_of(NetRef N, int k, double r, const LDS double *y)
+{
+    const GLB uint32_t *rx = glb(N.rx);
+    for (int h = 0; h < N.rx_w; h++) r = term4(ld_uint2(rx, k * N.rx_w + h), r, y);
+    return r;
+}
+
+// RHS f(y) (chemistry.f90:294-352 + the generated GETYDOT, odes.f90).  Input L.y (with its
+// constant factor slot set), output L.f; also leaves the pre-transfer surface total in
+// sc[S_SPRE], the fluxes in L.flux and totalSwap/safeMantle in the extended state for the
+// Jacobian.
+//
+// Three parts with a barrier after each.  Fluxes: every term is its rate times at most four
+// entries of the extended state (factors such as 1/safeMantle have slots there), so all lanes
+// run the same instructions; one wave evaluates the photo rates meanwhile and one forms totalSwap
+// and the terms that carry it.  Sums: one slice program over the signed production and loss terms
+// of each species, whose records do not depend on the state.  Ice transfer and totals: one wave.
+// Bound by the LDS gathers and the latency of the three parts: 7.7 us a call (default
+// network), against 17.5 for chunked sums with a second pass over the chunks, workgroup-wide
+// reductions for each total and serial photo-rate splines.
 UCG_BIG __device__ void block_rhs(NetRef N_, const Lds L)
 {
     NetRef N = fresh(N_);
     PhaseClock clk(L);
-    const int neq = N.neq;
+    const int neq = N.neq, w = wave_id(), lane = tid() & 63;
     LDS double *y = L.y, *f = L.f, *flux = L.flux, *sc = L.sc;
     double *rate = L.rate;
     const LDS double *prm = L.prm;
     const double D = y[neq - 1];
-    const double radfield = prm[P_RADFIELD];
     const double sm = fmax(1e-30, y[N.nsurface]);
     const double sbk = fmax(1e-30, y[N.nbulk]);
-    const double blr = fmin(1.0, NUM_SITES_PER_GRAIN / (GAS_DUST_DENSITY_RATIO * sbk));
-    double ts = 0.0;
-    for (int q = tid(); q < N.nswap; q += NT) ts += term_value(N, N.swap_list[q], rate, y, D, blr, 0.0, sm);
-    const double TS = block_sum(ts, L.red, RED_TS);
-    clk.mark(TM_SKIP);
-    // H2 and CO photodissociation depend on the current column densities (chemistry.f90:311-319):
-    // the last wave evaluates them (the seven CO row splines, the scattering term and the H2
-    // rate in separate lanes) and their two fluxes while the other waves take every other flux.
-    if (tid() >= NT - 64) {
-        const int ln = tid() - (NT - 64);
-        const double h2col = 0.5 * y[N.nh2] * D * (sc[S_CS] / 1.0);
-        const double cocol = 0.5 * y[N.nco] * D * (sc[S_CS] / 1.0);
-        double lognh2, lognco;
-        co_log_columns(h2col, cocol, lognh2, lognco);
-        double v = 0.0;
-        if (ln < 7) v = co_row_spline(ln, lognh2);
-        else if (ln == 7) v = co_scatter(h2col, cocol, sc[S_AV]);
-        else if (ln == 8) v = h2_photodiss_dev(h2col, radfield, sc[S_SCAT]);
-        double yy[7];
-#pragma unroll
-        for (int j = 0; j < 7; j++) yy[j] = __shfl(v, j);
-        const double scat = __shfl(v, 7), kh2 = __shfl(v, 8);
-        if (ln == 0) {
-            rate[N.r_co_hv] = co_rate_from_parts(radfield, co_shielding(yy, lognco), scat);
-            rate[N.r_h2_hv] = kh2;
-            flux[N.r_co_hv] = term_value(N, N.r_co_hv, rate, y, D, blr, TS, sm);
-            flux[N.r_h2_hv] = term_value(N, N.r_h2_hv, rate, y, D, blr, TS, sm);
+    const double ism = 1.0 / sm;
+    // every wave writes the same values and reads only after its own writes
+    if (lane == 0) {
+        y[neq + YX_BLR] = fmin(1.0, NUM_SITES_PER_GRAIN / (GAS_DUST_DENSITY_RATIO * sbk));
+        y[neq + YX_ISM] = ism;
+    }
+    if (w == NWAVE - 1) {
+        // H2 and CO photodissociation depend on the current column densities (chemistry.f90:311-319)
+        double kh, kc;
+        photo_rates_wave(0.5 * y[N.nh2] * D * (sc[S_CS] / 1.0), 0.5 * y[N.nco] * D * (sc[S_CS] / 1.0), prm[P_RADFIELD],
+                         sc[S_SCAT], sc[S_AV], kh, kc);
+        if (lane == 0) {
+            rate[N.r_co_hv] = kc;
+            rate[N.r_h2_hv] = kh;
+            flux[N.r_co_hv] = term_of(N, N.r_co_hv, kc, y);
+            flux[N.r_h2_hv] = term_of(N, N.r_h2_hv, kh, y);
+            flux[N.nreac] = 0.0;                       // padding of the sums
         }
+        if (lane == 63) f[neq - 1] = densdot_dev(prm, D);
     } else {
-        const GLB int *fp = glb(N.facp);
-        const GLB double *rg = glb(rate);
-        const int nr = N.nreac;
-        const int w = tid(), nw = NT - 64;
-        const int kh = N.r_h2_hv, kc = N.r_co_hv;
-        for (int k0 = w; k0 < nr; k0 += 4 * nw) {   // four reactions per pass, records loaded up front
-            int4 wr[4];
-            double r[4];
+        if (w == NWAVE - 2) {
+            double ts = 0.0;
+            for (int q = lane; q < N.nswap; q += 64) {
+                const int k = glb(N.swap_list)[q];
+                ts += term_of(N, k, glb(rate)[k], y);
+            }
+            ts = wave_sum(ts);
+            if (lane == 0) y[neq + YX_TSM] = ts * ism;
+            for (int q = lane; q < N.nswt; q += 64) {
+                const int k = glb(N.sx_list)[q];
+                flux[k] = term_of(N, k, glb(rate)[k], y);
+            }
+        }
+        const GLB uint32_t *rx = glb(N.rx);
+        const GLB double *rg = glb((const double *)rate);
+        const int nr = N.nreac, kh = N.r_h2_hv, kc = N.r_co_hv, r1 = glb(N.fx_row)[w + 1];
+        const unsigned tsm = (unsigned)(neq + YX_TSM);
+        if (N.rx_w == 1) {
+            for (int r0 = glb(N.fx_row)[w]; r0 < r1; r0 += 4) {
+                uint2 wr[4];
+                double r[4];
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int k = k0 + u * nw;
-                if (k < nr) {
-                    wr[u] = ld_int4(fp, k);
-                    r[u] = rg[k];
+                for (int u = 0; u < 4; u++) {
+                    const int k = (r0 + u) * 64 + lane, kk = (r0 + u < r1 && k < nr) ? k : 0;
+                    wr[u] = ld_uint2(rx, kk);
+                    r[u] = rg[kk];
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int k = (r0 + u) * 64 + lane;
+                    const double v = term4(wr[u], r[u], y);
+                    if (r0 + u < r1 && k < nr && k != kh && k != kc && (wr[u].y >> 16) != tsm) flux[k] = v;
                 }
             }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int k = k0 + u * nw;
-                if (k < nr && k != kh && k != kc) {
-                    int c[8];
-                    decode_codes(wr[u], c);
-                    flux[k] = term_from_codes(c, r[u], y, D, blr, TS, sm);
-                }
+        } else {
+            for (int r0 = glb(N.fx_row)[w]; r0 < r1; r0++) {
+                const int k = r0 * 64 + lane;
+                if (k < nr && k != kh && k != kc && (rx[2 * (k * N.rx_w + N.rx_w - 1) + 1] >> 16) != tsm)
+                    flux[k] = term_of(N, k, rg[k], y);
             }
         }
     }
     __syncthreads();
     clk.mark(TM_RHS_FLUX);
-    // production and loss sums in balanced chunks (partial sums in LDS after the fluxes),
-    // then per species in chunk order
-    LDS double *part = flux + N.gt_off;
     {
-        const GLB int *gr = glb(N.gt_rec);
-        const GLB int *lidx = glb(N.loss_idx), *pidx = glb(N.prod_idx);
-        for (int t = tid(); t < N.ngt; t += NT) {
-            const int4 rc = ld_int4(gr, t);
-            const GLB int *src = rc.w ? lidx : pidx;
-            double acc = 0.0;
-#pragma unroll 8
-            for (int q = rc.x; q < rc.y; q++) acc += flux[src[q]];
-            part[t] = acc;
+        const GLB uint32_t *rec = glb(N.pg_sum.rec), *hdr = glb(N.pg_sum.hdr);
+        const GLB int *slices = glb(N.pg_sum.slices);
+        const int s1 = glb(N.pg_sum.wave_ptr)[w + 1];
+        for (int s = glb(N.pg_sum.wave_ptr)[w]; s < s1; s++) {
+            const Slice sl = slice_at(slices, s);
+            const uint32_t h = hdr[sl.hdr + lane];
+            double a0 = 0.0, a1 = 0.0;
+#pragma unroll 2
+            for (int r = 0; r < sl.rows; r++) {
+                const uint2 q = ld_uint2(rec, (sl.row + r) * 64 + lane);
+                const auto val = [&](unsigned e) {
+                    const double v = flux[e & 0x7fff];
+                    return __hiloint2double(__double2hiint(v) ^ (int)((e & 0x8000u) << 16), __double2loint(v));
+                };
+                a0 += val(q.x);
+                a1 += val(q.x >> 16);
+                a0 += val(q.y);
+                a1 += val(q.y >> 16);
+            }
+            const double acc = group_sum(a0 + a1, sl.G);
+            if (h & HDR_VALID) f[h & HDR_INDEX] = acc;
         }
     }
     __syncthreads();
     clk.mark(TM_RHS_SUMS);
-    double pre[EPT];
-    double spre = 0.0;
-#pragma unroll
-    for (int e = 0; e < EPT; e++) {
-        const int i = tid() + e * NT;
-        pre[e] = 0.0;
-        if (i < N.nspec) {
-            double prod = 0.0, loss = 0.0;
-            const GLB int *spp = glb(N.gt_sp_ptr), *spt = glb(N.gt_sp_task);
-            const int q0 = spp[2 * i], q1 = spp[2 * i + 1], q2 = spp[2 * i + 2];
-            for (int q = q0; q < q1; q++) prod += part[spt[q]];
-            for (int q = q1; q < q2; q++) loss += part[spt[q]];
-            pre[e] = prod - loss;
-            if (N.is_surface[i]) spre += pre[e];
-        }
-    }
-    const double S = block_sum(spre, L.red, RED_S);
-    double tb = 0.0, tsu = 0.0;
-    double out[EPT];
-#pragma unroll
-    for (int e = 0; e < EPT; e++) {
-        const int i = tid() + e * NT;
-        out[e] = pre[e];
-        if (i < N.nspec) {
-            // bulk<->surface transfer (odes.f90:4818-5153)
-            if (N.is_surface[i]) {
-                const int b = N.bulk_partner_of_surface[i];
-                if (b >= 0) {
-                    if (S < 0) out[e] = out[e] - S * fmin(1.0, sbk / sm) * y[b] / sbk;
-                    else out[e] = out[e] - S * SURFACE_COVERAGE0 * y[i];
-                }
-                tsu += out[e];
-            } else if (N.is_bulk[i]) {
-                const int s = N.surface_partner_of_bulk[i];
-                if (S < 0) out[e] = out[e] + S * fmin(1.0, sbk / sm) * y[i] / sbk;
-                else out[e] = out[e] + S * SURFACE_COVERAGE0 * y[s];
-                tb += out[e];
-            }
-        }
-    }
-    block_sum2(tb, tsu, L.red, RED_TOTALS);
-#pragma unroll
-    for (int e = 0; e < EPT; e++) {
-        const int i = tid() + e * NT;
-        if (i < neq) {
-            double v = out[e];
-            if (i == N.nbulk) v = tb;
-            if (i == N.nsurface) v = tsu;
-            if (i == neq - 1) v = densdot_dev(prm, D);
+    if (w == 0) {
+        // bulk<->surface transfer (odes.f90:4818-5153), then the BULK and SURFACE totals
+        const GLB int *ls = glb(N.fin_surf), *lb = glb(N.fin_bulk);
+        double S = 0.0;
+        for (int q = lane; q < N.nfin_surf; q += 64) S += f[ls[2 * q]];
+        S = wave_sum(S);
+        const bool neg = S < 0;
+        const double fb = neg ? S * fmin(1.0, sbk / sm) / sbk : 0.0, fs = S * SURFACE_COVERAGE0;
+        double tsu = 0.0, tb = 0.0;
+        for (int q = lane; q < N.nfin_surf; q += 64) {
+            const int i = ls[2 * q], b = ls[2 * q + 1];
+            double v = f[i];
+            if (b >= 0) v -= neg ? fb * y[b] : fs * y[i];
             f[i] = v;
+            tsu += v;
+        }
+        for (int q = lane; q < N.nfin_bulk; q += 64) {
+            const int i = lb[2 * q], s = lb[2 * q + 1];
+            const double v = f[i] + (neg ? fb * y[i] : s >= 0 ? fs * y[s] : 0.0);
+            f[i] = v;
+            tb += v;
+        }
+        tsu = wave_sum(tsu);
+        tb = wave_sum(tb);
+        if (lane == 0) {
+            f[N.nbulk] = tb;
+            f[N.nsurface] = tsu;
+            sc[S_SPRE] = S;
         }
     }
-    if (tid() == 0) sc[S_SPRE] = S;
     __syncthreads();
     if (prm[P_ENFORCECHARGE] != 0.0 && N.nelec < N.nspec) {
         // enforceChargeConservation: ydot(e-) is the sum of the positive-ion rows (chemistry.f90:333-335)
-        double e = 0.0;
-        for (int q = tid(); q < N.nion; q += NT) e += f[N.ion_list[q]];
-        e = block_sum(e, L.red, RED_CHARGE);
-        if (tid() == 0) f[N.nelec] = e;
+        if (w == 0) {
+            double e = 0.0;
+            for (int q = lane; q < N.nion; q += 64) e += f[glb(N.ion_list)[q]];
+            e = wave_sum(e);
+            if (lane == 0) f[N.nelec] = e;
+        }
         __syncthreads();
     }
     clk.mark(TM_RHS_TOTALS);
@@ -1170,11 +1210,6 @@ using f64x4 = __attribute__((ext_vector_type(4))) double;
 // LDS doubles of the exchange buffers: two generations of inverse + panel
 __host__ __device__ inline int gj_stage_len(int n) { return 2 * ((n + 15) / 16 + 1) * GJ_TILE; }
 
-template <int K> __device__ __forceinline__ double row16_bcast(double v)
-{   // lane k of each row of 16 lanes, to the whole row
-    return __longlong_as_double(__builtin_amdgcn_update_dpp(__double_as_longlong(v), __double_as_longlong(v), 0x150 + K,
-                                                            0xf, 0xf, true));
-}
 template <int R> __device__ __forceinline__ unsigned rows_bcast32(unsigned v)
 {   // row R of 16 lanes, to all four rows
     const auto a = __builtin_amdgcn_permlane16_swap(v, v, false, false);
@@ -1753,14 +1788,6 @@ __device__ __forceinline__ double row_dot(VP V, IP cols, const LDS double *w, in
     }
     if (e < e1) a0 += (double)V[e] * w[cols[e]];
     return a0 + a1;
-}
-
-// Sum over an aligned group of G lanes (G a power of two <= 64); every lane of the wave
-// takes part, each lane ends with its group's sum.
-__device__ __forceinline__ double group_sum(double v, int G)
-{
-    for (int off = G >> 1; off > 0; off >>= 1) v += __shfl_xor(v, off);
-    return v;
 }
 
 // Level-scheduled substitutions of the static plan on the permuted work vector w (LDS):
@@ -2375,13 +2402,14 @@ __device__ void lds_layout(NetRef N, Lds &L, double *lds_raw, double *rate)
     L.rate = rate;
     L.flux = (LDS double *)lds_raw;
     L.y = L.flux + flux_region_len(N);
-    L.f = L.y + npad;
+    L.f = L.y + ((N.neq + YX_N + 7) & ~7);
     L.b = L.f + npad;
     L.g = L.b + npad;
     L.red = L.g + npad;
     L.sc = L.red + RED_LEN;
     L.prm = L.sc + S_NSCAL;
     L.timed = 0;
+    if (tid() == 0) L.y[N.neq + YX_ONE] = 1.0;   // the padding factor of the reaction terms
 }
 
 // Resets the work counter and the cancel flag and marks every point "not run" before a

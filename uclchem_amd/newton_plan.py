@@ -312,7 +312,7 @@ LDS_BYTES_PER_CU = 160 * 1024
 
 def lds_bytes(tables, staged: bool = True) -> int:
     """LDS one solve workgroup needs (mirror of lds_bytes/flux_region_len in the HIP
-    library): the shared region (fluxes and gather partials, Jacobian term partials, and
+    library): the shared region (fluxes, Jacobian term partials, and
     for a staged plan the staged factors, solve program and dense tail) plus the NEQ-long
     vectors, reduction slots, scalars and parameters."""
     a = tables.arrays
@@ -321,8 +321,7 @@ def lds_bytes(tables, staged: bool = True) -> int:
     npad = (tables.neq + 7) & ~7
     Npad = (N + 7) & ~7
     npart = int(a["nfac"].sum())
-    ngt = sum(int(np.sum((np.diff(a[k]) + 23) // 24)) for k in ("prod_ptr", "loss_ptr"))
-    b = max(tables.nreac, ((npart + 7) & ~7) + 2 * npad, ((tables.nreac + 7) & ~7) + ngt)
+    b = max(tables.nreac + 1, ((npart + 7) & ~7) + 2 * npad, 512)
     if staged:
         al = lambda x: (x + 15) & ~15
         stage = lambda nst, lut: al(nst * lut) + al(nsp * 4) + N * 16 + al((N + nlev + 1) * 4) + N * 8 + T * 8
@@ -332,7 +331,7 @@ def lds_bytes(tables, staged: bool = True) -> int:
     else:
         c = Npad
     from .params import NPARAM
-    return 8 * (max(b, c) + 4 * npad + 144 + 40 + NPARAM)   # + reduction slots, scalars, parameters
+    return 8 * (max(b, c) + ((tables.neq + 4 + 7) & ~7) + 3 * npad + 144 + 40 + NPARAM)   # + reduction slots, scalars, parameters
 
 
 def schur_sources(tables) -> int:
