@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -286,22 +287,37 @@ int check_params(int n, const double *params)
     return 0;
 }
 
-// Bytes of one workgroup slot's workspace: the Newton matrix (FP64 or FP32), the saved
-// J-form values of the sparse plan, and the rate coefficients, each 256-byte aligned.
+// Bytes of one workgroup slot's workspace: the Newton matrix or its factors (FP64 or FP32), the
+// sparse plan's second workspace (tail entries of a staged plan, J-form values of one that runs
+// from the workspace), and the rate coefficients, each 256-byte aligned.
 struct SlotLayout {
     size_t mat, jac, stride;
 };
 
+SlotLayout slot_layout(const ucg::DevNet &N, bool sparse, int lu_bits)
+{
+    const size_t elem = lu_bits == 64 ? sizeof(double) : sizeof(float);
+    const auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    SlotLayout s;
+    // the dense matrix, or a plan run from the workspace: its values and their J-form
+    s.mat = al((sparse ? (size_t)N.nw_nval : (size_t)N.ld * N.neq) * elem);
+    s.jac = sparse ? al((size_t)N.nw_nval * sizeof(double)) : 0;
+    size_t both = s.mat + s.jac;
+    if (sparse && N.nw_stage) {
+        // a staged plan's factors and waiting tail entries need less; the slot keeps that size, so
+        // that a budget or the fixed workspace holds the same number of slots either way
+        s.mat = al(((size_t)N.sp_nstream + ucg::tail_len(N.sp_T)) * elem);
+        s.jac = al((size_t)(N.pg_entries.n_hdr - N.sp_tail_hdr) * sizeof(double));
+        both = std::max(both, s.mat + s.jac);
+        s.jac = both - s.mat;
+    }
+    s.stride = both + al((size_t)N.nreac * sizeof(double));
+    return s;
+}
+
 SlotLayout slot_layout(const NetHandle &h, int lu_bits)
 {
-    const ucg::DevNet &N = h.dev;
-    const size_t elem = lu_bits == 64 ? sizeof(double) : sizeof(float);
-    const bool sparse = h.linear_solver == UCG_LINSOL_SPARSE;
-    SlotLayout s;
-    s.mat = (((sparse ? (size_t)N.nw_nval : (size_t)N.ld * N.neq) * elem) + 255) & ~(size_t)255;
-    s.jac = sparse ? (((size_t)N.nw_nval * sizeof(double) + 255) & ~(size_t)255) : 0;
-    s.stride = s.mat + s.jac + (((size_t)N.nreac * sizeof(double) + 255) & ~(size_t)255);
-    return s;
+    return slot_layout(h.dev, h.linear_solver == UCG_LINSOL_SPARSE, lu_bits);
 }
 
 int launch_kernel(const ucg::DevNet &N, const ucg::DevNet *dN, const ucg::SolveArgs &A, int n_slots, int lu_bits,
@@ -399,9 +415,9 @@ int piece_common(NetHandle &h, int n, const double *params, const double *phys, 
     A.n = n;
     A.params = (const double *)dp.p;
     A.phys = (const double *)dph.p;
-    const size_t mat = ((size_t)N.ld * N.neq * sizeof(double) + 255) & ~(size_t)255;
-    const size_t jac = ((size_t)N.nw_nval * sizeof(double) + 255) & ~(size_t)255;
-    const size_t stride = mat + jac + (((size_t)N.nreac * sizeof(double) + 255) & ~(size_t)255);
+    const SlotLayout dense = slot_layout(N, false, 64), sparse = slot_layout(N, true, 64);
+    const size_t mat = std::max(dense.mat, sparse.mat), jac = sparse.jac;
+    const size_t stride = mat + jac + (dense.stride - dense.mat);
     if ((rc = ensure_ws(h, stride * n))) return rc;
     A.ws = h.ws;
     A.ws_stride = stride;
@@ -723,6 +739,48 @@ int ucg_network_load_file(const char *path, int *handle)
     return ucg_network_load(&d, handle);
 }
 
+// The staged form of the sparse plan, when its tail fits the workgroup's registers and its working
+// set the device's LDS; otherwise the plan runs from the workspace (nw_stage = 0).
+static int load_staged_plan(const ucg_network_desc *d, NetHandle &h, size_t lds_limit)
+{
+    ucg::DevNet &N = h.dev;
+    N.nw_stage = 0;
+    std::vector<int> foff((size_t)d->nreac + 1, 0);
+    for (int k = 0; k < d->nreac; k++) foff[k + 1] = foff[k] + d->nfac[k];
+    ucg::SparsePrograms S;
+    try {
+        S = ucg::build_sparse_programs(d, ucg::NWAVE, ucg::GJ_MAX, foff, foff.back());
+    } catch (const std::exception &) {   // a pattern the planner cannot follow: run the given schedule
+        S.ok = false;
+    }
+    if (!S.ok) return 0;
+    N.px = ucg::partial_slots(foff.back(), N.nswt, d->nswap, d->nsurfl);
+    N.sp_ns = S.ns;
+    N.sp_T = S.t;
+    N.sp_nstream = (int)S.stream.size();
+    N.sp_L = S.at_L;
+    N.sp_tail_hdr = S.tail_hdr;
+    N.sp_slots = S.n_slots;
+    for (int k = 0; k < 4; k++) N.sp_at[k] = S.at[k];
+    N.sp_w0 = std::max(N.px.n, S.t * S.t - S.at_L);   // the tail must end before L21
+    N.sp_presum = S.presum ? 1 : 0;
+    N.nw_stage = 1;
+    if (lds_bytes(N) > lds_limit) {
+        N.nw_stage = 0;
+        return 0;
+    }
+    int rc;
+    if ((rc = upload(h, S.stream.data(), S.stream.size(), N.sp_stream)) ||
+        (rc = upload(h, S.sum_rows.data(), S.sum_rows.size(), N.sp_sum_rows)) ||
+        (rc = upload(h, S.sum_members.data(), S.sum_members.size(), N.sp_sum_members)) ||
+        (rc = upload_program(h, S.entries, N.pg_entries)) || (rc = upload_program(h, S.elim, N.pg_elim)) ||
+        (rc = upload_program(h, S.schur, N.pg_schur)))
+        return rc;
+    for (int k = 0; k < 4; k++)
+        if ((rc = upload_program(h, S.solve[k], N.pg_solve[k]))) return rc;
+    return 0;
+}
+
 // Uploads a network whose tables check_tables and check_plan have accepted.
 static int load_tables(const ucg_network_desc *d, NetHandle &h)
 {
@@ -797,7 +855,7 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
         int most = 1;
         for (size_t k = 0; k < R; k++) most = std::max(most, d->nfac[k]);
         N.rx_w = (most + 3) / 4;
-        std::vector<uint32_t> rx(2 * R * N.rx_w, 0u);
+        std::vector<uint32_t> rx(2 * R * N.rx_w, 0u), rp(2 * R * N.rx_w, 0u);
         std::vector<int> sx;
         for (size_t k = 0; k < R; k++) {
             std::vector<unsigned> f;
@@ -810,6 +868,13 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
                 if (c == ucg::FAC_D) f.back() = (unsigned)d->neq - 1;
             }
             f.resize(4 * N.rx_w, (unsigned)(d->neq + ucg::YX_ONE));
+            for (int m = 0; m < 4 * N.rx_w; m++) {   // term order, as the partials are numbered
+                const int c = m < d->nfac[k] ? d->fac[ucg::MAXFAC * k + m] : ucg::OP_NONE;
+                ucg::put16(&rp[2 * k * N.rx_w], m,
+                           (unsigned)(c >= 0 ? c : c == ucg::FAC_D ? d->neq - 1
+                                      : d->neq + (c == ucg::OP_BLR ? ucg::YX_BLR : c == ucg::OP_DIVSM ? ucg::YX_ISM
+                                                  : c == ucg::OP_SWAP ? ucg::YX_TSM : ucg::YX_ONE)));
+            }
             if (swaps) {   // last place of the last record, where the RHS looks for it
                 f.back() = (unsigned)(d->neq + ucg::YX_TSM);
                 sx.push_back((int)k);
@@ -817,7 +882,7 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
             for (int m = 0; m < 4 * N.rx_w; m++) ucg::put16(&rx[2 * k * N.rx_w], m, f[m]);
         }
         N.nswt = (int)sx.size();
-        if ((rc = upload(h, rx.data(), rx.size(), N.rx))) return rc;
+        if ((rc = upload(h, rx.data(), rx.size(), N.rx)) || (rc = upload(h, rp.data(), rp.size(), N.rp))) return rc;
         if ((rc = upload(h, sx.data(), sx.size(), N.sx_list))) return rc;
         // the last wave has the photo rates, the one before it totalSwap and half a share
         const int rows = (int)(R + 63) / 64;
@@ -939,30 +1004,6 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
             pr[2 * q + 1] = pu[q];
         }
         if ((rc = upload(h, pr.data(), pr.size(), N.nw_pr))) return rc;
-        {   // sources of the last phase when it is the pure Schur update of the tail
-            const int *pp = d->nw_ph_ptr;
-            const long t0 = pp[nph - 1], t1 = pp[nph];
-            const long q0 = tptr[t0], q1 = tptr[t1];
-            bool ok = nph >= 2 && q1 > q0;
-            for (long t = t0; t < t1 && ok; t++) ok = tslot[t] >= (int)nsp && tdiv[t] < 0;
-            for (long q = q0; q < q1 && ok; q++) ok = pl[q] < (int)nsp && pu[q] < (int)nsp;
-            N.nlp_src = 0;
-            if (ok) {
-                std::vector<int> local(nsp, -1), src, lpp(2 * (q1 - q0));
-                for (long q = q0; q < q1; q++)
-                    for (int h2 = 0; h2 < 2; h2++) {
-                        const int sl = h2 ? pu[q] : pl[q];
-                        if (local[sl] < 0) {
-                            local[sl] = (int)src.size();
-                            src.push_back(sl);
-                        }
-                        lpp[2 * (q - q0) + h2] = local[sl];
-                    }
-                N.nlp_src = (int)src.size();
-                if ((rc = upload(h, src.data(), src.size(), N.lp_src))) return rc;
-                if ((rc = upload(h, lpp.data(), lpp.size(), N.lp_pr))) return rc;
-            }
-        }
         std::vector<signed char> uns((size_t)N.nw_nval, 0);
         for (size_t i = 0; i < Q; i++) {
             if (d->nw_s1c[i] >= 0) uns[d->nw_s1c[i]] = 1;
@@ -994,8 +1035,7 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
     HIPCHK(hipMemset(h.cancel, 0, sizeof(int)));
     hipDeviceProp_t prop;
     HIPCHK(hipGetDeviceProperties(&prop, g_device));
-    if (lds_bytes(N) > (size_t)prop.sharedMemPerBlock || N.nw_T > ucg::GJ_MAX)
-        N.nw_stage = 0;   // factors stay in the workspace
+    if ((rc = load_staged_plan(d, h, (size_t)prop.sharedMemPerBlock))) return rc;
     size_t lds = lds_bytes(N);
     if (lds > (size_t)prop.sharedMemPerBlock)
         return fail(UCG_E_ARG, "network needs " + std::to_string(lds) + " B of LDS per workgroup, device allows " +

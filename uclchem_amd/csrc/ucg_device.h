@@ -129,12 +129,19 @@ struct DevNet {
     // RHS: factor records (extended-state indices, 4 per 8 bytes, rx_w records a reaction), the
     // waves' shares of the reactions (64 a row), the terms that carry totalSwap, the
     // production/loss sums per species, the ice transfer {species, partner}
-    const uint32_t *rx;
+    const uint32_t *rx, *rp;   // rp: the same in term order (the partials' order)
     int32_t rx_w, nswt;
     const int32_t *fx_row, *sx_list, *fin_surf, *fin_bulk;
     int32_t nfin_surf, nfin_bulk;
     DevProg pg_sum;
-    int32_t nw_stage;            // 1: factors and solve program are staged in LDS; 0: they stay in the workspace
+    // Newton matrix of a staged plan: operand slots, entries, elimination, Schur update, solves
+    PartialSlots px;
+    int32_t sp_ns, sp_T, sp_nstream, sp_L, sp_slots, sp_at[4], sp_w0, sp_presum;
+    int32_t sp_tail_hdr;         // first header of the tail entries; their values wait in the workspace from there on
+    const uint32_t *sp_stream;
+    const int32_t *sp_sum_rows, *sp_sum_members;
+    DevProg pg_entries, pg_elim, pg_schur, pg_solve[4];
+    int32_t nw_stage;            // 1: the plan runs from LDS and matrix-core registers; 0: from the workspace
     const int32_t *nw_perm, *nw_inv, *nw_sp_ptr, *nw_sp_col, *nw_sp_dpos, *nw_lev_ptr, *nw_lev_rows, *nw_ph_ptr;
     const int32_t *nw_tg_slot, *nw_tg_ptr, *nw_tg_div, *nw_pr_l, *nw_pr_u, *nw_jnz_slot, *nw_diag_slot;
     const int32_t *nw_ph_slot, *nw_tr_slot, *nw_s1c, *nw_s1r, *nw_s2c, *nw_s2r, *nw_gs_ptr, *nw_gs_slot;
@@ -143,11 +150,6 @@ struct DevNet {
     const int32_t *nw_erow, *nw_eion;   // then of its entries in the positive-ion columns
     const int32_t *sv_rec;   // solve rows {row, first, diagonal, end}: sparse rows in level order, then tail rows
     const int32_t *nw_pr;    // Crout pairs interleaved {L slot, U slot}
-    // the last elimination phase is the Schur-complement update of the dense tail; its
-    // sources (sparse factor entries) are gathered into LDS beside the staged tail
-    int32_t nlp_src;          // number of distinct source entries (0: the phase runs in place)
-    const int32_t *lp_src;    // [nlp_src] factor slots of the sources
-    const int32_t *lp_pr;     // the phase's pairs as {source index, source index}
     const int8_t *nw_unscaled;   // [nval] 1 where the Newton matrix takes the J-form value without gamma
 };
 
@@ -163,39 +165,24 @@ __device__ __forceinline__ NetRef fresh(NetRef N)
     return *(const CST DevNet *)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
 }
 
-// LDS bytes the sparse solve stages: factors (lut bytes each; FP32 all of them, FP64 the
-// sparse part), column indices, row records, permutation, work vector and the dense-tail
-// product's scratch (16-byte aligned parts)
-template <class Net>
-__host__ __device__ inline int solve_stage_bytes(const Net &N, int lut)
-{
-    const int nst = lut == 4 ? N.nw_nval : N.nw_nsp;
-    auto al = [](int x) { return (x + 15) & ~15; };
-    return al(nst * lut) + al(N.nw_nsp * 4) + N.nw_N * 16 + al((N.nw_N + N.nw_nlev + 1) * 4) + N.nw_N * 8 +
-           N.nw_T * 8;
-}
-
-// length (in doubles) of the LDS region shared by the reaction fluxes (RHS), the term
-// partials plus two NEQ-long scratch vectors (Jacobian assembly), and the staged factors
-// (all of them in FP32, the dense tail in FP64) plus the permuted work vector.  Plans too
-// large to stage (strongly coupled networks with a wide dense tail) keep their factors in
-// the workspace and need only the work vector here.
+// length (in doubles) of the LDS region the phases share: the reaction fluxes (RHS); the operands
+// of the Newton-matrix entries with the sparse pivots' working slots behind them; the dense tail,
+// which overlays both but for the L21 and U12 streams at the end; the exchange buffers of the
+// tail's inversion; the solve's three vectors.  Plans whose tail does not fit (strongly coupled
+// networks) keep their factors in the workspace and need the term partials and a work vector.
 template <class Net>
 __host__ __device__ inline int flux_region_len(const Net &N)
 {
     const int npad = (N.neq + 7) & ~7, Npad = (N.nw_N + 7) & ~7;
     const int a = N.npart_pad + 2 * npad;
-    const int b1 = N.nreac + 1 > a ? N.nreac + 1 : a;     // fluxes and the sums' padding value
+    const int b0 = N.nreac + 1 > a ? N.nreac + 1 : a;
+    const int b1 = b0 > 3 * Npad ? b0 : 3 * Npad;
     const int b = b1 > NT ? b1 : NT;                 // >= one value per thread (ordered_sum)
-    if (!N.nw_stage) return b > Npad ? b : Npad;               // unstaged plan: the work vector only
-    // staged tail beside the Schur sources, then beside the exchange buffers of its inversion
-    const int gj = 2 * ((N.nw_T + 15) / 16 + 1) * 16 * 17;
-    const int beside = ((N.nlp_src + 7) & ~7) + Npad > gj ? ((N.nlp_src + 7) & ~7) + Npad : gj;
-    const int t64 = N.nw_T * N.nw_T + beside;
-    const int s32 = (solve_stage_bytes(N, 4) + 7) / 8, s64 = (solve_stage_bytes(N, 8) + 7) / 8;
-    const int f = s32 > s64 ? s32 : s64;
-    const int c = t64 > f ? t64 : f;
-    return b > c ? b : c;
+    if (!N.nw_stage) return b;
+    const int c = N.sp_w0 + N.sp_slots;
+    const int gj = N.sp_T * N.sp_T + 2 * ((N.sp_T + 15) / 16 + 1) * 16 * 17;
+    const int e = c > gj ? c : gj;
+    return b > e ? b : e;
 }
 
 // static spline tables of the photo-rate functions (photoreactions.f90:14-39),

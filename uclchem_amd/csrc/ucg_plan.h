@@ -176,17 +176,20 @@ enum : uint32_t { ENTRY_TARGET = 0x7fffffu, ENTRY_TAIL = 1u << 23, ENTRY_UNSCALE
 enum : uint32_t { HDR_INDEX = 0xffffffu, HDR_RECIP = 1u << 30, HDR_VALID = 1u << 31 };
 constexpr unsigned NO_SLOT = 0xffffu;
 
-// Working slots of the sparse pivots in LDS, in order: scratch entries of L11 and U11 (with the
-// constants 1 and -1), then the four streams the solves read, in their slices' order: T = -inv(L11)
-// below the diagonal, X = inv(U11), L21, U12; then a zero.  The tail (t x t) overlays everything
-// before L21 once those streams are stored.
+// Working slots of the sparse pivots in LDS, in order: the constants 1 and -1 and the scratch
+// entries of L11 and U11; T = -inv(L11) below the diagonal; X = inv(U11); from slot at_L on L21,
+// U12 and a zero.  The tail (t x t) overlays everything before at_L once the factors are stored.
+// They are stored as four streams in the order the solves' slices read them, padded: stream
+// element q takes slot[q] & 0xffff, times slot[q] >> 16 unless that is NO_SLOT; stream k starts at
+// at[k].
 struct SparsePrograms {
     int ns = 0, t = 0, nlev = 0;
-    int n_work = 0, at_T = 0, at_X = 0, at_L = 0, at_U = 0, zero = 0, n_slots = 0;
+    int at_L = 0, zero = 0, n_slots = 0, tail_hdr = 0;
+    int at[4] = {0, 0, 0, 0};
+    std::vector<uint32_t> stream;
     bool presum = false;              // the sum rows are not all tail rows: subtract sums up front
     std::vector<int> sum_rows;        // presum: {row, first, end} of the permuted members
     std::vector<int> sum_members;
-    std::vector<int> scale;           // [stream slots] slot to multiply by, -1 none
     Program elim, schur, entries, solve[4];   // solve: T, X, L21, U12
     bool ok = false;
 };
@@ -217,11 +220,29 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
             if (c > r) Ucol[c].push_back(r);
         }
     };
-    for (int r = 0; r < NN; r++)
-        for (int q = d->nw_sp_ptr[r]; q < d->nw_sp_ptr[r + 1]; q++) {
-            const int c = d->nw_sp_col[q];
+    for (int r = 0; r < NN; r++) {
+        const std::set<int> cols(d->nw_sp_col + d->nw_sp_ptr[r], d->nw_sp_col + d->nw_sp_ptr[r + 1]);
+        for (int c : cols)
             if (std::min(r, c) < ns) pivot_row(r, c);
+    }
+    // the pattern must hold its own fill (and every pivot), or the caller's schedule is used as it is
+    {
+        std::set<std::pair<int, int>> has;
+        std::vector<std::vector<int>> Lcol(ns);
+        for (int r = 0; r < NN; r++)
+            for (int c : Lrow[r]) {
+                has.insert({r, c});
+                Lcol[c].push_back(r);
+            }
+        for (int r = 0; r < ns; r++) {
+            for (int c : Urow[r]) has.insert({r, c});
+            if (!has.count({r, r})) return S;
         }
+        for (int p = 0; p < ns; p++)
+            for (int r : Lcol[p])
+                for (int c : Urow[p])
+                    if (c > p && std::min(r, c) < ns && !has.count({r, c})) return S;
+    }
     std::vector<int> level(ns, 0);
     for (int k = 0; k < ns; k++) {
         for (int p : Lrow[k]) level[k] = std::max(level[k], level[p] + 1);
@@ -261,9 +282,9 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
         S.sum_members.insert(S.sum_members.end(), x.second.begin(), x.second.end());
         S.sum_rows.push_back((int)S.sum_members.size());
     }
-    // solve phases: rows and their operands (the stored value's place is its slot)
+    // solve phases: rows and their operands
     const int npad = (NN + 7) & ~7;   // w at 0, v at npad, x at 2 npad of the solve's vectors
-    struct Op { int col; int kind; };  // kind 0: pivot entry, 1: constant 1, 2: 1 under charge enforcement
+    struct Op { int col; int kind; };   // kind 0: pivot entry, 1: constant 1, 2: 1 under charge enforcement
     std::vector<std::vector<Op>> rows[4];
     for (int r = 0; r < ns; r++) {
         std::vector<Op> t, x, u;
@@ -294,26 +315,29 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
         for (int c : Urow[r])
             if (c > r && c < ns) slotU[{r, c}] = n++;
     }
-    S.n_work = n;
     const int first_row[4] = {0, 0, ns, 0};
-    int *at[4] = {&S.at_T, &S.at_X, &S.at_L, &S.at_U};
+    std::vector<int> stream_slot;     // -1: padding
     for (int ph = 0; ph < 4; ph++) {
         std::vector<int> len;
         for (auto &r : rows[ph]) len.push_back((int)r.size());
         const SliceSet P = pack_slices(len, nwave);
-        *at[ph] = n;
-        int row = 0;
+        if (ph == 2) S.at_L = n;
+        S.at[ph] = (int)stream_slot.size();
         S.solve[ph].add(
             P, nwave, 1, 1, 1,
             [&](int it, uint32_t *h) { h[0] = it >= 0 ? (HDR_VALID | (uint32_t)(first_row[ph] + it)) : 0u; },
             [&](int it, int e, int, uint32_t *w) { w[0] = e >= 0 ? (uint32_t)rows[ph][it][e].col : 0u; }, len);
         for (int s = 0; s < P.n(); s++)
-            for (int pos = 0; pos < P.len[s]; pos++, row++)
+            for (int pos = 0; pos < P.len[s]; pos++)
                 for (int l = 0; l < 64; l++) {
                     const int it = P.item[64 * s + l], e = pos * P.lanes[s] + l % P.lanes[s];
-                    if (it < 0 || e >= len[it]) continue;
+                    if (it < 0 || e >= len[it]) {
+                        stream_slot.push_back(-1);
+                        continue;
+                    }
                     const Op &o = rows[ph][it][e];
-                    const int sl = n + row * 64 + l, r = first_row[ph] + it;
+                    const int sl = n++, r = first_row[ph] + it;
+                    stream_slot.push_back(sl);
                     if (o.kind == 1) one_slots.push_back(sl);
                     else if (o.kind == 2) charge_slots.push_back(sl);
                     else if (ph == 0) slotT[{r, o.col}] = sl;
@@ -321,7 +345,6 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
                     else if (ph == 2) slotL[{r, o.col - npad}] = sl;
                     else slotU[{r, o.col - 2 * npad}] = sl;
                 }
-        n += row * 64;
     }
     S.zero = n++;
     S.n_slots = n;
@@ -385,12 +408,14 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
             },
             len);
     }
-    // stream slots that take their pivot's reciprocal before they are stored
-    S.scale.assign(S.zero - S.at_T, -1);
+    // X off the diagonal and L21 take their column's pivot when they are stored
+    std::vector<unsigned> scale(S.n_slots, NO_SLOT);
     for (auto &kv : slotX)
-        if (kv.first.first != kv.first.second) S.scale[kv.second - S.at_T] = X(kv.first.second, kv.first.second);
+        if (kv.first.first != kv.first.second) scale[kv.second] = (unsigned)X(kv.first.second, kv.first.second);
     for (auto &kv : slotL)
-        if (kv.first.first >= ns) S.scale[kv.second - S.at_T] = X(kv.first.second, kv.first.second);
+        if (kv.first.first >= ns) scale[kv.second] = (unsigned)X(kv.first.second, kv.first.second);
+    for (int sl : stream_slot)
+        S.stream.push_back(sl < 0 ? ((unsigned)ZERO | NO_SLOT << 16) : ((unsigned)sl | scale[sl] << 16));
     // Schur complement of the tail
     {
         std::vector<std::vector<std::array<int, 2>>> it;
@@ -567,6 +592,7 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
             for (int sl : charge_slots) item(ENTRY_VALID | ENTRY_CHARGE | ENTRY_CHARGE_ONE | (uint32_t)sl, none);
         }
         const SliceSet P = pack_slices(len, nwave);
+        S.tail_hdr = (int)S.entries.hdr.size();   // after the last part: the tail's first header
         S.entries.add(
             P, nwave, 1, 2, 4, [&](int i, uint32_t *h) { h[0] = i >= 0 ? head[i] : 0u; },
             [&](int i, int e, int k, uint32_t *w) { put16(w, k, e >= 0 ? op[i][e] : (unsigned)ps.zero); }, len);

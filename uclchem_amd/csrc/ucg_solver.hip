@@ -31,9 +31,6 @@ enum { S_SM, S_SBK, S_BLR, S_TS, S_SPRE, S_SCAT, S_H2COL, S_COCOL, S_CCOL, S_PHI
 #ifndef UCG_WAVES_PER_EU
 #define UCG_WAVES_PER_EU 1
 #endif
-#ifndef UCG_LDS_SCHUR
-#define UCG_LDS_SCHUR 1     // FP64: the tail's Schur update from sources gathered into LDS
-#endif
 
 struct Lds {
     double *rate;                                   // workspace (global memory)
@@ -464,17 +461,32 @@ __device__ __forceinline__ double group_sum(double v, int G)
     if (G >= 64) v += __shfl_xor(v, 32);
     return v;
 }
-struct Slice { int row, rows, G, hdr; };
-__device__ __forceinline__ Slice slice_at(const GLB int *slices, int s)
-{
-    return {slices[4 * s], slices[4 * s + 1], slices[4 * s + 2], slices[4 * s + 3]};
-}
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(tid() >> 6); }
+
+// A wave's slices of one program phase (ucg_plan.h): load(row) fetches a row's record, use(record)
+// adds it up, done(header, lanes per item, header index) ends a slice.  A plain loop on purpose:
+// keeping rows in flight across slice boundaries (a register ring, unrolled with the slice's end in
+// every position) made the phases slower, the set-up 60 -> 66 us: the code of a step is several
+// times the instruction cache, and its size costs more than the loads' latency.
+template <int U, class Load, class Use, class Done>
+__device__ __forceinline__ void run_slices(const CST DevProg &G, int phase, Load load, Use use, Done done)
+{
+    const GLB int *wp = glb(G.wave_ptr) + phase * (NWAVE + 1) + wave_id(), *slices = glb(G.slices);
+    const GLB uint32_t *hdr = glb(G.hdr) + (tid() & 63);
+    const int s1 = wp[1];
+    for (int s = wp[0]; s < s1; s++) {
+        const int row = slices[4 * s], rows = slices[4 * s + 1], G_ = slices[4 * s + 2], h0 = slices[4 * s + 3];
+        const uint32_t h = hdr[h0];
+#pragma unroll U
+        for (int r = 0; r < rows; r++) use(load(row + r));
+        done(h, G_, h0);
+    }
+}
 
 // a factor product over the extended state, four factors a record
 __device__ __forceinline__ double term4(uint2 w, double r, const LDS double *y)
 {
-    return r * y[w.x & 0xffff] * (y[w.x >> 16] * (y[w.y & 0xffff] * y[w.y >> 16]));
+    return r * y[w.x & 0xffff] * y[w.x >> 16] * y[w.y & 0xffff] * y[w.y >> 16];
 }
 __device__ __forceinline__ uint2 ld_uint2(const GLB uint32_t *p, int i)
 {
@@ -482,6 +494,12 @@ __device__ __forceinline__ uint2 ld_uint2(const GLB uint32_t *p, int i)
     r.x = p[2 * i];
     r.y = p[2 * i + 1];
     return r;
+}
+// v[index], negated when the sign bit is set
+__device__ __forceinline__ double signed_entry(const LDS double *v, unsigned e)
+{
+    const double x = v[e & 0x7fff];
+    return __hiloint2double(__double2hiint(x) ^ (int)((e & 0x8000u) << 16), __double2loint(x));
 }
 __device__ __forceinline__ double term_of(NetRef N, int k, double r, const LDS double *y)
 {
@@ -503,7 +521,7 @@ __device__ __forceinline__ double term_of(NetRef N, int k, double r, const LDS d
 // Bound by the LDS gathers and the latency of the three parts: 7.7 us a call (default
 // network), against 17.5 for chunked sums with a second pass over the chunks, workgroup-wide
 // reductions for each total and serial photo-rate splines.
-UCG_BIG __device__ void block_rhs(NetRef N_, const Lds L)
+__device__ __forceinline__ void block_rhs(NetRef N_, const Lds L)
 {
     NetRef N = fresh(N_);
     PhaseClock clk(L);
@@ -576,31 +594,25 @@ UCG_BIG __device__ void block_rhs(NetRef N_, const Lds L)
             }
         }
     }
+    const GLB uint32_t *srec = glb(N.pg_sum.rec) + 2 * lane;
+    const auto load = [&](int r) { return ld_uint2(srec, 64 * r); };
     __syncthreads();
     clk.mark(TM_RHS_FLUX);
     {
-        const GLB uint32_t *rec = glb(N.pg_sum.rec), *hdr = glb(N.pg_sum.hdr);
-        const GLB int *slices = glb(N.pg_sum.slices);
-        const int s1 = glb(N.pg_sum.wave_ptr)[w + 1];
-        for (int s = glb(N.pg_sum.wave_ptr)[w]; s < s1; s++) {
-            const Slice sl = slice_at(slices, s);
-            const uint32_t h = hdr[sl.hdr + lane];
-            double a0 = 0.0, a1 = 0.0;
-#pragma unroll 2
-            for (int r = 0; r < sl.rows; r++) {
-                const uint2 q = ld_uint2(rec, (sl.row + r) * 64 + lane);
-                const auto val = [&](unsigned e) {
-                    const double v = flux[e & 0x7fff];
-                    return __hiloint2double(__double2hiint(v) ^ (int)((e & 0x8000u) << 16), __double2loint(v));
-                };
-                a0 += val(q.x);
-                a1 += val(q.x >> 16);
-                a0 += val(q.y);
-                a1 += val(q.y >> 16);
-            }
-            const double acc = group_sum(a0 + a1, sl.G);
-            if (h & HDR_VALID) f[h & HDR_INDEX] = acc;
-        }
+        double a0 = 0.0, a1 = 0.0;
+        run_slices<2>(
+            N.pg_sum, 0, load,
+            [&](uint2 q) {
+                a0 += signed_entry(flux, q.x);
+                a1 += signed_entry(flux, q.x >> 16);
+                a0 += signed_entry(flux, q.y);
+                a1 += signed_entry(flux, q.y >> 16);
+            },
+            [&](uint32_t h, int G, int) {
+                const double acc = group_sum(a0 + a1, G);
+                if (h & HDR_VALID) f[h & HDR_INDEX] = acc;
+                a0 = a1 = 0.0;
+            });
     }
     __syncthreads();
     clk.mark(TM_RHS_SUMS);
@@ -1250,11 +1262,14 @@ template <int K> __device__ __forceinline__ void gj16_steps(f64x4 &d, int g, int
     }
 }
 
-// A: n x n, column-major, leading dimension n, in LDS; overwritten by its inverse.  `stage`: LDS
-// scratch of gj_stage_len(n) doubles outside A.  Returns nonzero (uniformly) on a zero or
-// non-finite pivot.
+// A: n x n, column-major, leading dimension n, in LDS.  The inverse goes to `out` in blocks of four
+// columns, row-major inside a block (tail_index), the order in which the solve's lanes read it.
+// `stage`: LDS scratch of gj_stage_len(n) doubles outside A.  Returns nonzero (uniformly) on a zero
+// or non-finite pivot.
+__device__ __forceinline__ int tail_index(int n, int row, int col) { return (col >> 2) * 4 * n + 4 * row + (col & 3); }
+__host__ __device__ inline int tail_len(int n) { return ((n + 3) & ~3) * n; }
 template <typename LUT>
-__device__ __forceinline__ int block_gj_inverse(LDS LUT *A, int n, LDS double *red, LDS double *stage)
+__device__ __forceinline__ int block_gj_inverse(const LDS double *A, int n, LDS double *red, LDS double *stage, LUT *out)
 {
     const int w = __builtin_amdgcn_readfirstlane(tid() >> 6), lane = tid() & 63, g = lane >> 4, c = lane & 15;
     const int nb = (n + 15) >> 4, gen = (nb + 1) * GJ_TILE;
@@ -1266,7 +1281,7 @@ __device__ __forceinline__ int block_gj_inverse(LDS LUT *A, int n, LDS double *r
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int row = 16 * I + 4 * i + g;
-            t[I][i] = (row < n && col < n) ? (double)A[col * n + row] : (row == col ? 1.0 : 0.0);
+            t[I][i] = (row < n && col < n) ? A[col * n + row] : (row == col ? 1.0 : 0.0);
         }
     __syncthreads();
     f64x4 mine = {0.0, 0.0, 0.0, 0.0};   // the owner's inverted pivot block
@@ -1330,64 +1345,16 @@ __device__ __forceinline__ int block_gj_inverse(LDS LUT *A, int n, LDS double *r
                 }
         }
     }
-    // every wave has read A and the last panel
-    __syncthreads();
+    GLB LUT *og = glbw(out);
 #pragma unroll
     for (int I = 0; I < NWAVE; I++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int row = 16 * I + 4 * i + g;
-            if (row < n && col < n) A[col * n + row] = (LUT)t[I][i];
+            if (row < n && col < ((n + 3) & ~3)) og[tail_index(n, row, col)] = (LUT)(col < n ? t[I][i] : 0.0);
         }
     __syncthreads();
     return 0;
-}
-
-// x <- Ainv x for the n x n inverse Ainv (column-major, leading dimension n) and the LDS
-// vector x: two threads per row (column halves) when 2n fits the workgroup, the second
-// half's partial passed through `scratch` (n doubles of LDS); x is overwritten only after
-// every thread has read it.
-template <typename TP>
-__device__ __forceinline__ void tail_matvec(TP Ainv, int n, LDS double *x, LDS double *scratch)
-{
-    const int t = tid();
-    if (2 * n <= NT) {
-        const int half = (n + 1) >> 1;
-        double acc = 0.0;
-        int r = -1;
-        if (t < 2 * n) {
-            r = t % n;
-            const int h = t / n;
-            const int c1 = h ? n : half;
-            int c = h ? half : 0;
-            double a1 = 0.0, a2 = 0.0, a3 = 0.0;
-            for (; c + 4 <= c1; c += 4) {
-                acc += (double)Ainv[(size_t)c * n + r] * x[c];
-                a1 += (double)Ainv[(size_t)(c + 1) * n + r] * x[c + 1];
-                a2 += (double)Ainv[(size_t)(c + 2) * n + r] * x[c + 2];
-                a3 += (double)Ainv[(size_t)(c + 3) * n + r] * x[c + 3];
-            }
-            for (; c < c1; c++) acc += (double)Ainv[(size_t)c * n + r] * x[c];
-            acc = (acc + a1) + (a2 + a3);
-            if (h) scratch[r] = acc;
-        }
-        __syncthreads();
-        if (t < n) x[r] = acc + scratch[r];
-    } else {
-        for (int r = t; r < n; r += NT) {
-            double a0 = 0.0, a1 = 0.0;
-            int c = 0;
-            for (; c + 2 <= n; c += 2) {
-                a0 += (double)Ainv[(size_t)c * n + r] * x[c];
-                a1 += (double)Ainv[(size_t)(c + 1) * n + r] * x[c + 1];
-            }
-            if (c < n) a0 += (double)Ainv[(size_t)c * n + r] * x[c];
-            scratch[r] = a0 + a1;
-        }
-        __syncthreads();
-        for (int r = t; r < n; r += NT) x[r] = scratch[r];
-    }
-    __syncthreads();
 }
 
 #ifndef UCG_SB
@@ -1695,73 +1662,20 @@ __device__ __forceinline__ void crout_phases(NetRef N, WP W, LDS double *red, in
     __syncthreads();
 }
 
+// Plans whose tail does not fit the workgroup run from the workspace: all elimination phases, then a
+// blocked LU of the tail.
 template <typename LUT>
-UCG_BIG __device__ int sparse_lu(NetRef N_, const Lds &L, LUT *V, LDS double *region, LDS double *red, LDS double *stage)
+UCG_BIG __device__ int workspace_lu(NetRef N_, const Lds &L, LUT *V)
 {
     NetRef N = fresh(N_);
-    const int nval = N.nw_nval, nsp = N.nw_nsp, T = N.nw_T;
-    if (tid() == 0) red[9] = 0.0;
-    int r = 0;
     PhaseClock clk(L);
-    if (!N.nw_stage) {                    // factors too large to stage: everything in the workspace
-        __syncthreads();
-        crout_phases<LUT>(N, glbw(V), red, N.nw_nph);
-        clk.mark(TM_LU_SPARSE);
-        if (red[9] != 0.0) return 1;
-        if (T > 0) r = block_lu_tiled<LUT>(V + nsp, T, T, red, stage);
-    } else {
-        __syncthreads();
-        const bool lp = UCG_LDS_SCHUR && N.nlp_src > 0;   // the last phase (Schur update of the tail) in LDS
-        if (lp) {
-            // the phases before it touch only the sparse part's nsp values (a staged region
-            // holds them): eliminate on an LDS copy, so that every dependent access of the
-            // phase chain is an LDS access, then store the factors back for the solve
-            LDS LUT *Ws = (LDS LUT *)region;
-            const GLB LUT *Vg = glb(V);
-            for (int q = tid(); q < nsp; q += NT) Ws[q] = Vg[q];
-            __syncthreads();
-            crout_phases<LUT>(N, Ws, red, N.nw_nph - 1);
-            if (red[9] != 0.0) return 1;
-            for (int q = tid(); q < nsp; q += NT) V[q] = Ws[q];
-            __syncthreads();
-        } else {
-            crout_phases<LUT>(N, glbw(V), red, N.nw_nph);
-            if (red[9] != 0.0) return 1;
-        }
-        LDS LUT *tl = (LDS LUT *)region;   // the tail, worked on in the factor precision
-        for (int q = tid(); q < T * T; q += NT) tl[q] = V[nsp + q];
-        if (lp) {
-            LDS LUT *src = tl + T * T;
-            const GLB LUT *Vg = glb(V);
-            const GLB int *lsrc = glb(N.lp_src), *tgs = glb(N.nw_tg_slot), *tgp = glb(N.nw_tg_ptr);
-            for (int k = tid(); k < N.nlp_src; k += NT) src[k] = Vg[lsrc[k]];
-            __syncthreads();
-            const int p = N.nw_nph - 1, t0 = N.nw_ph_ptr[p], t1 = N.nw_ph_ptr[p + 1], qb = N.nw_tg_ptr[t0];
-            const GLB int *pr = glb(N.lp_pr);
-            for (int t = t0 + tid(); t < t1; t += NT) {
-                const int e = tgs[t] - nsp;
-                LUT a0 = tl[e], a1 = 0, a2 = 0, a3 = 0;
-                const int q1 = tgp[t + 1] - qb;
-                int q = tgp[t] - qb;
-                for (; q + 4 <= q1; q += 4) {
-                    const int2 p0 = ld_int2(pr, q), p1 = ld_int2(pr, q + 1), p2 = ld_int2(pr, q + 2), p3 = ld_int2(pr, q + 3);
-                    a0 -= src[p0.x] * src[p0.y];
-                    a1 -= src[p1.x] * src[p1.y];
-                    a2 -= src[p2.x] * src[p2.y];
-                    a3 -= src[p3.x] * src[p3.y];
-                }
-                for (; q < q1; q++) {
-                    const int2 p0 = ld_int2(pr, q);
-                    a0 -= src[p0.x] * src[p0.y];
-                }
-                tl[e] = (a0 + a1) + (a2 + a3);
-            }
-        }
-        clk.mark(TM_LU_SPARSE);
-        __syncthreads();
-        if (T > 0) r = block_gj_inverse<LUT>(tl, T, red, region + T * T);
-        for (int q = tid(); q < T * T; q += NT) V[nsp + q] = tl[q];
-    }
+    if (tid() == 0) L.red[9] = 0.0;
+    __syncthreads();
+    crout_phases<LUT>(N, glbw(V), L.red, N.nw_nph);
+    clk.mark(TM_LU_SPARSE);
+    if (L.red[9] != 0.0) return 1;
+    int r = 0;
+    if (N.nw_T > 0) r = block_lu_tiled<LUT>(V + N.nw_nsp, N.nw_T, N.nw_T, L.red, L.flux);
     __syncthreads();
     clk.mark(TM_LU_TAIL);
     return r;
@@ -1844,10 +1758,7 @@ __device__ __forceinline__ void solve_program(NetRef N, VP V, IP cols, IP recs, 
     }
     __syncthreads();
     clk.mark(TM_SOL_SPARSE);
-    if (T > 0) {
-        if (N.nw_stage) tail_matvec(tail, T, w + ns, w + NN);   // staged plans hold the block's inverse
-        else block_lu_solve<LUT>(tail, T, T, w + ns);          // unstaged plans hold its LU factors
-    }
+    if (T > 0) block_lu_solve<LUT>(tail, T, T, w + ns);
     clk.mark(TM_SOL_TAIL);
     for (int l = N.nw_nlev - 1; l >= 0; l--) {   // backward, sparse rows by level
         const int q0 = lev[l];
@@ -1873,18 +1784,13 @@ __device__ __forceinline__ void solve_program(NetRef N, VP V, IP cols, IP recs, 
     clk.mark(TM_SOL_SPARSE);
 }
 
-// Solve M x = b with the factors of sparse_lu: b (length neq, in LDS) is overwritten by x.
-// A staged plan copies the solve program (row records in level order, column indices,
-// permutation) and the sparse factors into LDS (region) so that every dependent access of
-// the level-scheduled substitutions is an LDS access; FP32 factors bring their dense tail
-// too, FP64 tails are read from the workspace by the dense triangular solves.  An unstaged
-// plan reads all of it from the workspace and keeps only the work vector in region.
+// Solve M x = b with the factors of workspace_lu: b (length neq, in LDS) is overwritten by x; the
+// work vector lives in region.
 template <typename LUT>
-UCG_BIG __device__ void sparse_lu_solve(NetRef N_, const Lds L, const LUT *Vg, LDS double *b, LDS double *region)
+UCG_BIG __device__ void workspace_solve(NetRef N_, const Lds L, const LUT *Vg, LDS double *b, LDS double *region)
 {
     NetRef N = fresh(N_);
     PhaseClock clk(L);
-    const int NN = N.nw_N, nsp = N.nw_nsp;
     if (L.prm[P_ENFORCECHARGE] != 0.0 && N.nelec < N.nspec) {   // right-hand side of the charge row
         double se = 0.0;
         for (int q = tid(); q < N.nion; q += NT) se += b[N.ion_list[q]];
@@ -1895,52 +1801,324 @@ UCG_BIG __device__ void sparse_lu_solve(NetRef N_, const Lds L, const LUT *Vg, L
     double sb = 0.0, ss = 0.0;
     for (int q = tid(); q < N.nbulkl; q += NT) sb += b[N.bulk_list[q]];
     for (int q = tid(); q < N.nsurfl; q += NT) ss += b[N.surface_list[q]];
-    if (!N.nw_stage) {
-        block_sum2(sb, ss, L.red, RED_TOTALS);
-        solve_program<LUT>(N, Vg, N.nw_sp_col, N.sv_rec, N.nw_inv, N.nw_lev_ptr, Vg + nsp, region, b, sb, ss, clk);
+    block_sum2(sb, ss, L.red, RED_TOTALS);
+    solve_program<LUT>(N, Vg, N.nw_sp_col, N.sv_rec, N.nw_inv, N.nw_lev_ptr, Vg + N.nw_nsp, region, b, sb, ss, clk);
+}
+
+// ---------------------------------------------------------------- staged Newton system
+// The whole set-up of a staged plan (ucg_plan.h) in LDS and registers.  Nothing but the finished
+// factors goes to the workspace, in the order the solves stream them: T = -inv(L11), X = inv(U11),
+// L21 and U12 of the sparse pivots (inverting these small, very sparse triangles costs a few
+// hundred products and turns a solve's two level-by-level sweeps into two products), then the
+// inverse of the tail.  Default network, FP64, per call on an otherwise idle chip, against the form
+// with the Jacobian, the matrix and the level-by-level elimination passed through the workspace:
+// Jacobian and matrix 68 -> 18 us, sparse part 51 -> 27 us, solve 33 -> 7 us.  What bounds it now:
+// LDS gathers and the latency of a dozen short phases, and the instruction cache, which a step's
+// code exceeds several times.
+
+// Operands of the entries: partials of every term by each of its factors, and the structured
+// couplings' slots (PartialSlots).  Right after block_rhs at the same state, whose totalSwap it uses.
+__device__ __forceinline__ void partial_operands(NetRef N, const Lds &L, LDS double *P)
+{
+    const int neq = N.neq, w = wave_id(), lane = tid() & 63;
+    LDS double *y = L.y, *sc = L.sc;
+    const GLB double *rate = glb((const double *)L.rate);
+    const double D = y[neq - 1];
+    const double ysur = y[N.nsurface], ybulk = y[N.nbulk];
+    const double sm = fmax(1e-30, ysur), sbk = fmax(1e-30, ybulk);
+    const double blr = y[neq + YX_BLR], ism = y[neq + YX_ISM], tsm = y[neq + YX_TSM];
+    const double dblr = (blr < 1.0 && ybulk > 1e-30) ? -blr / sbk : 0.0;
+    const double dism = (ysur > 1e-30) ? -ism * ism : 0.0;
+    const double dtsm = (ysur > 1e-30) ? -tsm * ism : 0.0;
+    if (w == NWAVE - 1) {
+        // photo rates by the columns, one-sided differences: rows of 16 lanes take (h, c),
+        // (h (1 + eps), c) and (h, c (1 + eps)) together
+        const double cs = sc[S_CS], eps = 1e-6;
+        const double h2col = 0.5 * y[N.nh2] * D * cs, cocol = 0.5 * y[N.nco] * D * cs;
+        const int row = lane >> 4;
+        double kh, kc;
+        photo_rates_wave(row == 1 ? h2col * (1 + eps) : h2col, row == 2 ? cocol * (1 + eps) : cocol, L.prm[P_RADFIELD],
+                         sc[S_SCAT], sc[S_AV], kh, kc);
+        const double kh0 = wave_lane(kh, 0), kc0 = wave_lane(kc, 0);
+        const double dkh = h2col > 0 ? (wave_lane(kh, 16) - kh0) / (h2col * eps) : 0.0;
+        const double dkch = h2col > 0 ? (wave_lane(kc, 16) - kc0) / (h2col * eps) : 0.0;
+        const double dkcc = cocol > 0 ? (wave_lane(kc, 32) - kc0) / (cocol * eps) : 0.0;
+        if (lane == 0) {
+            const double ph = term_of(N, N.r_h2_hv, 1.0, y), pc = term_of(N, N.r_co_hv, 1.0, y);
+            LDS double *p = P + N.px.photo;
+            p[0] = ph * (dkh * 0.5 * D * cs);
+            p[1] = ph * (dkh * 0.5 * y[N.nh2] * cs);
+            p[2] = pc * (dkch * 0.5 * D * cs);
+            p[3] = pc * (dkcc * 0.5 * D * cs);
+            p[4] = pc * (dkch * 0.5 * y[N.nh2] * cs + dkcc * 0.5 * y[N.nco] * cs);
+            P[N.px.zero] = 0.0;
+            P[N.px.swap_nb] = (blr < 1.0 && ybulk > 1e-30) ? -(tsm * sm) / sbk : 0.0;
+        }
+        if (lane == 63) {
+            const double dn = D * 1e-7;
+            P[N.px.densdot] = (densdot_dev(L.prm, D + dn) - densdot_dev(L.prm, D)) / dn;
+        }
         return;
     }
-    constexpr bool STAGE_TAIL = sizeof(LUT) == 4;
-    const int nst = STAGE_TAIL ? N.nw_nval : nsp;                       // staged factor entries
-    // layout in bytes, 16-byte aligned parts (solve_stage_bytes sizes the same)
-    LDS char *base = (LDS char *)region;
-    int off = 0;
-    LDS LUT *Vs = (LDS LUT *)base;
-    off = (nst * (int)sizeof(LUT) + 15) & ~15;
-    LDS int *cols = (LDS int *)(base + off);
-    off += (nsp * 4 + 15) & ~15;
-    LDS int *recs = (LDS int *)(base + off);   // 4 ints per row: {row, first, diagonal, end}
-    off += NN * 16;
-    LDS int *inv = (LDS int *)(base + off);
-    off += ((NN + N.nw_nlev + 1) * 4 + 15) & ~15;   // permutation, then the level pointers
-    LDS double *w = (LDS double *)(base + off);
-    {
-        const GLB LUT *vg = glb(Vg);
-        const GLB int *cg = glb(N.nw_sp_col);
-        for (int q = tid(); q < nst; q += NT) Vs[q] = vg[q];
-        for (int q = tid(); q < nsp; q += NT) cols[q] = cg[q];
+    if (w == NWAVE - 2) {
+        for (int q = lane; q < N.nswt; q += 64) {   // the SURFSWAP term without its totalSwap
+            const int k = glb(N.sx_list)[q];
+            const GLB uint32_t *rx = glb(N.rx) + 2 * k * N.rx_w;
+            double v = rate[k] * ism;
+            for (int m = 0; m < 4 * N.rx_w - 1; m++) v *= y[(rx[m / 2] >> (16 * (m & 1))) & 0xffff];
+            P[N.px.swap_u + q] = v;
+        }
+        for (int q = lane; q < N.nswap; q += 64) P[N.px.swap_g + q] = rate[glb(N.swap_list)[q]] * blr;
     }
-    {
-        const GLB int *gr = glb(N.sv_rec);
-        for (int q = tid(); q < NN; q += NT) {
-            const int4 g = ld_int4(gr, q);
-            recs[4 * q] = g.x;
-            recs[4 * q + 1] = g.y;
-            recs[4 * q + 2] = g.z;
-            recs[4 * q + 3] = g.w;
+    if (w == NWAVE - 3) {   // transfer factors and their derivatives
+        const double S = sc[S_SPRE];
+        const bool neg = S < 0, ratio_lt1 = (sbk / sm) < 1.0;
+        for (int q = lane; q < N.nsurfl; q += 64) {
+            const int s_ = glb(N.surface_list)[q], b = glb(N.bulk_partner_of_surface)[s_];
+            P[N.px.transfer_t + q] = neg ? (ratio_lt1 ? y[b] / sm : y[b] / sbk) : SURFACE_COVERAGE0 * y[s_];
+            LDS double *d = P + N.px.transfer_d + 4 * q;
+            d[0] = neg ? 0.0 : S * SURFACE_COVERAGE0;
+            d[1] = neg ? S * (ratio_lt1 ? 1.0 / sm : 1.0 / sbk) : 0.0;
+            d[2] = (neg && ratio_lt1 && ysur > 1e-30) ? S * (-y[b] / (sm * sm)) : 0.0;
+            d[3] = (neg && !ratio_lt1 && ybulk > 1e-30) ? S * (-y[b] / (sbk * sbk)) : 0.0;
         }
     }
-    for (int q = tid(); q < NN; q += NT) inv[q] = glb(N.nw_inv)[q];
-    LDS int *lev = inv + NN;   // level pointers (nlev + 1), after the permutation
-    for (int q = tid(); q <= N.nw_nlev; q += NT) lev[q] = glb(N.nw_lev_ptr)[q];
-    block_sum2(sb, ss, L.red, RED_TOTALS);   // its barriers also publish the staged program
-    const LDS LUT *V = Vs;
-    if constexpr (STAGE_TAIL)
-        solve_program<LUT>(N, V, (const LDS int *)cols, (const LDS int *)recs, (const LDS int *)inv,
-                           (const LDS int *)lev, V + nsp, w, b, sb, ss, clk);
-    else
-        solve_program<LUT>(N, V, (const LDS int *)cols, (const LDS int *)recs, (const LDS int *)inv,
-                           (const LDS int *)lev, Vg + nsp, w, b, sb, ss, clk);
+    const GLB uint32_t *rp = glb(N.rp);
+    const GLB int *foff = glb(N.fac_off);
+    const int nr = N.nreac, r1 = glb(N.fx_row)[w + 1];
+    const auto deriv = [&](unsigned c) {   // of a factor by its own variable
+        const int x = (int)c - neq;
+        return x == YX_BLR ? dblr : x == YX_ISM ? dism : x == YX_TSM ? dtsm : 1.0;
+    };
+    if (N.rx_w == 1) {
+#pragma unroll 2
+        for (int r0 = glb(N.fx_row)[w]; r0 < r1; r0++) {
+            const int k = r0 * 64 + lane;
+            if (k >= nr) break;
+            const uint2 q = ld_uint2(rp, k);
+            const double r = rate[k];
+            const int o = foff[k], nf = foff[k + 1] - o;
+            const unsigned c[4] = {q.x & 0xffff, q.x >> 16, q.y & 0xffff, q.y >> 16};
+            const double v0 = y[c[0]], v1 = y[c[1]], v2 = y[c[2]], v3 = y[c[3]];
+            const double a = r * v0, b = v2 * v3;
+            if (nf > 0) P[o] = r * deriv(c[0]) * (v1 * b);
+            if (nf > 1) P[o + 1] = a * deriv(c[1]) * b;
+            if (nf > 2) P[o + 2] = a * v1 * (deriv(c[2]) * v3);
+            if (nf > 3) P[o + 3] = a * v1 * (v2 * deriv(c[3]));
+        }
+    } else {
+        for (int r0 = glb(N.fx_row)[w]; r0 < r1; r0++) {
+            const int k = r0 * 64 + lane;
+            if (k >= nr) break;
+            const int o = foff[k], nf = foff[k + 1] - o;
+            const GLB uint32_t *q = rp + 2 * k * N.rx_w;
+            for (int m = 0; m < nf; m++) {
+                double v = rate[k];
+                for (int u = 0; u < nf; u++) {
+                    const unsigned c = (q[u / 2] >> (16 * (u & 1))) & 0xffff;
+                    v *= u == m ? deriv(c) : y[c];
+                }
+                P[o + m] = v;
+            }
+        }
+    }
+}
+
+// Entries of M = I - gamma J: working slots to LDS (W), tail entries to the workspace, where the
+// same lane fetches them once the operands' LDS is free.
+__device__ __forceinline__ void newton_entries(NetRef N, const LDS double *P, LDS double *W, double *stage, double gamma,
+                                               bool charge)
+{
+    const int lane = tid() & 63;
+    const GLB uint32_t *rec = glb(N.pg_entries.rec) + 2 * lane;
+    GLB double *st = glbw(stage) - N.sp_tail_hdr + lane;
+    const auto load = [&](int r) { return ld_uint2(rec, 64 * r); };
+    for (int part = 0; part < 2; part++) {
+        double a0 = 0.0, a1 = 0.0;
+        run_slices<2>(
+            N.pg_entries, part, load,
+            [&](uint2 q) {
+                a0 += signed_entry(P, q.x);
+                a1 += signed_entry(P, q.x >> 16);
+                a0 += signed_entry(P, q.y);
+                a1 += signed_entry(P, q.y >> 16);
+            },
+            [&](uint32_t h, int G, int hdr) {
+                const double acc = group_sum(a0 + a1, G);
+                a0 = a1 = 0.0;
+                double v = (h & ENTRY_UNSCALED) ? acc : -gamma * acc;
+                v += (h & ENTRY_ONE) ? 1.0 : (h & ENTRY_MINUS) ? -1.0 : 0.0;
+                if (charge && (h & ENTRY_CHARGE)) v = (h & ENTRY_CHARGE_ONE) ? 1.0 : (h & ENTRY_CHARGE_MINUS) ? -1.0 : 0.0;
+                if (h & ENTRY_VALID) {
+                    if (part == 0) W[h & ENTRY_TARGET] = v;
+                    else st[hdr] = v;
+                }
+            });
+    }
+}
+
+// Elimination of the sparse pivots, one phase a level; zero or non-finite pivots raise red[9].
+__device__ __forceinline__ void eliminate(NetRef N, LDS double *W, LDS double *red)
+{
+    const GLB uint32_t *rec = glb(N.pg_elim.rec) + 2 * (tid() & 63);
+    const auto load = [&](int r) { return ld_uint2(rec, 64 * r); };
+    for (int p = 0; p < N.pg_elim.phases; p++) {
+        double acc = 0.0;
+        run_slices<2>(
+            N.pg_elim, p, load, [&](uint2 q) { acc += W[q.x & 0xffff] * (W[q.x >> 16] * W[q.y & 0xffff]); },
+            [&](uint32_t h, int G, int) {
+                const double s = group_sum(acc, G);
+                acc = 0.0;
+                if (h & HDR_VALID) {
+                    double v = W[h & HDR_INDEX] - s;
+                    if (h & HDR_RECIP) {
+                        if (!(v == v) || v == 0.0 || isinf(v)) red[9] = 1.0;
+                        v = fast_rcp(v);
+                    }
+                    W[h & HDR_INDEX] = v;
+                }
+            });
+        __syncthreads();
+    }
+}
+
+template <typename LUT>
+__device__ __forceinline__ int staged_setup(NetRef N_, const Lds &L, LUT *V, double *stage, double gamma)
+{
+    NetRef N = fresh(N_);
+    PhaseClock clk(L);
+    const int w = wave_id(), lane = tid() & 63, T = N.sp_T;
+    const bool charge = L.prm[P_ENFORCECHARGE] != 0.0 && N.nelec < N.nspec;
+    LDS double *P = L.flux, *W = L.flux + N.sp_w0, *tl = L.flux, *red = L.red;
+    if (tid() == 0) red[9] = 0.0;
+    for (int q = tid(); q < N.sp_slots; q += NT) W[q] = 0.0;
+    partial_operands(N, L, P);
+    __syncthreads();
+    newton_entries(N, P, W, stage, gamma, charge);
+    __syncthreads();
+    clk.mark(TM_JAC);
+    PhaseClock lu(L);
+    eliminate(N, W, red);
+    if (red[9] != 0.0) return 1;
+    {   // store the streams, scaled by their columns' pivots; the Schur update needs L21 scaled
+        const GLB uint32_t *from = glb(N.sp_stream);
+        GLB LUT *out = glbw(V);
+#pragma unroll 4
+        for (int q = tid(); q < N.sp_nstream; q += NT) {
+            const uint32_t f = from[q], sl = f & 0xffff, k = f >> 16;
+            double v = W[sl];
+            if (k != NO_SLOT) {
+                v *= W[k];
+                if ((int)sl >= N.sp_L) W[sl] = v;
+            }
+            out[q] = (LUT)v;
+        }
+    }
+    __syncthreads();
+    for (int q = tid(); q < T * T; q += NT) tl[q] = 0.0;
+    __syncthreads();
+    {   // this lane's tail entries
+        const GLB uint32_t *hdr = glb(N.pg_entries.hdr);
+        const GLB int *slices = glb(N.pg_entries.slices), *wp = glb(N.pg_entries.wave_ptr) + NWAVE + 1;
+        const GLB double *st = glb((const double *)stage) - N.sp_tail_hdr;
+        const int s1 = wp[w + 1];
+        for (int s = wp[w]; s < s1; s++) {
+            const int h0 = slices[4 * s + 3] + lane;
+            const uint32_t h = hdr[h0];
+            if (h & ENTRY_VALID) tl[h & ENTRY_TARGET] = st[h0];
+        }
+    }
+    __syncthreads();
+    {   // Schur complement
+        const GLB uint32_t *rec = glb(N.pg_schur.rec) + 2 * lane;
+        const auto load = [&](int r) { return ld_uint2(rec, 64 * r); };
+        double a0 = 0.0, a1 = 0.0;
+        run_slices<4>(
+            N.pg_schur, 0, load,
+            [&](uint2 q) {
+                a0 += W[q.x & 0xffff] * W[q.x >> 16];
+                a1 += W[q.y & 0xffff] * W[q.y >> 16];
+            },
+            [&](uint32_t h, int G, int) {
+                const double acc = group_sum(a0 + a1, G);
+                a0 = a1 = 0.0;
+                if (h & HDR_VALID) tl[h & HDR_INDEX] -= acc;
+            });
+    }
+    __syncthreads();
+    clk.mark(TM_LU_SPARSE);
+    const int r = T > 0 ? block_gj_inverse<LUT>(tl, T, red, L.flux + T * T, V + N.sp_nstream) : 0;
+    clk.mark(TM_LU_TAIL);
+    lu.mark(TM_LU);
+    return r;
+}
+
+// One stream phase of a solve: stored values times entries of the vectors at vec, summed by row.
+template <typename LUT, class Out>
+__device__ __forceinline__ void stream_phase(const CST DevProg &G, const LUT *v, const LDS double *vec, Out out)
+{
+    const GLB LUT *vals = glb(v) + (tid() & 63);
+    const GLB uint32_t *cols = glb(G.rec) + (tid() & 63);
+    double acc = 0.0;
+    run_slices<4>(
+        G, 0, [&](int r) { return 64 * r; }, [&](int e) { acc += (double)vals[e] * vec[cols[e]]; },
+        [&](uint32_t h, int lanes, int) {
+            const double s = group_sum(acc, lanes);
+            acc = 0.0;
+            if (h & HDR_VALID) out((int)(h & HDR_INDEX), s);
+        });
+}
+
+// M x = b from the stored streams: w (permuted right-hand side, at L.flux) -> x (two vectors
+// further).  Five products with a barrier after each.
+template <typename LUT>
+__device__ __forceinline__ void staged_solve(NetRef N_, const Lds &L, const LUT *V)
+{
+    NetRef N = fresh(N_);
+    PhaseClock clk(L);
+    const int npad = (N.nw_N + 7) & ~7, ns = N.sp_ns, T = N.sp_T;
+    LDS double *w = L.flux, *v = w + npad, *x = v + npad;
+    if (N.sp_presum) {   // sums of the replaced rows' right-hand sides
+        if (wave_id() == 0) {
+            const bool charge = L.prm[P_ENFORCECHARGE] != 0.0 && N.nelec < N.nspec;
+            const GLB int *sr = glb(N.sp_sum_rows), *sm = glb(N.sp_sum_members);
+            for (int k = charge ? 2 : 1; k >= 0; k--) {
+                double s = 0.0;
+                for (int q = sr[3 * k + 1] + (tid() & 63); q < sr[3 * k + 2]; q += 64) s += w[sm[q]];
+                s = wave_sum(s);
+                if (tid() == 0) w[sr[3 * k]] -= s;
+            }
+        }
+        __syncthreads();
+    }
+    stream_phase<LUT>(N.pg_solve[0], V + N.sp_at[0], w, [&](int r, double s) { v[r] = w[r] - s; });
+    __syncthreads();
+    stream_phase<LUT>(N.pg_solve[2], V + N.sp_at[2], w, [&](int r, double s) { v[r] = w[r] - s; });
+    __syncthreads();
+    clk.mark(TM_SOL_SPARSE);
+    if (T > 0) {   // four lanes a row of the tail's inverse, each every fourth column
+        const int t = tid(), h = t & 3, nst = (T + 3) >> 2;
+        const GLB LUT *S = glb(V + N.sp_nstream) + t;
+        double p0 = 0.0, p1 = 0.0;
+        if (t < 4 * T) {
+            int q = 0;
+#pragma unroll 4
+            for (; q + 2 <= nst - 1; q += 2) {
+                p0 += (double)S[q * 4 * T] * v[ns + 4 * q + h];
+                p1 += (double)S[(q + 1) * 4 * T] * v[ns + 4 * q + 4 + h];
+            }
+            for (; q < nst; q++) p0 += (double)S[q * 4 * T] * v[ns + min(4 * q + h, T - 1)];
+        }
+        const double s = group_sum(p0 + p1, 4);
+        if (t < 4 * T && h == 0) x[ns + (t >> 2)] = s;
+    }
+    __syncthreads();
+    clk.mark(TM_SOL_TAIL);
+    stream_phase<LUT>(N.pg_solve[3], V + N.sp_at[3], w, [&](int r, double s) { w[r] = v[r] - s; });
+    __syncthreads();
+    stream_phase<LUT>(N.pg_solve[1], V + N.sp_at[1], w, [&](int r, double s) { x[r] = s; });
+    __syncthreads();
+    clk.mark(TM_SOL_SPARSE);
 }
 
 // ---------------------------------------------------------------- BDF ops policy
@@ -1966,7 +2144,9 @@ PHASE void sparse_solve_phase(const DevNet *Np, Lds L_, const LUT *M)
 {
     const Lds L = uniform_lds(L_);
     PhaseClock clk(L);
-    sparse_lu_solve<LUT>(*(const CST DevNet *)uniform_ptr(Np), L, uniform_ptr(M), L.b, L.flux);
+    NetRef N = *(const CST DevNet *)uniform_ptr(Np);
+    if (N.nw_stage) staged_solve<LUT>(N, L, uniform_ptr(M));
+    else workspace_solve<LUT>(N, L, uniform_ptr(M), L.b, L.flux);
     clk.mark(TM_SOLVE);
 }
 
@@ -1980,18 +2160,20 @@ PHASE void dense_solve_phase(const DevNet *Np, Lds L_, const LUT *M)
     clk.mark(TM_SOLVE);
 }
 
+// J: workspace of a staged plan's tail entries, else the J-form values of a workspace plan
 template <typename LUT>
-PHASE int sparse_setup_phase(const DevNet *Np, Lds L_, LUT *M, double *J, double gamma, bool new_jacobian)
+PHASE int sparse_setup_phase(const DevNet *Np, Lds L_, LUT *M, double *J, double gamma)
 {
     const Lds L = uniform_lds(L_);
     NetRef N = *(const CST DevNet *)uniform_ptr(Np);
     M = uniform_ptr(M);
     J = uniform_ptr(J);
     PhaseClock clk(L);
-    if (new_jacobian) sparse_jacobian(N, L, J);
+    if (N.nw_stage) return staged_setup<LUT>(N, L, M, J, gamma);
+    sparse_jacobian(N, L, J);
     sparse_form_newton<LUT>(N, J, M, gamma, L.prm[P_ENFORCECHARGE] != 0.0);
     clk.mark(TM_JAC);
-    const int r = sparse_lu<LUT>(N, L, M, L.flux, L.red, L.b);
+    const int r = workspace_lu<LUT>(N, L, M);
     clk.mark(TM_LU);
     return r;
 }
@@ -2021,7 +2203,10 @@ struct GpuOps {
     double z0_norm = 0.0;   // WRMS norm of z[0] in the weights of the last set_ewt
     bool equilibrate = false;   // factor W M W^-1 (W = diag(ewt)) instead of M (dense form only)
     bool sparse = true;         // static-pattern sparse plan (else dense LU of the full matrix)
-    double *Jsave = nullptr;    // saved J-form values of the sparse plan (workspace)
+    bool staged = false;        // ...that runs from LDS
+    LDS double *rhs_vec, *sol_vec;
+    int pos[EPT];
+    double *Jsave = nullptr;    // the sparse plan's second workspace (sparse_setup_phase)
     const int *cancel = nullptr;  // highest cancelled launch generation, raised by the host while kernels run
     int gen = 0;                  // this launch's generation
     int polls = 0;
@@ -2030,7 +2215,20 @@ struct GpuOps {
     __device__ __forceinline__ bool cancelled() { return (polls++ & 15) == 0 && cancel_requested(cancel, gen); }
 
     __device__ GpuOps(const DevNet *np_, Lds &l_, LUT *m_)
-        : N(*(const CST DevNet *)np_), Np(np_), L(l_), M(m_), neq(((const CST DevNet *)np_)->neq) {}
+        : N(*(const CST DevNet *)np_), Np(np_), L(l_), M(m_), neq(((const CST DevNet *)np_)->neq)
+    {
+    }
+    // where the Newton system's right-hand side goes and its solution comes from: the staged plan's
+    // vectors in its row order, else L.b
+    __device__ __forceinline__ void use_solver(bool sparse_)
+    {
+        sparse = sparse_;
+        staged = sparse && N.nw_stage;
+        rhs_vec = staged ? L.flux : L.b;
+        sol_vec = staged ? L.flux + 2 * ((N.nw_N + 7) & ~7) : L.b;
+#pragma unroll
+        for (int e = 0; e < EPT; e++) pos[e] = (staged && own(e)) ? glb(N.nw_inv)[idx(e)] : idx(e);
+    }
 
     __device__ __forceinline__ bool own(int e) const { return tid() + e * NT < neq; }
     __device__ __forceinline__ int idx(int e) const { return tid() + e * NT; }
@@ -2179,8 +2377,9 @@ struct GpuOps {
             if (own(e)) {
                 const int i = idx(e);
                 // equilibrated system: b' = W b
-                L.b[i] = (gamma * L.f[i] - (rl1 * z[1][e] + acor[e])) * (equilibrate ? ewt[e] : 1.0);
+                rhs_vec[pos[e]] = (gamma * L.f[i] - (rl1 * z[1][e] + acor[e])) * (equilibrate ? ewt[e] : 1.0);
             }
+        if (staged && tid() < 2) rhs_vec[glb(N.nw_inv)[neq + tid()]] = 0.0;   // the border rows
         __syncthreads();
     }
     __device__ __forceinline__ void solve()
@@ -2195,7 +2394,7 @@ struct GpuOps {
         for (int e = 0; e < EPT; e++)
             if (own(e)) {
                 const int i = idx(e);
-                double d = scale * L.b[i];
+                double d = scale * sol_vec[pos[e]];
                 if (equilibrate) d = d / ewt[e];  // the equilibrated solve returns W d
                 double dw = d * ewt[e];
                 acc += dw * dw;
@@ -2207,16 +2406,15 @@ struct GpuOps {
     }
     // Reusing a saved J between Newton-matrix setups (DVODE's JSV=1) was measured on the
     // seeded grid: 31% more steps (slower Newton convergence) for 7x fewer J evaluations,
-    // a net loss since an analytic J costs under half a factorisation here; kept off.
-    bool reuse_jacobian = false;
-    __device__ bool can_reuse_jacobian() const { return sparse && reuse_jacobian; }
+    // a net loss since an analytic J costs under half a factorisation here; not built in.
+    __device__ bool can_reuse_jacobian() const { return false; }
     __device__ __forceinline__ int setup(double gamma, bool new_jacobian)
     {
 #pragma unroll
         for (int e = 0; e < EPT; e++)
             if (own(e)) L.g[idx(e)] = equilibrate ? ewt[e] : 1.0;
         __syncthreads();
-        const int r = sparse ? sparse_setup_phase<LUT>(Np, L, M, Jsave, gamma, new_jacobian)
+        const int r = sparse ? sparse_setup_phase<LUT>(Np, L, M, Jsave, gamma)
                              : dense_setup_phase<LUT>(Np, L, M, gamma, equilibrate);
         return __builtin_amdgcn_readfirstlane(r);
     }
@@ -2642,7 +2840,7 @@ __global__ __launch_bounds__(NT, UCG_WAVES_PER_EU) void solve_points_kernel(cons
             elemental_start(N, prm, L.y, L.sc[S_DENS]);
         }
         GpuOps<LUT> o(Nq, L, M);
-        o.sparse = A.sparse != 0;
+        o.use_solver(A.sparse != 0);
         o.Jsave = (double *)(slot + A.ws_mat_bytes);
         o.cancel = A.cancel;
         o.equilibrate = !o.sparse && A.equilibrate != 0;
@@ -2881,7 +3079,7 @@ __global__ __launch_bounds__(NT) void rhs_kernel(const DevNet *__restrict__ Np, 
     const int p = blockIdx.x;
     if (p >= A.n) return;
     piece_setup(N, L, A, p);
-    block_rhs(N, L);
+    rhs_phase(Np, L);
     for (int i = tid(); i < N.neq; i += NT) A.y_out[(size_t)p * N.neq + i] = L.f[i];
     if (A.rate_out)
         for (int k = tid(); k < N.nreac; k += NT) A.rate_out[(size_t)p * N.nreac + k] = L.rate[k];
@@ -2898,7 +3096,7 @@ __global__ __launch_bounds__(NT) void jac_kernel(const DevNet *__restrict__ Np, 
     const int p = blockIdx.x;
     if (p >= A.n) return;
     piece_setup(N, L, A, p);
-    block_rhs(N, L);   // leaves the pre-transfer surface total and the photo rates at y
+    rhs_phase(Np, L);   // leaves the pre-transfer surface total and the photo rates at y
     double *M = (double *)((char *)A.ws + (size_t)blockIdx.x * A.ws_stride);
     block_newton_matrix<double>(N, L, M, 0.0, false);   // J itself, before forming I - gamma J
     const int neq = N.neq;
@@ -2921,27 +3119,26 @@ __global__ __launch_bounds__(NT) void newton_solve_kernel(const DevNet *__restri
     // y holds the state for J; the right-hand side is rate_in reinterpreted as [n][neq]
     piece_setup(N, L, A, p);
     block_rates(N, L);
-    block_rhs(N, L);
+    rhs_phase(Np, L);
     for (int i = tid(); i < N.neq; i += NT) L.g[i] = 1.0;
     __syncthreads();
     LUT *M = (LUT *)((char *)A.ws + (size_t)blockIdx.x * A.ws_stride);
     int bad;
     if (A.sparse) {
         double *J = (double *)((char *)A.ws + (size_t)blockIdx.x * A.ws_stride + A.ws_mat_bytes);
-        sparse_jacobian(N, L, J);
-        sparse_form_newton<LUT>(N, J, M, A.gamma, L.prm[P_ENFORCECHARGE] != 0.0);
-        bad = sparse_lu<LUT>(N, L, M, L.flux, L.red, L.b);
+        bad = sparse_setup_phase<LUT>(Np, L, M, J, A.gamma);
     } else {
         block_newton_matrix<LUT>(N, L, M, A.gamma);
         bad = block_lu<LUT>(M, N.neq, N.ld, L.red, L.flux);
     }
-    for (int i = tid(); i < N.neq; i += NT) L.b[i] = A.scal_out[(size_t)p * N.neq + i];
     __syncthreads();
-    if (!bad) {
-        if (A.sparse) sparse_lu_solve<LUT>(N, L, M, L.b, L.flux);
-        else block_lu_solve<LUT>(M, N.neq, N.ld, L.b);
-    }
-    for (int i = tid(); i < N.neq; i += NT) A.y_out[(size_t)p * N.neq + i] = bad ? NAN : L.b[i];
+    GpuOps<LUT> o(Np, L, M);
+    o.use_solver(A.sparse != 0);
+    for (int i = tid(); i < N.neq; i += NT) o.rhs_vec[o.pos[i / NT]] = A.scal_out[(size_t)p * N.neq + i];
+    if (o.staged && tid() < 2) o.rhs_vec[N.nw_inv[N.neq + tid()]] = 0.0;
+    __syncthreads();
+    if (!bad) o.solve();
+    for (int i = tid(); i < N.neq; i += NT) A.y_out[(size_t)p * N.neq + i] = bad ? NAN : o.sol_vec[o.pos[i / NT]];
 }
 
 template __global__ void solve_points_kernel<double>(const DevNet *, SolveArgs);
