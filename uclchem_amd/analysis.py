@@ -37,24 +37,23 @@ def construct_incidence(tables: mh.NetworkTables) -> np.ndarray:
     """[nreac, nspec] int8: +1 per product, -1 per reactant (analysis.py:711-734)."""
     a = tables.arrays
     inc = np.zeros((tables.nreac, tables.nspec), dtype=np.int8)
-    for k in range(tables.nreac):
-        for j in a["pr"][k]:
-            if 0 <= j < tables.nspec:
-                inc[k, j] += 1
-        for j in a["re"][k]:
-            if 0 <= j < tables.nspec:
-                inc[k, j] -= 1
+    for side, sign in ((a["pr"], 1), (a["re"], -1)):
+        side = np.asarray(side)
+        k, m = np.nonzero((side >= 0) & (side < tables.nspec))
+        np.add.at(inc, (k, side[k, m]), np.int8(sign))
     return inc
 
 
 def _swap_pairs(tables: mh.NetworkTables):
     """BULKSWAP and SURFSWAP reactions, each list ordered by its reactant's species index,
     paired in that order (analysis.py:815-826: zip, so as many pairs as the shorter list)."""
-    a = tables.arrays
-    kinds = [mh.ALL_TYPES[int(c)] for c in a["rtype"]]
-    bulk = sorted([k for k in range(tables.nreac) if kinds[k] == "BULKSWAP"], key=lambda k: int(a["re"][k][0]))
-    surf = sorted([k for k in range(tables.nreac) if kinds[k] == "SURFSWAP"], key=lambda k: int(a["re"][k][0]))
-    return list(zip(bulk, surf))
+    rtype, re0 = np.asarray(tables.arrays["rtype"]), np.asarray(tables.arrays["re"])[:, 0]
+
+    def ordered(kind):
+        k = np.flatnonzero(rtype == mh.ALL_TYPES.index(kind))
+        return k[np.argsort(re0[k], kind="stable")].tolist()
+
+    return list(zip(ordered("BULKSWAP"), ordered("SURFSWAP")))
 
 
 def get_total_swap(rates: np.ndarray, abundances: np.ndarray, tables: mh.NetworkTables) -> np.ndarray:
@@ -73,18 +72,18 @@ def flux_names(tables: mh.NetworkTables) -> List[str]:
     C + D", analysis.py's column names): one per reaction, then the geometric swap terms (the
     swap reactions' strings with SWAP replaced by SWAP_GEOMETRIC: every BULKSWAP pair first,
     then every SURFSWAP pair)."""
-    a, names = tables.arrays, tables.species_names
-    kinds = [mh.ALL_TYPES[int(c)] for c in a["rtype"]]
+    a, names, ns = tables.arrays, tables.species_names, tables.nspec
+    re_, pr_ = np.asarray(a["re"]).tolist(), np.asarray(a["pr"]).tolist()
+    tail = ["" if t == "TWOBODY" else " + " + t for t in mh.ALL_TYPES]
 
-    def text(k, kind):
-        re = [names[j] for j in a["re"][k] if 0 <= j < tables.nspec]
-        pr = [names[j] for j in a["pr"][k] if 0 <= j < tables.nspec]
-        return " + ".join(re + ([kind] if kind != "TWOBODY" else [])) + " -> " + " + ".join(pr)
+    def text(k, kind):   # kind: what follows the reactants
+        return (" + ".join([names[j] for j in re_[k] if 0 <= j < ns]) + kind + " -> " +
+                " + ".join([names[j] for j in pr_[k] if 0 <= j < ns]))
 
-    cols = [text(k, kinds[k]) for k in range(tables.nreac)]
+    cols = [text(k, tail[c]) for k, c in enumerate(np.asarray(a["rtype"]).tolist())]
     pairs = _swap_pairs(tables)
-    cols += [text(b, "BULKSWAP_GEOMETRIC") for b, _ in pairs]
-    cols += [text(s, "SURFSWAP_GEOMETRIC") for _, s in pairs]
+    cols += [text(b, " + BULKSWAP_GEOMETRIC") for b, _ in pairs]
+    cols += [text(s, " + SURFSWAP_GEOMETRIC") for _, s in pairs]
     return cols
 
 
@@ -132,20 +131,21 @@ def rates_to_dy_and_flux(physics: np.ndarray, abundances: np.ndarray, rates: np.
     inc = construct_incidence(tables).astype(np.float64)
     a = tables.arrays
     ab = abundances.reshape(n, -1)
-    pre = flux @ inc                                            # dy before the bulk<->surface transfer
-    surface = pre[:, np.asarray(a["surface_list"], dtype=int)].sum(axis=1)
+    # what the terms change of the surface as a whole, before the bulk<->surface transfer
+    surface = flux @ inc[:, np.asarray(a["surface_list"], dtype=int)].sum(axis=1)
     ysurf, ybulk = ab[:, tables.scalars["nsurface"]], ab[:, tables.scalars["nbulk"]]
     pairs = _swap_pairs(tables)
     geo = np.zeros((n, 2 * len(pairs)))
     cover_up = 0.5 * GAS_DUST_DENSITY_RATIO / NUM_SITES_PER_GRAIN
-    with np.errstate(divide="ignore", invalid="ignore"):
-        for i, (b, s) in enumerate(pairs):
-            shrink = surface < 0.0
-            cov = np.minimum(1.0, ybulk / ysurf)
-            geo[:, i] = np.where(shrink, surface * cov * ab[:, int(a["re"][b][0])] / ybulk, 0.0)
-            geo[:, len(pairs) + i] = np.where(shrink, 0.0, surface * cover_up * ab[:, int(a["re"][s][0])])
+    if pairs:
+        yb, ys = ab[:, np.asarray(a["re"])[[b for b, _ in pairs], 0]], ab[:, np.asarray(a["re"])[[s for _, s in pairs], 0]]
+        shrink, col = (surface < 0.0)[:, None], surface[:, None]
+        with np.errstate(divide="ignore", invalid="ignore"):
+            cov = np.minimum(1.0, ybulk / ysurf)[:, None]
+            geo[:, :len(pairs)] = np.where(shrink, col * cov * yb / ybulk[:, None], 0.0)
+            geo[:, len(pairs):] = np.where(shrink, 0.0, col * cover_up * ys)
     if reference_signs:   # analysis.py:846-870 and 884-885, as the reference applies them
-        d = pre.copy()
+        d = flux @ inc                                          # dy before the transfer
         for i, (b, s) in enumerate(pairs):
             rb, pb = int(a["re"][b][0]), int(a["pr"][b][0])
             rs, ps = int(a["re"][s][0]), int(a["pr"][s][0])
