@@ -183,13 +183,14 @@ int upload(NetHandle &h, const T *src, size_t n, const T *&dst)
 int upload_program(NetHandle &h, const ucg::Program &P, ucg::DevProg &D)
 {
     int rc;
-    if ((rc = upload(h, P.slices.data(), P.slices.size(), D.slices)) ||
-        (rc = upload(h, P.wave_ptr.data(), P.wave_ptr.size(), D.wave_ptr)) ||
-        (rc = upload(h, P.hdr.data(), P.hdr.size(), D.hdr)) || (rc = upload(h, P.rec.data(), P.rec.size(), D.rec)))
+    if ((rc = upload(h, P.list.data(), P.list.size(), D.list)) ||
+        (rc = upload(h, P.list_ptr.data(), P.list_ptr.size(), D.list_ptr)) ||
+        (rc = upload(h, P.hdr.data(), P.hdr.size(), D.hdr)))
         return rc;
-    D.phases = P.phases;
-    D.n_hdr = (int)P.hdr.size();
-    return 0;
+    // a lane may fetch one record past a list's end
+    std::vector<uint32_t> rec(P.rec);
+    rec.resize(rec.size() + 512, 0u);
+    return upload(h, rec.data(), rec.size(), D.rec);
 }
 
 NetHandle *get(int handle)
@@ -307,7 +308,7 @@ SlotLayout slot_layout(const ucg::DevNet &N, bool sparse, int lu_bits)
         // a staged plan's factors and waiting tail entries need less; the slot keeps that size, so
         // that a budget or the fixed workspace holds the same number of slots either way
         s.mat = al(((size_t)N.sp_nstream + ucg::tail_len(N.sp_T)) * elem);
-        s.jac = al((size_t)(N.pg_entries.n_hdr - N.sp_tail_hdr) * sizeof(double));
+        s.jac = al((size_t)(N.sp_end_hdr - N.sp_tail_hdr) * sizeof(double));
         both = std::max(both, s.mat + s.jac);
         s.jac = both - s.mat;
     }
@@ -760,6 +761,7 @@ static int load_staged_plan(const ucg_network_desc *d, NetHandle &h, size_t lds_
     N.sp_nstream = (int)S.stream.size();
     N.sp_L = S.at_L;
     N.sp_tail_hdr = S.tail_hdr;
+    N.sp_end_hdr = S.end_hdr;
     N.sp_slots = S.n_slots;
     for (int k = 0; k < 4; k++) N.sp_at[k] = S.at[k];
     N.sp_w0 = std::max(N.px.n, S.t * S.t - S.at_L);   // the tail must end before L21
@@ -771,6 +773,7 @@ static int load_staged_plan(const ucg_network_desc *d, NetHandle &h, size_t lds_
     }
     int rc;
     if ((rc = upload(h, S.stream.data(), S.stream.size(), N.sp_stream)) ||
+        (rc = upload(h, S.tail_wave.data(), S.tail_wave.size(), N.sp_tail_wave)) ||
         (rc = upload(h, S.sum_rows.data(), S.sum_rows.size(), N.sp_sum_rows)) ||
         (rc = upload(h, S.sum_members.data(), S.sum_members.size(), N.sp_sum_members)) ||
         (rc = upload_program(h, S.entries, N.pg_entries)) || (rc = upload_program(h, S.elim, N.pg_elim)) ||
@@ -914,6 +917,7 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
         P.add(ucg::pack_slices(len, ucg::NWAVE), ucg::NWAVE, 1, 2, 4,
               [&](int it, uint32_t *w) { w[0] = it >= 0 ? (ucg::HDR_VALID | (uint32_t)it) : 0u; },
               [&](int it, int e, int k, uint32_t *w) { ucg::put16(w, k, e >= 0 ? op[it][e] : (unsigned)d->nreac); }, len);
+        P.finish(ucg::NWAVE, true);
         if ((rc = upload_program(h, P, N.pg_sum))) return rc;
     }
     {   // packed term records {n_d, ops[6], nfac}

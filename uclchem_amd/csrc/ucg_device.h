@@ -88,10 +88,8 @@ constexpr double MIN_ABUND = 1.0e-30;
 
 // A program of the planner (ucg_plan.h) on the device.
 struct DevProg {
-    const int32_t *slices;     // [n][4]
-    const int32_t *wave_ptr;   // [phases][NWAVE + 1]
+    const int32_t *list, *list_ptr;   // slice descriptors by wave, [NWAVE + 1] their ranges
     const uint32_t *hdr, *rec;
-    int32_t phases, n_hdr;
 };
 constexpr int NWAVE = NT / 64;
 
@@ -137,7 +135,8 @@ struct DevNet {
     // Newton matrix of a staged plan: operand slots, entries, elimination, Schur update, solves
     PartialSlots px;
     int32_t sp_ns, sp_T, sp_nstream, sp_L, sp_slots, sp_at[4], sp_w0, sp_presum;
-    int32_t sp_tail_hdr;         // first header of the tail entries; their values wait in the workspace from there on
+    int32_t sp_tail_hdr, sp_end_hdr;   // headers of the tail entries, whose values wait in the workspace
+    const int32_t *sp_tail_wave;       // [NWAVE + 1] the waves' shares of them
     const uint32_t *sp_stream;
     const int32_t *sp_sum_rows, *sp_sum_members;
     DevProg pg_entries, pg_elim, pg_schur, pg_solve[4];
@@ -168,7 +167,7 @@ __device__ __forceinline__ NetRef fresh(NetRef N)
 // length (in doubles) of the LDS region the phases share: the reaction fluxes (RHS); the operands
 // of the Newton-matrix entries with the sparse pivots' working slots behind them; the dense tail,
 // which overlays both but for the L21 and U12 streams at the end; the exchange buffers of the
-// tail's inversion; the solve's three vectors.  Plans whose tail does not fit (strongly coupled
+// tail's inversion, in the tail's place; the solve's three vectors.  Plans whose tail does not fit (strongly coupled
 // networks) keep their factors in the workspace and need the term partials and a work vector.
 template <class Net>
 __host__ __device__ inline int flux_region_len(const Net &N)
@@ -180,8 +179,9 @@ __host__ __device__ inline int flux_region_len(const Net &N)
     const int b = b1 > NT ? b1 : NT;                 // >= one value per thread (ordered_sum)
     if (!N.nw_stage) return b;
     const int c = N.sp_w0 + N.sp_slots;
-    const int gj = N.sp_T * N.sp_T + 2 * ((N.sp_T + 15) / 16 + 1) * 16 * 17;
-    const int e = c > gj ? c : gj;
+    const int gj = (2 * ((N.sp_T + 15) / 16 + 1) + 1) * 16 * 17, tt = N.sp_T * N.sp_T;
+    const int e0 = c > gj ? c : gj;
+    const int e = e0 > tt ? e0 : tt;
     return b > e ? b : e;
 }
 

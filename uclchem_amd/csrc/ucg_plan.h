@@ -98,14 +98,38 @@ inline SliceSet pack_slices(const std::vector<int> &length, int nwave, double co
     return best;
 }
 
-// Device form of one or more phases: slice descriptors (int4), the waves' slice ranges, headers
-// (one per lane) and operand records (RW 32-bit words per lane and row; `per_row` positions a row).
+// Device form of one or more phases: slice descriptors, headers (one per lane) and operand records
+// (RW 32-bit words per lane and row; `per_row` positions a row).  finish() gives every wave its
+// slices of all phases as one list with the barriers that follow each, so that a wave can hold its
+// descriptors in its lanes and fetch ahead across phases; `joined` puts no barriers between phases.
 struct Program {
     std::vector<int> slices;       // [n][4] {first record row, rows, lanes per item, first header}
     std::vector<int> wave_ptr;     // [phases][nwave + 1]
     std::vector<uint32_t> hdr;     // [slice][64][hw]
     std::vector<uint32_t> rec;     // [row][64][rw]
+    std::vector<int> list;         // [n][4] {first record row, rows, lanes per item + 256 x barriers after, first header}
+    std::vector<int> list_ptr;     // [nwave + 1]
     int phases = 0;
+
+    void finish(int nwave, bool joined = false)
+    {
+        const int none = (int)hdr.size();             // a header row of lanes without an item
+        hdr.resize(hdr.size() + 64, 0u);
+        list.clear();
+        list_ptr.assign(1, 0);
+        for (int w = 0; w < nwave; w++) {
+            const size_t at = list.size();
+            for (int p = 0; p < phases; p++) {
+                const int *wp = &wave_ptr[p * (nwave + 1) + w];
+                for (int s = wp[0]; s < wp[1]; s++) list.insert(list.end(), &slices[4 * s], &slices[4 * s] + 4);
+                if (joined) continue;
+                if (list.size() == at) list.insert(list.end(), {0, 0, 1, none});   // nothing yet in any phase
+                list[list.size() - 2] += 256;
+            }
+            list_ptr.push_back((int)list.size() / 4);
+        }
+        list.resize(list.size() + 4 * 64, 0);         // lanes read a full wave of descriptors
+    }
 
     // head(item or -1, words): fills the lane's header; entry(item, e, slot in row, words): fills
     // operand e of the item (or padding when e < 0) at its place in the row's words.
@@ -184,9 +208,10 @@ constexpr unsigned NO_SLOT = 0xffffu;
 // at[k].
 struct SparsePrograms {
     int ns = 0, t = 0, nlev = 0;
-    int at_L = 0, zero = 0, n_slots = 0, tail_hdr = 0;
+    int at_L = 0, zero = 0, n_slots = 0, tail_hdr = 0, end_hdr = 0;
     int at[4] = {0, 0, 0, 0};
     std::vector<uint32_t> stream;
+    std::vector<int> tail_wave;       // [nwave + 1] first tail-entry header of each wave
     bool presum = false;              // the sum rows are not all tail rows: subtract sums up front
     std::vector<int> sum_rows;        // presum: {row, first, end} of the permuted members
     std::vector<int> sum_members;
@@ -597,6 +622,15 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
             P, nwave, 1, 2, 4, [&](int i, uint32_t *h) { h[0] = i >= 0 ? head[i] : 0u; },
             [&](int i, int e, int k, uint32_t *w) { put16(w, k, e >= 0 ? op[i][e] : (unsigned)ps.zero); }, len);
     }
+    S.end_hdr = (int)S.entries.hdr.size();
+    for (int w = 0; w <= nwave; w++) {   // the waves' tail headers: contiguous, one row of 64 a slice
+        const int s = S.entries.wave_ptr[nwave + 1 + w];
+        S.tail_wave.push_back(4 * (size_t)s < S.entries.slices.size() ? S.entries.slices[4 * s + 3] : S.end_hdr);
+    }
+    S.elim.finish(nwave);
+    S.schur.finish(nwave, true);
+    S.entries.finish(nwave, true);
+    for (Program &P : S.solve) P.finish(nwave, true);
     S.ok = ps.n < 0x8000;
     return S;
 }

@@ -463,25 +463,72 @@ __device__ __forceinline__ double group_sum(double v, int G)
 }
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(tid() >> 6); }
 
-// A wave's slices of one program phase (ucg_plan.h): load(row) fetches a row's record, use(record)
-// adds it up, done(header, lanes per item, header index) ends a slice.  A plain loop on purpose:
-// keeping rows in flight across slice boundaries (a register ring, unrolled with the slice's end in
-// every position) made the phases slower, the set-up 60 -> 66 us: the code of a step is several
-// times the instruction cache, and its size costs more than the loads' latency.
-template <int U, class Load, class Use, class Done>
-__device__ __forceinline__ void run_slices(const CST DevProg &G, int phase, Load load, Use use, Done done)
-{
-    const GLB int *wp = glb(G.wave_ptr) + phase * (NWAVE + 1) + wave_id(), *slices = glb(G.slices);
-    const GLB uint32_t *hdr = glb(G.hdr) + (tid() & 63);
-    const int s1 = wp[1];
-    for (int s = wp[0]; s < s1; s++) {
-        const int row = slices[4 * s], rows = slices[4 * s + 1], G_ = slices[4 * s + 2], h0 = slices[4 * s + 3];
-        const uint32_t h = hdr[h0];
-#pragma unroll U
-        for (int r = 0; r < rows; r++) use(load(row + r));
-        done(h, G_, h0);
+// A wave's slices of a program (ucg_plan.h): load(row) fetches a row's record, use(record) adds it
+// up, done(header, lanes per item, header index) ends a slice; then the slice's barriers.  The
+// descriptors sit in the wave's lanes (scalar loads share the LDS counter, so that every gather
+// would wait for the next descriptor), and the header and first records of the next slice are in
+// flight while a slice is worked on, across barriers too.  Against scalar descriptors and no
+// fetching ahead: matrix entries 17.6 -> 16.1 us a set-up, elimination and Schur update 27 -> 24.
+// list() and first() can be called well ahead of run(), before the barrier that the phase's data
+// waits for; D rows of a slice are fetched ahead.
+template <class Rec, int D>
+struct Slices {
+    int s0, n;
+    int4 d;
+    Rec cur[D];
+    uint32_t h;
+    static __device__ __forceinline__ int field(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
+    __device__ __forceinline__ void list(const CST DevProg &G)
+    {
+        const GLB int *lp = glb(G.list_ptr) + wave_id();
+        s0 = lp[0];
+        n = lp[1] - s0;
+        d = ld_int4(glb(G.list), s0 + (tid() & 63));
     }
-}
+    template <class Load>
+    __device__ __forceinline__ void ahead(const CST DevProg &G, int i, Rec *buf, uint32_t &hd, Load load)
+    {
+        const int row = field(d.x, i), rows = field(d.y, i);
+        hd = glb(G.hdr)[field(d.w, i) + (tid() & 63)];
+#pragma unroll
+        for (int u = 0; u < D; u++)
+            if (u < rows) buf[u] = load(row + u);
+    }
+    template <class Load>
+    __device__ __forceinline__ void first(const CST DevProg &G, Load load)
+    {
+        if (n > 0) ahead(G, 0, cur, h, load);
+    }
+    template <int U, class Load, class Use, class Done>
+    __device__ __forceinline__ void run(const CST DevProg &G, Load load, Use use, Done done)
+    {
+        while (n > 0) {
+            const int m = min(64, n);
+#pragma unroll 1
+            for (int i = 0; i < m; i++) {
+                const int row = field(d.x, i), rows = field(d.y, i), gb = field(d.z, i), hi = field(d.w, i);
+                Rec nxt[D];
+                uint32_t hn = 0;
+                if (i + 1 < m) ahead(G, i + 1, nxt, hn, load);
+#pragma unroll
+                for (int u = 0; u < D; u++)
+                    if (u < rows) use(cur[u]);
+#pragma unroll U
+                for (int r = D; r < rows; r++) use(load(row + r));
+                done(h, gb & 255, hi);
+#pragma unroll
+                for (int u = 0; u < D; u++) cur[u] = nxt[u];
+                h = hn;
+                for (int k = gb >> 8; k > 0; k--) __syncthreads();
+            }
+            n -= 64;
+            if (n <= 0) return;
+            s0 += 64;
+            d = ld_int4(glb(G.list), s0 + (tid() & 63));
+            first(G, load);
+        }
+    }
+};
 
 // a factor product over the extended state, four factors a record
 __device__ __forceinline__ double term4(uint2 w, double r, const LDS double *y)
@@ -529,6 +576,8 @@ __device__ __forceinline__ void block_rhs(NetRef N_, const Lds L)
     LDS double *y = L.y, *f = L.f, *flux = L.flux, *sc = L.sc;
     double *rate = L.rate;
     const LDS double *prm = L.prm;
+    Slices<uint2, 8> sums;
+    sums.list(N.pg_sum);
     const double D = y[neq - 1];
     const double sm = fmax(1e-30, y[N.nsurface]);
     const double sbk = fmax(1e-30, y[N.nbulk]);
@@ -596,12 +645,13 @@ __device__ __forceinline__ void block_rhs(NetRef N_, const Lds L)
     }
     const GLB uint32_t *srec = glb(N.pg_sum.rec) + 2 * lane;
     const auto load = [&](int r) { return ld_uint2(srec, 64 * r); };
+    sums.first(N.pg_sum, load);
     __syncthreads();
     clk.mark(TM_RHS_FLUX);
     {
         double a0 = 0.0, a1 = 0.0;
-        run_slices<2>(
-            N.pg_sum, 0, load,
+        sums.run<2>(
+            N.pg_sum, load,
             [&](uint2 q) {
                 a0 += signed_entry(flux, q.x);
                 a1 += signed_entry(flux, q.x >> 16);
@@ -1206,21 +1256,22 @@ UCG_BIG __device__ int block_lu_tiled(MP M, int n, int ld, LDS double *red, LDS 
 // layout of v_mfma_f64_16x16x4: wave w holds block column w as nb tiles of four doubles per lane
 // (lane 16g + c, register i: row 4i + g, column c) from the first sweep to the last.  In that
 // layout a tile is also a B operand (register i = k-step i), so a sweep only exchanges the pivot
-// column: its owner inverts the pivot block in registers and publishes the inverse and the
-// negated column panel through LDS (double-buffered: one barrier a sweep); every wave then forms
+// column: its owner publishes the pivot block, a wave without a column inverts it in registers
+// while the others finish their updates of the sweep before, and the owner publishes its negated
+// column panel (double-buffered, two barriers a sweep); every wave then forms
 // P = inv(A_KK) A_KJ and A_IJ += (-A_IK) P with 4 MFMAs a tile.  The owner's own column takes the
 // same update with P = inv(A_KK) and zero tiles, which leaves -A_IK inv(A_KK).
 //
 // The register-blocked sweeps over LDS that this replaces (8 pivots a sweep) took 105 us for the
 // default network's 104 rows, bound by LDS round trips and three barriers a sweep; this form takes
-// 35 us.  Its floor is the matrix cores' 10 us for 2 n^3 FLOP at FP64 on one CU; the pivot
-// blocks' serial inversions (16 dependent steps each) are most of the rest.
+// 26 us, 32 when the owner inverts its block itself.  Its floor is the matrix cores' 10 us for
+// 2 n^3 FLOP at FP64 on one CU; a pivot block's inversion is 16 dependent steps, 1.5 us.
 constexpr int GJ_MAX = 16 * NWAVE;        // rows one workgroup's waves can hold
 constexpr int GJ_TILE = 16 * 17;          // LDS tile, column-major, column stride 17 (bank spread)
 using f64x4 = __attribute__((ext_vector_type(4))) double;
 
-// LDS doubles of the exchange buffers: two generations of inverse + panel
-__host__ __device__ inline int gj_stage_len(int n) { return 2 * ((n + 15) / 16 + 1) * GJ_TILE; }
+// LDS doubles of the exchange buffers: two generations of inverse + panel, the next pivot block
+__host__ __device__ inline int gj_stage_len(int n) { return (2 * ((n + 15) / 16 + 1) + 1) * GJ_TILE; }
 
 template <int R> __device__ __forceinline__ unsigned rows_bcast32(unsigned v)
 {   // row R of 16 lanes, to all four rows
@@ -1264,7 +1315,7 @@ template <int K> __device__ __forceinline__ void gj16_steps(f64x4 &d, int g, int
 
 // A: n x n, column-major, leading dimension n, in LDS.  The inverse goes to `out` in blocks of four
 // columns, row-major inside a block (tail_index), the order in which the solve's lanes read it.
-// `stage`: LDS scratch of gj_stage_len(n) doubles outside A.  Returns nonzero (uniformly) on a zero
+// `stage`: LDS scratch of gj_stage_len(n) doubles, which may be A's own.  Returns nonzero (uniformly) on a zero
 // or non-finite pivot.
 __device__ __forceinline__ int tail_index(int n, int row, int col) { return (col >> 2) * 4 * n + 4 * row + (col & 3); }
 __host__ __device__ inline int tail_len(int n) { return ((n + 3) & ~3) * n; }
@@ -1284,44 +1335,54 @@ __device__ __forceinline__ int block_gj_inverse(const LDS double *A, int n, LDS 
             t[I][i] = (row < n && col < n) ? A[col * n + row] : (row == col ? 1.0 : 0.0);
         }
     __syncthreads();
-    f64x4 mine = {0.0, 0.0, 0.0, 0.0};   // the owner's inverted pivot block
+    // the pivot blocks are inverted by a wave without a column while the others update theirs; with
+    // eight columns by the block's owner
+    LDS double *diag = stage + 2 * gen;
     for (int K = -1; K < nb; K++) {
         const LDS double *inv = stage + (K & 1) * gen, *panel = inv + GJ_TILE;
-        f64x4 P = mine;
+        LDS double *ninv = stage + ((K + 1) & 1) * gen, *npanel = ninv + GJ_TILE;
+        const bool next = w == K + 1 && w < nb;
+        f64x4 P = {0.0, 0.0, 0.0, 0.0};
         if (K >= 0) {
             __syncthreads();
             if (red[8] != 0.0) return 1;
-            if (w != K && w < nb) {
+            if (w == K) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) P[i] = inv[17 * c + 4 * i + g];
+            } else if (w < nb) {
                 f64x4 b = t[0];
 #pragma unroll
                 for (int I = 1; I < NWAVE; I++)
                     if (I == K) b = t[I];
-                P = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
                 for (int s = 0; s < 4; s++)
                     P = __builtin_amdgcn_mfma_f64_16x16x4f64(inv[17 * (4 * s + g) + c], b[s], P, 0, 0, 0);
             }
         }
-        // the next pivot block's owner updates that block first and inverts it while the other
-        // waves' matrix instructions of this sweep run
-        const bool next = w == K + 1 && w < nb;
-        LDS double *ninv = stage + ((K + 1) & 1) * gen, *npanel = ninv + GJ_TILE;
-        if (next) {
-            mine = t[0];
+        if (next) {   // the next pivot block first
+            f64x4 m = t[0];
 #pragma unroll
             for (int I = 1; I < NWAVE; I++)
-                if (I == w) mine = t[I];
+                if (I == w) m = t[I];
             if (K >= 0) {
                 const LDS double *pw = panel + w * GJ_TILE;
 #pragma unroll
                 for (int s = 0; s < 4; s++)
-                    mine = __builtin_amdgcn_mfma_f64_16x16x4f64(pw[17 * (4 * s + g) + c], P[s], mine, 0, 0, 0);
+                    m = __builtin_amdgcn_mfma_f64_16x16x4f64(pw[17 * (4 * s + g) + c], P[s], m, 0, 0, 0);
             }
+#pragma unroll
+            for (int i = 0; i < 4; i++) diag[17 * c + 4 * i + g] = m[i];
+        }
+        __syncthreads();
+        if (K + 1 < nb && w == (nb < NWAVE ? nb : K + 1)) {
+            f64x4 m;
+#pragma unroll
+            for (int i = 0; i < 4; i++) m[i] = diag[17 * c + 4 * i + g];
             bool bad = false;
-            gj16_steps<0>(mine, g, c, bad);
+            gj16_steps<0>(m, g, c, bad);
             if (bad) red[8] = 1.0;
 #pragma unroll
-            for (int i = 0; i < 4; i++) ninv[17 * c + 4 * i + g] = mine[i];
+            for (int i = 0; i < 4; i++) ninv[17 * c + 4 * i + g] = m[i];
         }
         if (K >= 0 && w < nb) {
 #pragma unroll
@@ -1812,9 +1873,8 @@ UCG_BIG __device__ void workspace_solve(NetRef N_, const Lds L, const LUT *Vg, L
 // hundred products and turns a solve's two level-by-level sweeps into two products), then the
 // inverse of the tail.  Default network, FP64, per call on an otherwise idle chip, against the form
 // with the Jacobian, the matrix and the level-by-level elimination passed through the workspace:
-// Jacobian and matrix 68 -> 18 us, sparse part 51 -> 27 us, solve 33 -> 7 us.  What bounds it now:
-// LDS gathers and the latency of a dozen short phases, and the instruction cache, which a step's
-// code exceeds several times.
+// Jacobian and matrix 68 -> 18 us, sparse part 51 -> 27 us, solve 33 -> 7 us.  Bound by LDS gathers
+// and the latency of some twenty short phases.
 
 // Operands of the entries: partials of every term by each of its factors, and the structured
 // couplings' slots (PartialSlots).  Right after block_rhs at the same state, whose totalSwap it uses.
@@ -1926,60 +1986,55 @@ __device__ __forceinline__ void partial_operands(NetRef N, const Lds &L, LDS dou
 
 // Entries of M = I - gamma J: working slots to LDS (W), tail entries to the workspace, where the
 // same lane fetches them once the operands' LDS is free.
-__device__ __forceinline__ void newton_entries(NetRef N, const LDS double *P, LDS double *W, double *stage, double gamma,
-                                               bool charge)
+__device__ __forceinline__ void newton_entries(NetRef N, Slices<uint2, 2> &run, const LDS double *P, LDS double *W, double *stage,
+                                               double gamma, bool charge)
 {
     const int lane = tid() & 63;
     const GLB uint32_t *rec = glb(N.pg_entries.rec) + 2 * lane;
     GLB double *st = glbw(stage) - N.sp_tail_hdr + lane;
     const auto load = [&](int r) { return ld_uint2(rec, 64 * r); };
-    for (int part = 0; part < 2; part++) {
-        double a0 = 0.0, a1 = 0.0;
-        run_slices<2>(
-            N.pg_entries, part, load,
-            [&](uint2 q) {
-                a0 += signed_entry(P, q.x);
-                a1 += signed_entry(P, q.x >> 16);
-                a0 += signed_entry(P, q.y);
-                a1 += signed_entry(P, q.y >> 16);
-            },
-            [&](uint32_t h, int G, int hdr) {
-                const double acc = group_sum(a0 + a1, G);
-                a0 = a1 = 0.0;
-                double v = (h & ENTRY_UNSCALED) ? acc : -gamma * acc;
-                v += (h & ENTRY_ONE) ? 1.0 : (h & ENTRY_MINUS) ? -1.0 : 0.0;
-                if (charge && (h & ENTRY_CHARGE)) v = (h & ENTRY_CHARGE_ONE) ? 1.0 : (h & ENTRY_CHARGE_MINUS) ? -1.0 : 0.0;
-                if (h & ENTRY_VALID) {
-                    if (part == 0) W[h & ENTRY_TARGET] = v;
-                    else st[hdr] = v;
-                }
-            });
-    }
+    double a0 = 0.0, a1 = 0.0;
+    run.run<2>(
+        N.pg_entries, load,
+        [&](uint2 q) {
+            a0 += signed_entry(P, q.x);
+            a1 += signed_entry(P, q.x >> 16);
+            a0 += signed_entry(P, q.y);
+            a1 += signed_entry(P, q.y >> 16);
+        },
+        [&](uint32_t h, int G, int hdr) {
+            const double acc = group_sum(a0 + a1, G);
+            a0 = a1 = 0.0;
+            double v = (h & ENTRY_UNSCALED) ? acc : -gamma * acc;
+            v += (h & ENTRY_ONE) ? 1.0 : (h & ENTRY_MINUS) ? -1.0 : 0.0;
+            if (charge && (h & ENTRY_CHARGE)) v = (h & ENTRY_CHARGE_ONE) ? 1.0 : (h & ENTRY_CHARGE_MINUS) ? -1.0 : 0.0;
+            if (h & ENTRY_VALID) {
+                if (h & ENTRY_TAIL) st[hdr] = v;
+                else W[h & ENTRY_TARGET] = v;
+            }
+        });
 }
 
 // Elimination of the sparse pivots, one phase a level; zero or non-finite pivots raise red[9].
-__device__ __forceinline__ void eliminate(NetRef N, LDS double *W, LDS double *red)
+__device__ __forceinline__ void eliminate(NetRef N, Slices<uint2, 2> &run, LDS double *W, LDS double *red)
 {
     const GLB uint32_t *rec = glb(N.pg_elim.rec) + 2 * (tid() & 63);
     const auto load = [&](int r) { return ld_uint2(rec, 64 * r); };
-    for (int p = 0; p < N.pg_elim.phases; p++) {
-        double acc = 0.0;
-        run_slices<2>(
-            N.pg_elim, p, load, [&](uint2 q) { acc += W[q.x & 0xffff] * (W[q.x >> 16] * W[q.y & 0xffff]); },
-            [&](uint32_t h, int G, int) {
-                const double s = group_sum(acc, G);
-                acc = 0.0;
-                if (h & HDR_VALID) {
-                    double v = W[h & HDR_INDEX] - s;
-                    if (h & HDR_RECIP) {
-                        if (!(v == v) || v == 0.0 || isinf(v)) red[9] = 1.0;
-                        v = fast_rcp(v);
-                    }
-                    W[h & HDR_INDEX] = v;
+    double acc = 0.0;
+    run.run<2>(
+        N.pg_elim, load, [&](uint2 q) { acc += W[q.x & 0xffff] * (W[q.x >> 16] * W[q.y & 0xffff]); },
+        [&](uint32_t h, int G, int) {
+            const double s = group_sum(acc, G);
+            acc = 0.0;
+            if (h & HDR_VALID) {
+                double v = W[h & HDR_INDEX] - s;
+                if (h & HDR_RECIP) {
+                    if (!(v == v) || v == 0.0 || isinf(v)) red[9] = 1.0;
+                    v = fast_rcp(v);
                 }
-            });
-        __syncthreads();
-    }
+                W[h & HDR_INDEX] = v;
+            }
+        });
 }
 
 template <typename LUT>
@@ -1992,13 +2047,22 @@ __device__ __forceinline__ int staged_setup(NetRef N_, const Lds &L, LUT *V, dou
     LDS double *P = L.flux, *W = L.flux + N.sp_w0, *tl = L.flux, *red = L.red;
     if (tid() == 0) red[9] = 0.0;
     for (int q = tid(); q < N.sp_slots; q += NT) W[q] = 0.0;
+    const auto rec_of = [&](const CST DevProg &G) {
+        return [rec = glb(G.rec) + 2 * lane](int r) { return ld_uint2(rec, 64 * r); };
+    };
+    Slices<uint2, 2> entries, pivots;
+    Slices<uint2, 4> schur;
+    entries.list(N.pg_entries);
     partial_operands(N, L, P);
+    entries.first(N.pg_entries, rec_of(N.pg_entries));
+    pivots.list(N.pg_elim);
     __syncthreads();
-    newton_entries(N, P, W, stage, gamma, charge);
+    newton_entries(N, entries, P, W, stage, gamma, charge);
+    pivots.first(N.pg_elim, rec_of(N.pg_elim));
     __syncthreads();
     clk.mark(TM_JAC);
     PhaseClock lu(L);
-    eliminate(N, W, red);
+    eliminate(N, pivots, W, red);
     if (red[9] != 0.0) return 1;
     {   // store the streams, scaled by their columns' pivots; the Schur update needs L21 scaled
         const GLB uint32_t *from = glb(N.sp_stream);
@@ -2014,27 +2078,27 @@ __device__ __forceinline__ int staged_setup(NetRef N_, const Lds &L, LUT *V, dou
             out[q] = (LUT)v;
         }
     }
+    schur.list(N.pg_schur);
     __syncthreads();
     for (int q = tid(); q < T * T; q += NT) tl[q] = 0.0;
     __syncthreads();
     {   // this lane's tail entries
         const GLB uint32_t *hdr = glb(N.pg_entries.hdr);
-        const GLB int *slices = glb(N.pg_entries.slices), *wp = glb(N.pg_entries.wave_ptr) + NWAVE + 1;
         const GLB double *st = glb((const double *)stage) - N.sp_tail_hdr;
-        const int s1 = wp[w + 1];
-        for (int s = wp[w]; s < s1; s++) {
-            const int h0 = slices[4 * s + 3] + lane;
+        const int h1 = glb(N.sp_tail_wave)[w + 1];
+#pragma unroll 4
+        for (int h0 = glb(N.sp_tail_wave)[w] + lane; h0 < h1; h0 += 64) {
             const uint32_t h = hdr[h0];
-            if (h & ENTRY_VALID) tl[h & ENTRY_TARGET] = st[h0];
+            const double v = st[h0];
+            if (h & ENTRY_VALID) tl[h & ENTRY_TARGET] = v;
         }
     }
+    schur.first(N.pg_schur, rec_of(N.pg_schur));
     __syncthreads();
     {   // Schur complement
-        const GLB uint32_t *rec = glb(N.pg_schur.rec) + 2 * lane;
-        const auto load = [&](int r) { return ld_uint2(rec, 64 * r); };
         double a0 = 0.0, a1 = 0.0;
-        run_slices<4>(
-            N.pg_schur, 0, load,
+        schur.run<4>(
+            N.pg_schur, rec_of(N.pg_schur),
             [&](uint2 q) {
                 a0 += W[q.x & 0xffff] * W[q.x >> 16];
                 a1 += W[q.y & 0xffff] * W[q.y >> 16];
@@ -2047,27 +2111,43 @@ __device__ __forceinline__ int staged_setup(NetRef N_, const Lds &L, LUT *V, dou
     }
     __syncthreads();
     clk.mark(TM_LU_SPARSE);
-    const int r = T > 0 ? block_gj_inverse<LUT>(tl, T, red, L.flux + T * T, V + N.sp_nstream) : 0;
+    const int r = T > 0 ? block_gj_inverse<LUT>(tl, T, red, L.flux, V + N.sp_nstream) : 0;
     clk.mark(TM_LU_TAIL);
     lu.mark(TM_LU);
     return r;
 }
 
 // One stream phase of a solve: stored values times entries of the vectors at vec, summed by row.
-template <typename LUT, class Out>
-__device__ __forceinline__ void stream_phase(const CST DevProg &G, const LUT *v, const LDS double *vec, Out out)
-{
-    const GLB LUT *vals = glb(v) + (tid() & 63);
-    const GLB uint32_t *cols = glb(G.rec) + (tid() & 63);
-    double acc = 0.0;
-    run_slices<4>(
-        G, 0, [&](int r) { return 64 * r; }, [&](int e) { acc += (double)vals[e] * vec[cols[e]]; },
-        [&](uint32_t h, int lanes, int) {
-            const double s = group_sum(acc, lanes);
-            acc = 0.0;
-            if (h & HDR_VALID) out((int)(h & HDR_INDEX), s);
-        });
-}
+template <typename LUT>
+struct Stream {
+    struct Rec { LUT v; uint32_t c; };
+    Slices<Rec, 8> run;
+    const GLB LUT *vals;
+    const GLB uint32_t *cols;
+    __device__ __forceinline__ Rec load(int r) const { return Rec{vals[64 * r], cols[64 * r]}; }
+    __device__ __forceinline__ void list(const CST DevProg &G, const LUT *v)
+    {
+        vals = glb(v) + (tid() & 63);
+        cols = glb(G.rec) + (tid() & 63);
+        run.list(G);
+    }
+    __device__ __forceinline__ void first(const CST DevProg &G)
+    {
+        run.first(G, [&](int r) { return load(r); });
+    }
+    template <class Out>
+    __device__ __forceinline__ void finish(const CST DevProg &G, const LDS double *vec, Out out)
+    {
+        double acc = 0.0;
+        run.template run<4>(
+            G, [&](int r) { return load(r); }, [&](Rec q) { acc += (double)q.v * vec[q.c]; },
+            [&](uint32_t h, int lanes, int) {
+                const double s = group_sum(acc, lanes);
+                acc = 0.0;
+                if (h & HDR_VALID) out((int)(h & HDR_INDEX), s);
+            });
+    }
+};
 
 // M x = b from the stored streams: w (permuted right-hand side, at L.flux) -> x (two vectors
 // further).  Five products with a barrier after each.
@@ -2078,6 +2158,20 @@ __device__ __forceinline__ void staged_solve(NetRef N_, const Lds &L, const LUT 
     PhaseClock clk(L);
     const int npad = (N.nw_N + 7) & ~7, ns = N.sp_ns, T = N.sp_T;
     LDS double *w = L.flux, *v = w + npad, *x = v + npad;
+    // every phase's descriptors at once, its first operands ahead of the barrier before it
+    Stream<LUT> sT, sX, sL, sU;
+    sT.list(N.pg_solve[0], V + N.sp_at[0]);
+    sL.list(N.pg_solve[2], V + N.sp_at[2]);
+    sU.list(N.pg_solve[3], V + N.sp_at[3]);
+    sX.list(N.pg_solve[1], V + N.sp_at[1]);
+    sT.first(N.pg_solve[0]);
+    sL.first(N.pg_solve[2]);
+    constexpr int TAIL_AHEAD = 16;   // of the at most 32 columns a lane multiplies
+    const int t = tid(), h = t & 3, nst = (T + 3) >> 2, T1 = max(T - 1, 0);
+    const GLB LUT *S = glb(V + N.sp_nstream) + t;
+    LUT Sa[TAIL_AHEAD];
+#pragma unroll
+    for (int q = 0; q < TAIL_AHEAD; q++) Sa[q] = (q < nst && t < 4 * T) ? S[q * 4 * T] : (LUT)0;
     if (N.sp_presum) {   // sums of the replaced rows' right-hand sides
         if (wave_id() == 0) {
             const bool charge = L.prm[P_ENFORCECHARGE] != 0.0 && N.nelec < N.nspec;
@@ -2091,32 +2185,29 @@ __device__ __forceinline__ void staged_solve(NetRef N_, const Lds &L, const LUT 
         }
         __syncthreads();
     }
-    stream_phase<LUT>(N.pg_solve[0], V + N.sp_at[0], w, [&](int r, double s) { v[r] = w[r] - s; });
+    sT.finish(N.pg_solve[0], w, [&](int r, double s) { v[r] = w[r] - s; });
     __syncthreads();
-    stream_phase<LUT>(N.pg_solve[2], V + N.sp_at[2], w, [&](int r, double s) { v[r] = w[r] - s; });
+    sL.finish(N.pg_solve[2], w, [&](int r, double s) { v[r] = w[r] - s; });
+    sU.first(N.pg_solve[3]);
     __syncthreads();
     clk.mark(TM_SOL_SPARSE);
-    if (T > 0) {   // four lanes a row of the tail's inverse, each every fourth column
-        const int t = tid(), h = t & 3, nst = (T + 3) >> 2;
-        const GLB LUT *S = glb(V + N.sp_nstream) + t;
+    {   // four lanes a row of the tail's inverse, each every fourth column
         double p0 = 0.0, p1 = 0.0;
+#pragma unroll
+        for (int q = 0; q < TAIL_AHEAD; q++) p0 += (double)Sa[q] * v[ns + min(4 * q + h, T1)];
         if (t < 4 * T) {
-            int q = 0;
-#pragma unroll 4
-            for (; q + 2 <= nst - 1; q += 2) {
-                p0 += (double)S[q * 4 * T] * v[ns + 4 * q + h];
-                p1 += (double)S[(q + 1) * 4 * T] * v[ns + 4 * q + 4 + h];
-            }
-            for (; q < nst; q++) p0 += (double)S[q * 4 * T] * v[ns + min(4 * q + h, T - 1)];
+#pragma unroll 8
+            for (int q = TAIL_AHEAD; q < nst; q++) p1 += (double)S[q * 4 * T] * v[ns + min(4 * q + h, T1)];
         }
         const double s = group_sum(p0 + p1, 4);
         if (t < 4 * T && h == 0) x[ns + (t >> 2)] = s;
     }
     __syncthreads();
     clk.mark(TM_SOL_TAIL);
-    stream_phase<LUT>(N.pg_solve[3], V + N.sp_at[3], w, [&](int r, double s) { w[r] = v[r] - s; });
+    sX.first(N.pg_solve[1]);
+    sU.finish(N.pg_solve[3], w, [&](int r, double s) { w[r] = v[r] - s; });
     __syncthreads();
-    stream_phase<LUT>(N.pg_solve[1], V + N.sp_at[1], w, [&](int r, double s) { x[r] = s; });
+    sX.finish(N.pg_solve[1], w, [&](int r, double s) { x[r] = s; });
     __syncthreads();
     clk.mark(TM_SOL_SPARSE);
 }
