@@ -307,7 +307,8 @@ SlotLayout slot_layout(const ucg::DevNet &N, bool sparse, int lu_bits)
     if (sparse && N.nw_stage) {
         // a staged plan's factors and waiting tail entries need less; the slot keeps that size, so
         // that a budget or the fixed workspace holds the same number of slots either way
-        s.mat = al(((size_t)N.sp_nstream + ucg::tail_len(N.sp_T)) * elem);
+        s.mat = N.nw_stage == 2 ? al((size_t)N.sp_nstream * elem) + al((size_t)N.sp_T * N.sp_T * sizeof(double))
+                                : al(((size_t)N.sp_nstream + ucg::tail_len(N.sp_T)) * elem);
         s.jac = al((size_t)(N.sp_end_hdr - N.sp_tail_hdr) * sizeof(double));
         both = std::max(both, s.mat + s.jac);
         s.jac = both - s.mat;
@@ -764,21 +765,26 @@ static int load_staged_plan(const ucg_network_desc *d, NetHandle &h, size_t lds_
     N.sp_end_hdr = S.end_hdr;
     N.sp_slots = S.n_slots;
     for (int k = 0; k < 4; k++) N.sp_at[k] = S.at[k];
-    N.sp_w0 = std::max(N.px.n, S.t * S.t - S.at_L);   // the tail must end before L21
+    // the tail, or a panel of a wide one, must end before L21; a wide tail's slots may take the
+    // operands' place (their values wait)
+    N.sp_w0 = S.wide ? std::max(0, ucg::WIDE_COLS * ucg::WIDE_LD - S.at_L) : std::max(N.px.n, S.t * S.t - S.at_L);
+    N.sp_panels = (int)S.schur.size();
+    if (N.sp_panels > ucg::WIDE_PANELS) return 0;
     N.sp_presum = S.presum ? 1 : 0;
-    N.nw_stage = 1;
+    N.nw_stage = S.wide ? 2 : 1;
     if (lds_bytes(N) > lds_limit) {
         N.nw_stage = 0;
         return 0;
     }
     int rc;
     if ((rc = upload(h, S.stream.data(), S.stream.size(), N.sp_stream)) ||
-        (rc = upload(h, S.tail_wave.data(), S.tail_wave.size(), N.sp_tail_wave)) ||
+        (rc = upload(h, S.part_wave.data(), S.part_wave.size(), N.sp_part_wave)) ||
         (rc = upload(h, S.sum_rows.data(), S.sum_rows.size(), N.sp_sum_rows)) ||
         (rc = upload(h, S.sum_members.data(), S.sum_members.size(), N.sp_sum_members)) ||
-        (rc = upload_program(h, S.entries, N.pg_entries)) || (rc = upload_program(h, S.elim, N.pg_elim)) ||
-        (rc = upload_program(h, S.schur, N.pg_schur)))
+        (rc = upload_program(h, S.entries, N.pg_entries)) || (rc = upload_program(h, S.elim, N.pg_elim)))
         return rc;
+    for (int k = 0; k < N.sp_panels; k++)
+        if ((rc = upload_program(h, S.schur[k], N.pg_schur[k]))) return rc;
     for (int k = 0; k < 4; k++)
         if ((rc = upload_program(h, S.solve[k], N.pg_solve[k]))) return rc;
     return 0;

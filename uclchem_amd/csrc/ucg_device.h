@@ -135,12 +135,14 @@ struct DevNet {
     // Newton matrix of a staged plan: operand slots, entries, elimination, Schur update, solves
     PartialSlots px;
     int32_t sp_ns, sp_T, sp_nstream, sp_L, sp_slots, sp_at[4], sp_w0, sp_presum;
-    int32_t sp_tail_hdr, sp_end_hdr;   // headers of the tail entries, whose values wait in the workspace
-    const int32_t *sp_tail_wave;       // [NWAVE + 1] the waves' shares of them
+    int32_t sp_tail_hdr, sp_end_hdr;   // headers of the entries whose values wait in the workspace
+    const int32_t *sp_part_wave;       // [entry parts][NWAVE + 1] the waves' shares of the headers
     const uint32_t *sp_stream;
     const int32_t *sp_sum_rows, *sp_sum_members;
-    DevProg pg_entries, pg_elim, pg_schur, pg_solve[4];
-    int32_t nw_stage;            // 1: the plan runs from LDS and matrix-core registers; 0: from the workspace
+    int32_t sp_panels;           // of a wide tail; else 1
+    DevProg pg_entries, pg_elim, pg_schur[WIDE_PANELS], pg_solve[4];
+    int32_t nw_stage;            // 1: the plan runs from LDS and matrix-core registers; 2: so, with a wide
+                                 // tail; 0: from the workspace
     const int32_t *nw_perm, *nw_inv, *nw_sp_ptr, *nw_sp_col, *nw_sp_dpos, *nw_lev_ptr, *nw_lev_rows, *nw_ph_ptr;
     const int32_t *nw_tg_slot, *nw_tg_ptr, *nw_tg_div, *nw_pr_l, *nw_pr_u, *nw_jnz_slot, *nw_diag_slot;
     const int32_t *nw_ph_slot, *nw_tr_slot, *nw_s1c, *nw_s1r, *nw_s2c, *nw_s2r, *nw_gs_ptr, *nw_gs_slot;
@@ -178,7 +180,11 @@ __host__ __device__ inline int flux_region_len(const Net &N)
     const int b1 = b0 > 3 * Npad ? b0 : 3 * Npad;
     const int b = b1 > NT ? b1 : NT;                 // >= one value per thread (ordered_sum)
     if (!N.nw_stage) return b;
-    const int c = N.sp_w0 + N.sp_slots;
+    const int c = N.sp_w0 + N.sp_slots > N.px.n ? N.sp_w0 + N.sp_slots : N.px.n;
+    if (N.nw_stage == 2) {   // working slots behind a panel, or one block as a matrix operand
+        const int m = WIDE_ROWS * WIDE_LD, e = c > m ? c : m;
+        return b > e ? b : e;
+    }
     const int gj = (2 * ((N.sp_T + 15) / 16 + 1) + 1) * 16 * 17, tt = N.sp_T * N.sp_T;
     const int e0 = c > gj ? c : gj;
     const int e = e0 > tt ? e0 : tt;

@@ -192,7 +192,8 @@ inline PartialSlots partial_slots(int npart, int nsx, int nswap, int nsurfl)
     return p;
 }
 
-// Entry headers: target in bits 0..22 (a working slot, or a tail element when ENTRY_TAIL), flags.
+// Entry headers: target in bits 0..22 (a working slot, or a place in the tail or its panel), flags
+// (ENTRY_TAIL: the value waits in the workspace).
 enum : uint32_t { ENTRY_TARGET = 0x7fffffu, ENTRY_TAIL = 1u << 23, ENTRY_UNSCALED = 1u << 24, ENTRY_ONE = 1u << 25,
                   ENTRY_MINUS = 1u << 26, ENTRY_CHARGE = 1u << 27, ENTRY_CHARGE_ONE = 1u << 28,
                   ENTRY_CHARGE_MINUS = 1u << 29, ENTRY_VALID = 1u << 31 };
@@ -211,12 +212,15 @@ struct SparsePrograms {
     int at_L = 0, zero = 0, n_slots = 0, tail_hdr = 0, end_hdr = 0;
     int at[4] = {0, 0, 0, 0};
     std::vector<uint32_t> stream;
-    std::vector<int> tail_wave;       // [nwave + 1] first tail-entry header of each wave
+    std::vector<int> part_wave;       // [entry parts][nwave + 1] first header of each wave
     bool presum = false;              // the sum rows are not all tail rows: subtract sums up front
     std::vector<int> sum_rows;        // presum: {row, first, end} of the permuted members
     std::vector<int> sum_members;
-    Program elim, schur, entries, solve[4];   // solve: T, X, L21, U12
-    bool ok = false;
+    Program elim, entries, solve[4];   // solve: T, X, L21, U12
+    // the tail's Schur update: one program, or with a wide tail one for each panel of 128 rows (x) 64
+    // columns that is formed in LDS at a time
+    std::vector<Program> schur;
+    bool wide = false, ok = false;
 };
 
 struct EntryItem {
@@ -224,18 +228,32 @@ struct EntryItem {
     std::vector<std::pair<int, int>> c;   // (partial, coefficient)
 };
 
+// A wide tail (more rows than the waves hold as block columns) is inverted as 2 x 2 blocks, the
+// first of WIDE_ROWS rows, and formed panel by panel: (row half, 64 columns), in columns of
+// WIDE_LD doubles in LDS.
+constexpr int WIDE_ROWS = 128, WIDE_COLS = 64, WIDE_LD = 130, WIDE_PANELS = 8;
+
 // One network's tables as the planner reads them (the fields of ucg_network_desc it needs).
 template <class Desc>
 SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, const std::vector<int> &fac_off, int npart)
 {
     SparsePrograms S;
     const int neq = d->neq, NN = d->nw_sizes[0], ns0 = d->nw_sizes[1], T0 = d->nw_sizes[2], nsp0 = d->nw_sizes[3];
-    if (T0 > max_tail) return S;
+    if (T0 > 2 * max_tail) return S;
+    S.wide = T0 > max_tail;
+    if (S.wide) max_tail *= 2;
     // the tail fills whole 16-row blocks: the rows up to the next block cost its inversion nothing
     // and leave the sparse pivots with fewer levels
     const int T = std::min(std::min((T0 + 15) / 16 * 16, max_tail), NN), ns = NN - T;
     S.ns = ns;
     S.t = T;
+    if (S.wide && T % 16 != 0) return S;
+    // tail element -> panel and place in it
+    const int halves = S.wide ? 2 : 1, cols = S.wide ? (T + WIDE_COLS - 1) / WIDE_COLS : 1, panels = halves * cols;
+    auto panel_of = [&](int r, int c) { return S.wide ? ((c - ns) / WIDE_COLS) * halves + (r - ns) / WIDE_ROWS : 0; };
+    auto place_of = [&](int r, int c) {
+        return S.wide ? ((c - ns) % WIDE_COLS) * WIDE_LD + (r - ns) % WIDE_ROWS : (c - ns) * T + (r - ns);
+    };
     // filled pattern
     std::vector<std::vector<int>> Lrow(NN), Urow(ns), Ucol(NN);   // L(r, c < r), U(r, c >= r), sparse pivots only
     auto pivot_row = [&](int r, int c) {
@@ -443,32 +461,33 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
         S.stream.push_back(sl < 0 ? ((unsigned)ZERO | NO_SLOT << 16) : ((unsigned)sl | scale[sl] << 16));
     // Schur complement of the tail
     {
-        std::vector<std::vector<std::array<int, 2>>> it;
-        std::vector<int> where, len;
         std::vector<std::vector<int>> ucols(ns);
         for (int r = 0; r < ns; r++)
             for (int c : Urow[r])
                 if (c >= ns) ucols[r].push_back(c);
-        std::map<std::pair<int, int>, int> idx;
+        std::vector<std::map<std::pair<int, int>, std::vector<std::array<int, 2>>>> by(panels);
         for (int r = ns; r < NN; r++)
             for (int p : Lrow[r])
-                for (int c : ucols[p]) {
-                    auto f = idx.emplace(std::make_pair(r, c), (int)it.size());
-                    if (f.second) {
-                        it.emplace_back();
-                        where.push_back((c - ns) * T + (r - ns));
-                    }
-                    it[f.first->second].push_back({slotL.at({r, p}), slotU.at({p, c})});
-                }
-        for (auto &x : it) len.push_back((int)x.size());
-        const SliceSet P = pack_slices(len, nwave);
-        S.schur.add(
-            P, nwave, 1, 2, 2, [&](int i, uint32_t *h) { h[0] = i >= 0 ? (HDR_VALID | (uint32_t)where[i]) : 0u; },
-            [&](int i, int e, int k, uint32_t *w) {
-                put16(w, 2 * k, e >= 0 ? it[i][e][0] : ZERO);
-                put16(w, 2 * k + 1, e >= 0 ? it[i][e][1] : ZERO);
-            },
-            len);
+                for (int c : ucols[p]) by[panel_of(r, c)][{r, c}].push_back({slotL.at({r, p}), slotU.at({p, c})});
+        for (auto &m : by) {
+            std::vector<const std::vector<std::array<int, 2>> *> it;
+            std::vector<int> where, len;
+            for (auto &kv : m) {
+                it.push_back(&kv.second);
+                where.push_back(place_of(kv.first.first, kv.first.second));
+                len.push_back((int)kv.second.size());
+            }
+            const SliceSet P = pack_slices(len, nwave);
+            S.schur.emplace_back();
+            S.schur.back().add(
+                P, nwave, 1, 2, 2, [&](int i, uint32_t *h) { h[0] = i >= 0 ? (HDR_VALID | (uint32_t)where[i]) : 0u; },
+                [&](int i, int e, int k, uint32_t *w) {
+                    put16(w, 2 * k, e >= 0 ? (*it[i])[e][0] : ZERO);
+                    put16(w, 2 * k + 1, e >= 0 ? (*it[i])[e][1] : ZERO);
+                },
+                len);
+            S.schur.back().finish(nwave, true);
+        }
     }
     // ---------------- entries of M = I - gamma J (augmented), by place
     std::vector<std::pair<int, int>> place(nsp0 + T0 * T0);   // plan slot -> (row, column)
@@ -584,14 +603,16 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
         for (int q = 0; q < d->nion; q++) E(d->nw_eion[q]).flags |= ENTRY_CHARGE | ENTRY_CHARGE_MINUS;
         if (d->nw_diag_slot[NE] >= 0) E(d->nw_diag_slot[NE]).flags |= ENTRY_CHARGE | ENTRY_CHARGE_ONE;
     }
-    // items: working slots (with the constant slots of the streams), then tail elements
+    // items: working slots (with the constant slots of the streams), then the panels of the tail.
+    // Values whose place the operands still occupy wait in the workspace (ENTRY_TAIL).
     std::vector<uint32_t> head;
     std::vector<std::vector<unsigned>> op;
     std::vector<int> len;
-    for (int part = 0; part < 2; part++) {
+    for (int part = 0; part < 1 + panels; part++) {
         head.clear();
         op.clear();
         len.clear();
+        const uint32_t waits = part > 0 || S.wide ? ENTRY_TAIL : 0u;
         auto item = [&](uint32_t h, const std::vector<std::pair<int, int>> &c) {
             std::map<int, int> merged;
             for (auto &x : c) merged[x.first] += x.second;
@@ -605,30 +626,26 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
         for (auto &kv : ent) {
             const int r = kv.first.first, c = kv.first.second;
             const bool tail = r >= ns && c >= ns;
-            if (tail != (part == 1)) continue;
-            const int target = tail ? (c - ns) * T + (r - ns) : c < r ? slotL.at({r, c}) : Us(r, c);
-            item(ENTRY_VALID | kv.second.flags | (tail ? ENTRY_TAIL : 0u) | (uint32_t)target, kv.second.c);
+            if ((tail ? 1 + panel_of(r, c) : 0) != part) continue;
+            const int target = tail ? place_of(r, c) : c < r ? slotL.at({r, c}) : Us(r, c);
+            item(ENTRY_VALID | kv.second.flags | waits | (uint32_t)target, kv.second.c);
         }
         if (part == 0) {
             const std::vector<std::pair<int, int>> none;
-            item(ENTRY_VALID | ENTRY_ONE | (uint32_t)ONE, none);
-            item(ENTRY_VALID | ENTRY_MINUS | (uint32_t)MONE, none);
-            for (int sl : one_slots) item(ENTRY_VALID | ENTRY_ONE | (uint32_t)sl, none);
-            for (int sl : charge_slots) item(ENTRY_VALID | ENTRY_CHARGE | ENTRY_CHARGE_ONE | (uint32_t)sl, none);
+            item(ENTRY_VALID | waits | ENTRY_ONE | (uint32_t)ONE, none);
+            item(ENTRY_VALID | waits | ENTRY_MINUS | (uint32_t)MONE, none);
+            for (int sl : one_slots) item(ENTRY_VALID | waits | ENTRY_ONE | (uint32_t)sl, none);
+            for (int sl : charge_slots) item(ENTRY_VALID | waits | ENTRY_CHARGE | ENTRY_CHARGE_ONE | (uint32_t)sl, none);
         }
         const SliceSet P = pack_slices(len, nwave);
-        S.tail_hdr = (int)S.entries.hdr.size();   // after the last part: the tail's first header
+        if (part == (S.wide ? 0 : 1)) S.tail_hdr = (int)S.entries.hdr.size();   // the first that waits
+        for (int w = 0; w <= nwave; w++) S.part_wave.push_back((int)S.entries.hdr.size() + 64 * P.wave_ptr[w]);
         S.entries.add(
             P, nwave, 1, 2, 4, [&](int i, uint32_t *h) { h[0] = i >= 0 ? head[i] : 0u; },
             [&](int i, int e, int k, uint32_t *w) { put16(w, k, e >= 0 ? op[i][e] : (unsigned)ps.zero); }, len);
     }
     S.end_hdr = (int)S.entries.hdr.size();
-    for (int w = 0; w <= nwave; w++) {   // the waves' tail headers: contiguous, one row of 64 a slice
-        const int s = S.entries.wave_ptr[nwave + 1 + w];
-        S.tail_wave.push_back(4 * (size_t)s < S.entries.slices.size() ? S.entries.slices[4 * s + 3] : S.end_hdr);
-    }
     S.elim.finish(nwave);
-    S.schur.finish(nwave, true);
     S.entries.finish(nwave, true);
     for (Program &P : S.solve) P.finish(nwave, true);
     S.ok = ps.n < 0x8000;

@@ -1313,27 +1313,22 @@ template <int K> __device__ __forceinline__ void gj16_steps(f64x4 &d, int g, int
     }
 }
 
-// A: n x n, column-major, leading dimension n, in LDS.  The inverse goes to `out` in blocks of four
-// columns, row-major inside a block (tail_index), the order in which the solve's lanes read it.
-// `stage`: LDS scratch of gj_stage_len(n) doubles, which may be A's own.  Returns nonzero (uniformly) on a zero
-// or non-finite pivot.
+// The place of an element in a stored block of n rows: blocks of four columns, row-major inside a
+// block, the order in which the solve's lanes read it.
 __device__ __forceinline__ int tail_index(int n, int row, int col) { return (col >> 2) * 4 * n + 4 * row + (col & 3); }
 __host__ __device__ inline int tail_len(int n) { return ((n + 3) & ~3) * n; }
-template <typename LUT>
-__device__ __forceinline__ int block_gj_inverse(const LDS double *A, int n, LDS double *red, LDS double *stage, LUT *out)
+
+// by-value select, as bdf::sel: keeps the tiles out of scratch memory
+__device__ __forceinline__ f64x4 sel_tile(bool c, f64x4 a, f64x4 b) { return c ? a : b; }
+
+// Inverts the nb x nb blocks the waves hold (t[I]: block row I of block column w).  `stage`: LDS
+// scratch of gj_stage_len doubles.  Called by every wave; returns nonzero (uniformly) on a zero or
+// non-finite pivot.
+__device__ __forceinline__ int gj_sweeps(f64x4 (&t)[NWAVE], int nb, LDS double *red, LDS double *stage)
 {
-    const int w = __builtin_amdgcn_readfirstlane(tid() >> 6), lane = tid() & 63, g = lane >> 4, c = lane & 15;
-    const int nb = (n + 15) >> 4, gen = (nb + 1) * GJ_TILE;
-    const int col = 16 * w + c;
-    f64x4 t[NWAVE];
+    const int w = wave_id(), lane = tid() & 63, g = lane >> 4, c = lane & 15;
+    const int gen = (nb + 1) * GJ_TILE;
     if (tid() == 0) red[8] = 0.0;
-#pragma unroll
-    for (int I = 0; I < NWAVE; I++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int row = 16 * I + 4 * i + g;
-            t[I][i] = (row < n && col < n) ? A[col * n + row] : (row == col ? 1.0 : 0.0);
-        }
     __syncthreads();
     // the pivot blocks are inverted by a wave without a column while the others update theirs; with
     // eight columns by the block's owner
@@ -1352,8 +1347,7 @@ __device__ __forceinline__ int block_gj_inverse(const LDS double *A, int n, LDS 
             } else if (w < nb) {
                 f64x4 b = t[0];
 #pragma unroll
-                for (int I = 1; I < NWAVE; I++)
-                    if (I == K) b = t[I];
+                for (int I = 1; I < NWAVE; I++) b = sel_tile(I == K, t[I], b);
 #pragma unroll
                 for (int s = 0; s < 4; s++)
                     P = __builtin_amdgcn_mfma_f64_16x16x4f64(inv[17 * (4 * s + g) + c], b[s], P, 0, 0, 0);
@@ -1362,8 +1356,7 @@ __device__ __forceinline__ int block_gj_inverse(const LDS double *A, int n, LDS 
         if (next) {   // the next pivot block first
             f64x4 m = t[0];
 #pragma unroll
-            for (int I = 1; I < NWAVE; I++)
-                if (I == w) m = t[I];
+            for (int I = 1; I < NWAVE; I++) m = sel_tile(I == w, t[I], m);
             if (K >= 0) {
                 const LDS double *pw = panel + w * GJ_TILE;
 #pragma unroll
@@ -1406,6 +1399,29 @@ __device__ __forceinline__ int block_gj_inverse(const LDS double *A, int n, LDS 
                 }
         }
     }
+    return 0;
+}
+
+// A: n x n, column-major, leading dimension n, in LDS; its inverse goes to `out` (tail_index).
+// `stage` may be A's own place.
+template <typename LUT>
+PHASE int block_gj_inverse(LDS double *A, int n, LDS double *red, LDS double *stage, LUT *out)
+{
+    A = uniform_ptr(A);
+    n = __builtin_amdgcn_readfirstlane(n);
+    red = uniform_ptr(red);
+    stage = uniform_ptr(stage);
+    out = uniform_ptr(out);
+    const int w = wave_id(), lane = tid() & 63, g = lane >> 4, c = lane & 15, col = 16 * w + c;
+    f64x4 t[NWAVE];
+#pragma unroll
+    for (int I = 0; I < NWAVE; I++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int row = 16 * I + 4 * i + g;
+            t[I][i] = (row < n && col < n) ? A[col * n + row] : (row == col ? 1.0 : 0.0);
+        }
+    if (gj_sweeps(t, (n + 15) >> 4, red, stage)) return 1;
     GLB LUT *og = glbw(out);
 #pragma unroll
     for (int I = 0; I < NWAVE; I++)
@@ -1414,6 +1430,115 @@ __device__ __forceinline__ int block_gj_inverse(const LDS double *A, int n, LDS 
             const int row = 16 * I + 4 * i + g;
             if (row < n && col < ((n + 3) & ~3)) og[tail_index(n, row, col)] = (LUT)(col < n ? t[I][i] : 0.0);
         }
+    __syncthreads();
+    return 0;
+}
+
+// ---------------------------------------------------------------- wide tails
+// A tail of more rows than the waves hold as block columns (up to 256) is factored as 2 x 2 blocks
+// with the first n1 = 128 rows: I11 = inv(A11), B = I11 A12, S = A22 - A21 B, I22 = inv(S).  A solve
+// then is x1 = I11 b1, x2 = I22 (b2 - A21 x1), x1 -= B x2: the same reads as the full inverse, which
+// would cost four more block products.  500/6000 network (252 rows), FP64: 1270 us a set-up and 109
+// a solve with the blocked LU and triangular sweeps in the workspace, 260 and 14 like this (a step
+// 494 -> 112 us); 40 % of a set-up is the Schur update's LDS gathers, as much the two inversions.
+// The blocks come from the workspace as tiles in the
+// accumulator layout (one 32-byte store a lane and tile); products take their left factor from LDS
+// and their right factor from the waves' registers.
+struct WideBlocks {
+    int n1, n2;
+    __device__ __forceinline__ explicit WideBlocks(int T) : n1(WIDE_ROWS), n2(T - WIDE_ROWS) {}
+    // offsets (doubles) of blocks 11, 21, 12, 22 in the tail's workspace
+    __device__ __forceinline__ int at(int rh, int ch) const { return ch ? (n1 + n2) * n1 + (rh ? n1 * n2 : 0) : (rh ? n1 * n1 : 0); }
+};
+__device__ __forceinline__ void load_tiles(const double *A, int nbr, int col, f64x4 (&t)[NWAVE])
+{   // block column `col` of a block of nbr block rows
+    const GLB f64x4 *p = (const GLB f64x4 *)glb(A) + (size_t)col * nbr * 64 + (tid() & 63);
+#pragma unroll
+    for (int I = 0; I < NWAVE; I++) t[I] = I < nbr ? p[I * 64] : f64x4{0.0, 0.0, 0.0, 0.0};
+}
+template <typename LUT>
+__device__ __forceinline__ void store_block(LUT *A, int nbr, int col, const f64x4 (&t)[NWAVE])
+{
+    const int lane = tid() & 63, g = lane >> 4, c = lane & 15;
+    GLB LUT *o = glbw(A);
+#pragma unroll
+    for (int I = 0; I < NWAVE; I++)
+        if (I < nbr) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) o[tail_index(16 * nbr, 16 * I + 4 * i + g, 16 * col + c)] = (LUT)t[I][i];
+        }
+}
+// this wave's block column as columns of the LDS matrix operand M
+__device__ __forceinline__ void operand_column(LDS double *M, int nbr, int col, const f64x4 (&t)[NWAVE], double sign)
+{
+    const int lane = tid() & 63, g = lane >> 4, c = lane & 15;
+#pragma unroll
+    for (int I = 0; I < NWAVE; I++)
+        if (I < nbr) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) M[(16 * col + c) * WIDE_LD + 16 * I + 4 * i + g] = sign * t[I][i];
+        }
+}
+// acc += M R for this wave's block column R (nbk block rows), M of nbr block rows in LDS
+__device__ __forceinline__ void block_product(const LDS double *M, int nbr, int nbk, const f64x4 (&R)[NWAVE],
+                                              f64x4 (&acc)[NWAVE])
+{
+    const int lane = tid() & 63, g = lane >> 4, c = lane & 15;
+#pragma unroll
+    for (int kb = 0; kb < NWAVE; kb++)
+        if (kb < nbk) {
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const LDS double *m = M + (16 * kb + 4 * s + g) * WIDE_LD + c;
+#pragma unroll
+                for (int I = 0; I < NWAVE; I++)
+                    if (I < nbr) acc[I] = __builtin_amdgcn_mfma_f64_16x16x4f64(m[16 * I], R[kb][s], acc[I], 0, 0, 0);
+            }
+        }
+}
+// The blocks are factored in place: every load of a block has returned before the barrier after
+// which another wave may store to it.
+__device__ __forceinline__ void loads_returned() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+template <typename LUT>
+PHASE int wide_tail(const DevNet *Np, Lds L_, double *tail)
+{
+    const Lds L = uniform_lds(L_);
+    NetRef N = *(const CST DevNet *)uniform_ptr(Np);
+    tail = uniform_ptr(tail);
+    const int w = wave_id();
+    const WideBlocks B(N.sp_T);
+    const int nb1 = B.n1 / 16, nb2 = B.n2 / 16;
+    LDS double *M = L.flux;
+    f64x4 t[NWAVE], r[NWAVE];
+    load_tiles(tail + B.at(0, 0), nb1, w, t);
+    if (gj_sweeps(t, nb1, L.red, M)) return 1;
+    __syncthreads();                                    // exchange buffers and A11 are done with
+    operand_column(M, nb1, w, t, 1.0);
+    store_block<LUT>((LUT *)(tail + B.at(0, 0)), nb1, w, t);
+    if (w < nb2) load_tiles(tail + B.at(0, 1), nb1, w, r);
+#pragma unroll
+    for (int I = 0; I < NWAVE; I++) t[I] = f64x4{0.0, 0.0, 0.0, 0.0};
+    loads_returned();
+    __syncthreads();
+    if (w < nb2) {                                      // B = I11 A12
+        block_product(M, nb1, nb1, r, t);
+        store_block<LUT>((LUT *)(tail + B.at(0, 1)), nb1, w, t);
+    }
+    load_tiles(tail + B.at(1, 0), nb2, w, r);
+    loads_returned();
+    __syncthreads();                                    // M and A21's tiles are read
+    operand_column(M, nb2, w, r, -1.0);
+    store_block<LUT>((LUT *)(tail + B.at(1, 0)), nb2, w, r);
+    if (w < nb2) load_tiles(tail + B.at(1, 1), nb2, w, r);
+    __syncthreads();
+    if (w < nb2) block_product(M, nb2, nb1, t, r);      // S = A22 - A21 B
+    else {
+#pragma unroll
+        for (int I = 0; I < NWAVE; I++) r[I] = f64x4{0.0, 0.0, 0.0, 0.0};
+    }
+    __syncthreads();
+    if (gj_sweeps(r, nb2, L.red, M)) return 1;
+    if (w < nb2) store_block<LUT>((LUT *)(tail + B.at(1, 1)), nb2, w, r);
     __syncthreads();
     return 0;
 }
@@ -2038,7 +2163,7 @@ __device__ __forceinline__ void eliminate(NetRef N, Slices<uint2, 2> &run, LDS d
 }
 
 template <typename LUT>
-__device__ __forceinline__ int staged_setup(NetRef N_, const Lds &L, LUT *V, double *stage, double gamma)
+__device__ __forceinline__ int staged_setup(const DevNet *Np, NetRef N_, const Lds &L, LUT *V, double *stage, double gamma)
 {
     NetRef N = fresh(N_);
     PhaseClock clk(L);
@@ -2046,7 +2171,22 @@ __device__ __forceinline__ int staged_setup(NetRef N_, const Lds &L, LUT *V, dou
     const bool charge = L.prm[P_ENFORCECHARGE] != 0.0 && N.nelec < N.nspec;
     LDS double *P = L.flux, *W = L.flux + N.sp_w0, *tl = L.flux, *red = L.red;
     if (tid() == 0) red[9] = 0.0;
-    for (int q = tid(); q < N.sp_slots; q += NT) W[q] = 0.0;
+    const bool wide = N.nw_stage == 2;
+    // a part's waiting values, by the lanes that computed them
+    const auto fetch_part = [&](int part, LDS double *to) {
+        const GLB uint32_t *hdr = glb(N.pg_entries.hdr);
+        const GLB double *st = glb((const double *)stage) - N.sp_tail_hdr;
+        const GLB int *pw = glb(N.sp_part_wave) + part * (NWAVE + 1) + w;
+        const int h1 = pw[1];
+#pragma unroll 4
+        for (int h0 = pw[0] + lane; h0 < h1; h0 += 64) {
+            const uint32_t h = hdr[h0];
+            const double v = st[h0];
+            if (h & ENTRY_VALID) to[h & ENTRY_TARGET] = v;
+        }
+    };
+    if (!wide)
+        for (int q = tid(); q < N.sp_slots; q += NT) W[q] = 0.0;
     const auto rec_of = [&](const CST DevProg &G) {
         return [rec = glb(G.rec) + 2 * lane](int r) { return ld_uint2(rec, 64 * r); };
     };
@@ -2060,6 +2200,12 @@ __device__ __forceinline__ int staged_setup(NetRef N_, const Lds &L, LUT *V, dou
     newton_entries(N, entries, P, W, stage, gamma, charge);
     pivots.first(N.pg_elim, rec_of(N.pg_elim));
     __syncthreads();
+    if (wide) {   // the slots take the operands' place
+        for (int q = tid(); q < N.sp_slots; q += NT) W[q] = 0.0;
+        __syncthreads();
+        fetch_part(0, W);
+        __syncthreads();
+    }
     clk.mark(TM_JAC);
     PhaseClock lu(L);
     eliminate(N, pivots, W, red);
@@ -2078,27 +2224,19 @@ __device__ __forceinline__ int staged_setup(NetRef N_, const Lds &L, LUT *V, dou
             out[q] = (LUT)v;
         }
     }
-    schur.list(N.pg_schur);
-    __syncthreads();
-    for (int q = tid(); q < T * T; q += NT) tl[q] = 0.0;
-    __syncthreads();
-    {   // this lane's tail entries
-        const GLB uint32_t *hdr = glb(N.pg_entries.hdr);
-        const GLB double *st = glb((const double *)stage) - N.sp_tail_hdr;
-        const int h1 = glb(N.sp_tail_wave)[w + 1];
-#pragma unroll 4
-        for (int h0 = glb(N.sp_tail_wave)[w] + lane; h0 < h1; h0 += 64) {
-            const uint32_t h = hdr[h0];
-            const double v = st[h0];
-            if (h & ENTRY_VALID) tl[h & ENTRY_TARGET] = v;
-        }
-    }
-    schur.first(N.pg_schur, rec_of(N.pg_schur));
-    __syncthreads();
-    {   // Schur complement
+    double *tail = (double *)((char *)V + (((size_t)N.sp_nstream * sizeof(LUT) + 255) & ~(size_t)255));   // wide
+    for (int p = 0; p < N.sp_panels; p++) {
+        const int len = wide ? WIDE_COLS * WIDE_LD : T * T;
+        schur.list(N.pg_schur[p]);
+        __syncthreads();
+        for (int q = tid(); q < len; q += NT) tl[q] = 0.0;
+        __syncthreads();
+        fetch_part(1 + p, tl);
+        schur.first(N.pg_schur[p], rec_of(N.pg_schur[p]));
+        __syncthreads();
         double a0 = 0.0, a1 = 0.0;
         schur.run<4>(
-            N.pg_schur, rec_of(N.pg_schur),
+            N.pg_schur[p], rec_of(N.pg_schur[p]),
             [&](uint2 q) {
                 a0 += W[q.x & 0xffff] * W[q.x >> 16];
                 a1 += W[q.y & 0xffff] * W[q.y >> 16];
@@ -2108,10 +2246,31 @@ __device__ __forceinline__ int staged_setup(NetRef N_, const Lds &L, LUT *V, dou
                 a0 = a1 = 0.0;
                 if (h & HDR_VALID) tl[h & HDR_INDEX] -= acc;
             });
+        __syncthreads();
+        if (wide) {   // this panel's tiles to the workspace (stores complete before wide_tail's barrier): half of a wave's four block columns each
+            const WideBlocks B(T);
+            const int rh = p & 1, cb = 4 * (p >> 1) + (w & 3), ch = cb >= WIDE_ROWS / 16, nbr = (rh ? B.n2 : B.n1) / 16;
+            if (16 * cb < T) {
+                const int g = lane >> 4, c = lane & 15;
+                GLB f64x4 *o = (GLB f64x4 *)glbw(tail + B.at(rh, ch)) + (size_t)(cb - ch * (WIDE_ROWS / 16)) * nbr * 64 + lane;
+                for (int I = w >> 2; I < nbr; I += 2) {
+                    f64x4 v;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) v[i] = tl[(16 * (w & 3) + c) * WIDE_LD + 16 * I + 4 * i + g];
+                    o[I * 64] = v;
+                }
+            }
+        }
     }
-    __syncthreads();
     clk.mark(TM_LU_SPARSE);
-    const int r = T > 0 ? block_gj_inverse<LUT>(tl, T, red, L.flux, V + N.sp_nstream) : 0;
+    int r = 0;
+    if (wide) {
+        loads_returned();   // and stores
+        __syncthreads();
+        r = __builtin_amdgcn_readfirstlane(wide_tail<LUT>(Np, L, tail));
+    } else if (T > 0) {
+        r = __builtin_amdgcn_readfirstlane(block_gj_inverse<LUT>(tl, T, red, L.flux, V + N.sp_nstream));
+    }
     clk.mark(TM_LU_TAIL);
     lu.mark(TM_LU);
     return r;
@@ -2167,7 +2326,7 @@ __device__ __forceinline__ void staged_solve(NetRef N_, const Lds &L, const LUT 
     sT.first(N.pg_solve[0]);
     sL.first(N.pg_solve[2]);
     constexpr int TAIL_AHEAD = 16;   // of the at most 32 columns a lane multiplies
-    const int t = tid(), h = t & 3, nst = (T + 3) >> 2, T1 = max(T - 1, 0);
+    const int t = tid(), h = t & 3, nst = N.nw_stage == 2 ? 0 : (T + 3) >> 2, T1 = max(T - 1, 0);
     const GLB LUT *S = glb(V + N.sp_nstream) + t;
     LUT Sa[TAIL_AHEAD];
 #pragma unroll
@@ -2191,6 +2350,31 @@ __device__ __forceinline__ void staged_solve(NetRef N_, const Lds &L, const LUT 
     sU.first(N.pg_solve[3]);
     __syncthreads();
     clk.mark(TM_SOL_SPARSE);
+    if (N.nw_stage == 2) {
+        const WideBlocks B(T);
+        const double *tail = (const double *)((const char *)V + (((size_t)N.sp_nstream * sizeof(LUT) + 255) & ~(size_t)255));
+        LDS double *v1 = v + ns, *v2 = v1 + B.n1, *x1 = x + ns, *x2 = x1 + B.n1;
+        // four lanes a row, each every fourth column: out(row, row of the block times vec)
+        const auto apply = [&](int rh, int ch, const LDS double *vec, auto out) {
+            const int rows = rh ? B.n2 : B.n1, nc = (ch ? B.n2 : B.n1) >> 2, t = tid(), h = t & 3;
+            const GLB LUT *A = glb((const LUT *)(tail + B.at(rh, ch))) + t;
+            double p0 = 0.0, p1 = 0.0;
+            if (t < 4 * rows) {
+#pragma unroll 8
+                for (int q = 0; q < nc; q += 2) {
+                    p0 += (double)A[q * 4 * rows] * vec[4 * q + h];
+                    p1 += (double)A[(q + 1) * 4 * rows] * vec[4 * q + 4 + h];
+                }
+            }
+            const double s = group_sum(p0 + p1, 4);
+            if (t < 4 * rows && h == 0) out(t >> 2, s);
+            __syncthreads();
+        };
+        apply(0, 0, v1, [&](int r, double s) { x1[r] = s; });
+        apply(1, 0, x1, [&](int r, double s) { v2[r] -= s; });
+        apply(1, 1, v2, [&](int r, double s) { x2[r] = s; });
+        apply(0, 1, x2, [&](int r, double s) { x1[r] -= s; });
+    } else
     {   // four lanes a row of the tail's inverse, each every fourth column
         double p0 = 0.0, p1 = 0.0;
 #pragma unroll
@@ -2260,7 +2444,7 @@ PHASE int sparse_setup_phase(const DevNet *Np, Lds L_, LUT *M, double *J, double
     M = uniform_ptr(M);
     J = uniform_ptr(J);
     PhaseClock clk(L);
-    if (N.nw_stage) return staged_setup<LUT>(N, L, M, J, gamma);
+    if (N.nw_stage) return staged_setup<LUT>(uniform_ptr(Np), N, L, M, J, gamma);
     sparse_jacobian(N, L, J);
     sparse_form_newton<LUT>(N, J, M, gamma, L.prm[P_ENFORCECHARGE] != 0.0);
     clk.mark(TM_JAC);
