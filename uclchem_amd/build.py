@@ -16,6 +16,10 @@ FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "-shared", f"--offload-arch={ARCH}",
     # keep the compiler from emitting packed FP32 instructions
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # 64-bit literals stay where they are used: hoisted out of the step loop they exceed the
+    # registers that survive the phase calls, and every step reloads them from scratch memory
+    # (default network, 8 points: 50.0 us a step with the hoisting, 45.8 without)
+    "-mllvm", "-disable-machine-licm",
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
 ]
 
