@@ -8,6 +8,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include "bdf_core.h"
 #include "ucg_plan.h"
 
 namespace ucg {
@@ -343,7 +344,7 @@ __device__ __forceinline__ double pick_uniform(double x, double lo, const double
 {   // v[number of knots lo + 1, lo + 2, ... below x], at most n - 1
     double r = v[0];
 #pragma unroll
-    for (int i = 1; i < n; i++) r = x > lo + i ? v[i] : r;
+    for (int i = 1; i < n; i++) r = bdf::sel(x > lo + i, v[i], r);   // by value: not from a computed address
     return r;
 }
 __device__ __forceinline__ void photo_rates_wave(double h2col, double cocol, double radfield, double scat1000, double av,
@@ -405,15 +406,24 @@ __device__ __forceinline__ void photo_rates_wave(double h2col, double cocol, dou
         double lb = (5675.0 - 200.6 * lw) - (571.6 - 24.09 * lw) * lu + (18.22 - 0.7664 * lw) * (lu * lu);
         if (lb > 1076.1) lb = 1076.1;
         if (lb < 913.6) lb = 913.6;
-        double x0 = c_photo.lam[0], x1 = c_photo.lam[1], v0 = c_photo.xl[0], v1 = c_photo.xl[1], e0 = c_photo.xl_d2[0],
-               e1 = c_photo.xl_d2[1];
+        double lam[5], xv[5], xd[5];
 #pragma unroll
-        for (int k = 1; k < 4; k++)
-            if (lb > c_photo.lam[k]) {
-                x0 = c_photo.lam[k]; x1 = c_photo.lam[k + 1];
-                v0 = c_photo.xl[k]; v1 = c_photo.xl[k + 1];
-                e0 = c_photo.xl_d2[k]; e1 = c_photo.xl_d2[k + 1];
-            }
+        for (int k = 0; k < 5; k++) {
+            lam[k] = c_photo.lam[k];
+            xv[k] = c_photo.xl[k];
+            xd[k] = c_photo.xl_d2[k];
+        }
+        double x0 = lam[0], x1 = lam[1], v0 = xv[0], v1 = xv[1], e0 = xd[0], e1 = xd[1];
+#pragma unroll
+        for (int k = 1; k < 4; k++) {
+            const bool c = lb > lam[k];
+            x0 = bdf::sel(c, lam[k], x0);
+            x1 = bdf::sel(c, lam[k + 1], x1);
+            v0 = bdf::sel(c, xv[k], v0);
+            v1 = bdf::sel(c, xv[k + 1], v1);
+            e0 = bdf::sel(c, xd[k], e0);
+            e1 = bdf::sel(c, xd[k + 1], e1);
+        }
         const double h = x1 - x0, a = (x1 - lb) / h, b = (lb - x0) / h;
         double xl = a * v0 + b * v1 + ((a * a * a - a) * e0 + (b * b * b - b) * e1) * (h * h) / 6.0;
         if (xl < 0.0) xl = 0.0;

@@ -13,7 +13,6 @@
 // registers: rate and flux arrays [NREAC], the RHS input/output and solve vectors
 // [NEQ], and each thread's slice of the Nordsieck history (registers).
 #include "ucg_device.h"
-#include "bdf_core.h"
 
 namespace ucg {
 
@@ -565,9 +564,9 @@ __device__ __forceinline__ double term_of(NetRef N, int k, double r, const LDS d
 // run the same instructions; one wave evaluates the photo rates meanwhile and one forms totalSwap
 // and the terms that carry it.  Sums: one slice program over the signed production and loss terms
 // of each species, whose records do not depend on the state.  Ice transfer and totals: one wave.
-// Bound by the LDS gathers and the latency of the three parts: 7.7 us a call (default
-// network), against 17.5 for chunked sums with a second pass over the chunks, workgroup-wide
-// reductions for each total and serial photo-rate splines.
+// Bound by the LDS gathers and the latency of the three parts: 6.8 us a call (default
+// network; 6.2 with 150 species), against 17.5 for chunked sums with a second pass over the
+// chunks, workgroup-wide reductions for each total and serial photo-rate splines.
 __device__ __forceinline__ void block_rhs(NetRef N_, const Lds L)
 {
     NetRef N = fresh(N_);
@@ -599,7 +598,6 @@ __device__ __forceinline__ void block_rhs(NetRef N_, const Lds L)
             flux[N.r_h2_hv] = term_of(N, N.r_h2_hv, kh, y);
             flux[N.nreac] = 0.0;                       // padding of the sums
         }
-        if (lane == 63) f[neq - 1] = densdot_dev(prm, D);
     } else {
         if (w == NWAVE - 2) {
             double ts = 0.0;
@@ -646,6 +644,14 @@ __device__ __forceinline__ void block_rhs(NetRef N_, const Lds L)
     const GLB uint32_t *srec = glb(N.pg_sum.rec) + 2 * lane;
     const auto load = [&](int r) { return ld_uint2(srec, 64 * r); };
     sums.first(N.pg_sum, load);
+    // the transfer's first 64 pairs of each list, ahead of the two barriers
+    const GLB int *ls = glb(N.fin_surf), *lb = glb(N.fin_bulk);
+    const int ns = N.nfin_surf, nb = N.nfin_bulk;
+    int2 sp0 = make_int2(0, 0), bp0 = make_int2(0, 0);
+    if (w == 0) {
+        if (lane < ns) sp0 = make_int2(ls[2 * lane], ls[2 * lane + 1]);
+        if (lane < nb) bp0 = make_int2(lb[2 * lane], lb[2 * lane + 1]);
+    }
     __syncthreads();
     clk.mark(TM_RHS_FLUX);
     {
@@ -666,24 +672,24 @@ __device__ __forceinline__ void block_rhs(NetRef N_, const Lds L)
     }
     __syncthreads();
     clk.mark(TM_RHS_SUMS);
+    if (w == 1 && lane == 0) f[neq - 1] = densdot_dev(prm, D);
     if (w == 0) {
         // bulk<->surface transfer (odes.f90:4818-5153), then the BULK and SURFACE totals
-        const GLB int *ls = glb(N.fin_surf), *lb = glb(N.fin_bulk);
         double S = 0.0;
-        for (int q = lane; q < N.nfin_surf; q += 64) S += f[ls[2 * q]];
+        for (int q = lane; q < ns; q += 64) S += f[q == lane ? sp0.x : ls[2 * q]];
         S = wave_sum(S);
         const bool neg = S < 0;
         const double fb = neg ? S * fmin(1.0, sbk / sm) / sbk : 0.0, fs = S * SURFACE_COVERAGE0;
         double tsu = 0.0, tb = 0.0;
-        for (int q = lane; q < N.nfin_surf; q += 64) {
-            const int i = ls[2 * q], b = ls[2 * q + 1];
+        for (int q = lane; q < ns; q += 64) {
+            const int i = q == lane ? sp0.x : ls[2 * q], b = q == lane ? sp0.y : ls[2 * q + 1];
             double v = f[i];
             if (b >= 0) v -= neg ? fb * y[b] : fs * y[i];
             f[i] = v;
             tsu += v;
         }
-        for (int q = lane; q < N.nfin_bulk; q += 64) {
-            const int i = lb[2 * q], s = lb[2 * q + 1];
+        for (int q = lane; q < nb; q += 64) {
+            const int i = q == lane ? bp0.x : lb[2 * q], s = q == lane ? bp0.y : lb[2 * q + 1];
             const double v = f[i] + (neg ? fb * y[i] : s >= 0 ? fs * y[s] : 0.0);
             f[i] = v;
             tb += v;
