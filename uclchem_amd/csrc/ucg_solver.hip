@@ -450,14 +450,31 @@ __device__ __forceinline__ double term_value(NetRef N, int k, const double *rate
 }
 
 // Sum over aligned groups of G lanes (a power of two, uniform); every lane gets its group's sum.
+// Lanes of a subgroup hold the same sum, so that a mirror of the lanes serves as well as an
+// exchange: DPP within rows of 16 and lane swaps beyond them, about 20 cycles a level against the
+// 60 to 90 of a shuffle through the LDS pipe.
+template <int CTRL> __device__ __forceinline__ double dpp_all(double v)
+{   // a DPP control that brings every lane a value
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
 __device__ __forceinline__ double group_sum(double v, int G)
 {
-    if (G >= 2) v += __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0xB1, 0xf, 0xf, true));
-    if (G >= 4) v += __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x4E, 0xf, 0xf, true));
-    if (G >= 8) v += __shfl_xor(v, 4);
-    if (G >= 16) v += __shfl_xor(v, 8);
-    if (G >= 32) v += __shfl_xor(v, 16);
-    if (G >= 64) v += __shfl_xor(v, 32);
+    if (G >= 2) v += dpp_all<0xB1>(v);     // quad_perm 1 0 3 2
+    if (G >= 4) v += dpp_all<0x4E>(v);     // quad_perm 2 3 0 1
+    if (G >= 8) v += dpp_all<0x141>(v);    // row_half_mirror
+    if (G >= 16) v += dpp_all<0x140>(v);   // row_mirror
+    if (G >= 32) {                         // a pair of rows each
+        const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
+        v = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    }
+    if (G >= 64) {                         // the two halves
+        const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(v), (unsigned)__double2loint(v), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(v), (unsigned)__double2hiint(v), false, false);
+        v = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    }
     return v;
 }
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(tid() >> 6); }
@@ -479,7 +496,7 @@ struct Slices {
     static __device__ __forceinline__ int field(int v, int i) { return __builtin_amdgcn_readlane(v, i); }
     __device__ __forceinline__ void list(const CST DevProg &G)
     {
-        const GLB int *lp = glb(G.list_ptr) + wave_id();
+        const CST int *lp = (const CST int *)G.list_ptr + wave_id();   // one scalar load ahead of the vector one
         s0 = lp[0];
         n = lp[1] - s0;
         d = ld_int4(glb(G.list), s0 + (tid() & 63));
