@@ -926,21 +926,11 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
         P.finish(ucg::NWAVE, true);
         if ((rc = upload_program(h, P, N.pg_sum))) return rc;
     }
-    {   // packed term records {n_d, ops[6], nfac}
-        std::vector<int> prog(8 * R);
-        for (size_t k = 0; k < R; k++) {
-            prog[8 * k] = d->n_d[k];
-            for (int q = 0; q < ucg::MAXOPS; q++) prog[8 * k + 1 + q] = d->ops[ucg::MAXOPS * k + q];
-            prog[8 * k + 7] = d->nfac[k];
-        }
-        if ((rc = upload(h, prog.data(), prog.size(), N.prog))) return rc;
-    }
     UP(type_ranges, (size_t)2 * ucg::NTYPES);
-    UP(loss_ptr, (size_t)d->nspec + 1); UP(loss_idx, (size_t)d->nloss);
-    UP(prod_ptr, (size_t)d->nspec + 1); UP(prod_idx, (size_t)d->nprod); UP(swap_list, (size_t)d->nswap);
+    UP(swap_list, (size_t)d->nswap);
     UP(surface_list, (size_t)d->nsurfl); UP(bulk_list, (size_t)d->nbulkl);
-    UP(bulk_partner_of_surface, Q); UP(surface_partner_of_bulk, Q);
-    UP(freeze_partners, (size_t)d->nfp); UP(is_surface, Q); UP(is_bulk, Q);
+    UP(bulk_partner_of_surface, Q);
+    UP(freeze_partners, (size_t)d->nfp);
     UP(jnz_row, (size_t)d->nnz); UP(jnz_col, (size_t)d->nnz); UP(jnz_ptr, (size_t)d->nnz + 1);
     UP(jc_k, (size_t)d->ncontrib); UP(jc_m, (size_t)d->ncontrib); UP(jc_c, (size_t)d->ncontrib);
     UP(aff_ptr, R + 1); UP(aff_sp, (size_t)d->naff); UP(aff_cf, (size_t)d->naff);

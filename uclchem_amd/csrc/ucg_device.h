@@ -98,15 +98,12 @@ struct DevNet {
     int32_t nspec, neq, nreac, nice, nsurfl, nbulkl, nfp, nswap, nnz, ld;
     const double *alpha, *beta, *gama, *tmin, *tmax, *mass, *rstat;  // rstat [nreac*5]
     const int32_t *rtype, *re, *pr, *ice_kind, *n_d, *ops, *fac, *nfac;
-    const int32_t *prog;   // [nreac*8] {n_d, ops[6], nfac}, 32-byte aligned records
     const int32_t *facp;   // [nreac*4] factor codes as int16 x 8 (density factors first), -1 padded
     const int32_t *fac_off, *jc_pk;   // partial offsets [nreac+1]; contributions (partial << 4 | coef + 8)
     int32_t npart, npart_pad;         // number of partials; LDS offset of the scratch after them
     const int8_t *extrapolate;
     const int32_t *type_ranges;                                     // [NTYPES*2]
-    const int32_t *loss_ptr, *loss_idx, *prod_ptr, *prod_idx, *swap_list;
-    const int32_t *surface_list, *bulk_list, *bulk_partner_of_surface, *surface_partner_of_bulk;
-    const int32_t *freeze_partners, *is_surface, *is_bulk;          // is_*: [neq]
+    const int32_t *swap_list, *surface_list, *bulk_list, *bulk_partner_of_surface, *freeze_partners;
     const int32_t *jnz_row, *jnz_col, *jnz_ptr, *jc_k, *jc_m, *jc_c;
     // Jacobian entries in evaluation order: nj_short with at most JZ_LONG contributions (one
     // lane each, dealt so that every lane gets a near-equal share), nj_long with more (one

@@ -311,27 +311,23 @@ LDS_BYTES_PER_CU = 160 * 1024
 
 
 def lds_bytes(tables, staged: bool = True) -> int:
-    """LDS one solve workgroup needs (mirror of lds_bytes/flux_region_len in the HIP
-    library): the shared region (fluxes, Jacobian term partials, and
-    for a staged plan the staged factors, solve program and dense tail) plus the NEQ-long
-    vectors, reduction slots, scalars and parameters."""
+    """LDS one solve workgroup needs.  With staged=False (plans that run from the workspace, and the
+    dense form) this is the library's size: fluxes or Jacobian term partials, the NEQ-long vectors,
+    reduction slots, scalars and parameters.  For a staged plan it is an upper estimate: partials
+    and sparse factors side by side, the dense tail (a panel of it beyond 128 rows), or the exchange
+    buffers of its inversion; the library's planner gives slots only to values that meet there."""
     a = tables.arrays
     z = a["nw_sizes"]
-    N, T, nsp, nlev = int(z[0]), int(z[2]), int(z[3]), int(z[4])
+    N, T, nsp = int(z[0]), (int(z[2]) + 15) & ~15, int(z[3])
     npad = (tables.neq + 7) & ~7
-    Npad = (N + 7) & ~7
     npart = int(a["nfac"].sum())
-    b = max(tables.nreac + 1, ((npart + 7) & ~7) + 2 * npad, 512)
+    b = max(tables.nreac + 1, ((npart + 7) & ~7) + 2 * npad, 3 * ((N + 7) & ~7), 512)
     if staged:
-        al = lambda x: (x + 15) & ~15
-        stage = lambda nst, lut: al(nst * lut) + al(nsp * 4) + N * 16 + al((N + nlev + 1) * 4) + N * 8 + T * 8
-        gj = 2 * ((T + 15) // 16 + 1) * 16 * 17          # exchange buffers of the tail's inversion
-        c = max(T * T + max(((schur_sources(tables) + 7) & ~7) + Npad, gj), (stage(nsp + T * T, 4) + 7) // 8,
-                (stage(nsp, 8) + 7) // 8)
-    else:
-        c = Npad
+        tail = T * T if T <= 128 else 128 * 130
+        gj = (2 * (min(T, 128) // 16 + 1) + 1) * 16 * 17
+        b = max(b, (npart if T <= 128 else 64 * 130) + nsp, tail, gj)
     from .params import NPARAM
-    return 8 * (max(b, c) + ((tables.neq + 4 + 7) & ~7) + 3 * npad + 144 + 40 + NPARAM)   # + reduction slots, scalars, parameters
+    return 8 * (b + ((tables.neq + 4 + 7) & ~7) + 3 * npad + 144 + 40 + NPARAM)   # + reduction slots, scalars, parameters
 
 
 def schur_sources(tables) -> int:
@@ -354,6 +350,6 @@ def schur_sources(tables) -> int:
 
 
 def plan_is_staged(tables) -> bool:
-    """Whether the library stages this network's plan in LDS (else it runs it from the workspace):
-    it fits, and the tail fits the waves that invert it in registers (128 rows)."""
-    return lds_bytes(tables, True) <= LDS_BYTES_PER_CU and int(tables.arrays["nw_sizes"][2]) <= 128
+    """Whether the library is sure to stage this network's plan in LDS (else it may run it from the
+    workspace): the tail fits the registers of the waves that invert it (256 rows), the estimate LDS."""
+    return lds_bytes(tables, True) <= LDS_BYTES_PER_CU and int(tables.arrays["nw_sizes"][2]) <= 256
