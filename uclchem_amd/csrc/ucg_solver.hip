@@ -43,7 +43,7 @@ __device__ __forceinline__ int tid() { return (int)threadIdx.x; }
 // the integrator's state stays in callee-saved registers across them and each phase is
 // allocated by itself, in a single copy of its code.  With everything inlined the history and the
 // control state lived in scratch memory: the work of a step outside these phases took 35 us, 13
-// like this (default network, FP64).  Arguments arrive in vector registers; these move the
+// like this, 9 with 64-bit literals left at their uses (a build flag; default network, FP64).  Arguments arrive in vector registers; these move the
 // uniform ones back to scalar registers.
 #define PHASE __device__ __attribute__((noinline))
 __device__ __forceinline__ uint64_t uniform64(uint64_t p)
@@ -1287,8 +1287,10 @@ UCG_BIG __device__ int block_lu_tiled(MP M, int n, int ld, LDS double *red, LDS 
 //
 // The register-blocked sweeps over LDS that this replaces (8 pivots a sweep) took 105 us for the
 // default network's 104 rows, bound by LDS round trips and three barriers a sweep; this form takes
-// 26 us, 32 when the owner inverts its block itself.  Its floor is the matrix cores' 10 us for
-// 2 n^3 FLOP at FP64 on one CU; a pivot block's inversion is 16 dependent steps, 1.5 us.
+// 27 us, 33 when the owner inverts its block itself.  Its floor is the matrix cores' 10 us for
+// 2 n^3 FLOP at FP64 on one CU.  A sweep is 3.7 us, of which the inversion of the next pivot block
+// (16 dependent steps) is 2.4: alone it takes 1.6, but FP64 vector instructions and the FP64 MFMAs
+// of the column wave on the same SIMD share one unit.
 constexpr int GJ_MAX = 16 * NWAVE;        // rows one workgroup's waves can hold
 constexpr int GJ_TILE = 16 * 17;          // LDS tile, column-major, column stride 17 (bank spread)
 using f64x4 = __attribute__((ext_vector_type(4))) double;
@@ -2398,13 +2400,22 @@ __device__ __forceinline__ void staged_solve(NetRef N_, const Lds &L, const LUT 
         apply(1, 1, v2, [&](int r, double s) { x2[r] = s; });
         apply(0, 1, x2, [&](int r, double s) { x1[r] -= s; });
     } else
-    {   // four lanes a row of the tail's inverse, each every fourth column
+    {   // four lanes a row of the tail's inverse, each every fourth column, in two chains (one chain
+        // over the columns fetched ahead took 0.3 us more a step: 43.9 against 43.5)
         double p0 = 0.0, p1 = 0.0;
 #pragma unroll
-        for (int q = 0; q < TAIL_AHEAD; q++) p0 += (double)Sa[q] * v[ns + min(4 * q + h, T1)];
+        for (int q = 0; q < TAIL_AHEAD; q += 2) {
+            p0 += (double)Sa[q] * v[ns + min(4 * q + h, T1)];
+            p1 += (double)Sa[q + 1] * v[ns + min(4 * q + 4 + h, T1)];
+        }
         if (t < 4 * T) {
-#pragma unroll 8
-            for (int q = TAIL_AHEAD; q < nst; q++) p1 += (double)S[q * 4 * T] * v[ns + min(4 * q + h, T1)];
+            int q = TAIL_AHEAD;
+#pragma unroll 4
+            for (; q + 2 <= nst - 1; q += 2) {
+                p0 += (double)S[q * 4 * T] * v[ns + min(4 * q + h, T1)];
+                p1 += (double)S[(q + 1) * 4 * T] * v[ns + min(4 * q + 4 + h, T1)];
+            }
+            for (; q < nst; q++) p0 += (double)S[q * 4 * T] * v[ns + min(4 * q + h, T1)];
         }
         const double s = group_sum(p0 + p1, 4);
         if (t < 4 * T && h == 0) x[ns + (t >> 2)] = s;
