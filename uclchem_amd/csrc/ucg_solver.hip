@@ -13,6 +13,7 @@
 // registers: rate and flux arrays [NREAC], the RHS input/output and solve vectors
 // [NEQ], and each thread's slice of the Nordsieck history (registers).
 #include "ucg_device.h"
+#include "ucg_reduce.h"
 
 namespace ucg {
 
@@ -133,10 +134,8 @@ __device__ __forceinline__ double wave_max0(double v)   // v >= 0
     return wave_lane(v, 63);
 }
 
-// Workgroup reductions with one barrier: each wave's total goes to its slot of a buffer, every
-// wave adds all of them.  A buffer may be used again once a barrier lies between its last use
-// and the next; the call sites use distinct buffers (RED_*) so that this always holds.
-enum { RED_TS, RED_S, RED_TOTALS, RED_CHARGE, RED_EWT, RED_ACOR, RED_CORR, RED_HIST, RED_NBUF };
+// Workgroup reductions with one barrier: each wave's total goes to its slot of buffer `id`
+// (ucg_reduce.h says when two may share one), every wave adds all of them.
 constexpr int RED_FLAGS = 16;                                   // red[0..15]: flags and small scratch
 constexpr int RED_LEN = RED_FLAGS + RED_NBUF * 2 * NWAVE;
 __device__ __forceinline__ double block_sum(double v, LDS double *red, int id)
@@ -2568,7 +2567,7 @@ struct GpuOps {
                 double t = x * ewt[e];
                 acc += t * t;
             }
-        return bdf_uni(sqrt(block_sum(acc, L.red, v == bdf::ACOR ? RED_ACOR : RED_HIST) / neq));
+        return bdf_uni(sqrt(block_sum(acc, L.red, v == bdf::ACOR ? OpsBuffers::acor : OpsBuffers::history) / neq));
     }
     __device__ __forceinline__ double wrms_acor_minus(double c, int zj)
     {
@@ -2579,7 +2578,7 @@ struct GpuOps {
                 double t = (acor[e] - c * zget(zj, e)) * ewt[e];
                 acc += t * t;
             }
-        return bdf_uni(sqrt(block_sum(acc, L.red, RED_CORR) / neq));
+        return bdf_uni(sqrt(block_sum(acc, L.red, OpsBuffers::order) / neq));
     }
     // error weights of z[0], their check and z[0]'s norm in them, one reduction
     __device__ __forceinline__ bool set_ewt(double rtol)
@@ -2594,7 +2593,7 @@ struct GpuOps {
                 double t = z[0][e] * ewt[e];
                 acc += t * t;
             }
-        block_sum2(acc, bad, L.red, RED_EWT);
+        block_sum2(acc, bad, L.red, OpsBuffers::weights);
         z0_norm = bdf_uni(sqrt(acc / neq));
         return bad == 0.0;
     }
@@ -2710,7 +2709,7 @@ struct GpuOps {
                 acor[e] += d;
                 L.y[i] = z[0][e] + acor[e];
             }
-        double r = bdf_uni(sqrt(block_sum(acc, L.red, RED_CORR) / neq));
+        double r = bdf_uni(sqrt(block_sum(acc, L.red, OpsBuffers::correction) / neq));
         return r;
     }
     // Reusing a saved J between Newton-matrix setups (DVODE's JSV=1) was measured on the
@@ -2733,7 +2732,7 @@ struct GpuOps {
 #pragma unroll
         for (int e = 0; e < EPT; e++)
             if (own(e)) m = fmax(m, fabs(f0[e]) / (fac * fabs(z[0][e]) + atol[e]));
-        return block_max0(m, L.red, RED_HIST);
+        return block_max0(m, L.red, OpsBuffers::first_step);
     }
     __device__ __forceinline__ double ydd_norm(double t0, double hg)
     {
@@ -2749,7 +2748,7 @@ struct GpuOps {
                 double t = (L.f[idx(e)] - f0[e]) / hg * ewt[e];
                 acc += t * t;
             }
-        return bdf_uni(sqrt(block_sum(acc, L.red, RED_CORR) / neq));
+        return bdf_uni(sqrt(block_sum(acc, L.red, OpsBuffers::ydd) / neq));
     }
     __device__ void finish_at_tn() {}
     __device__ __forceinline__ void interpolate(double s, int q)

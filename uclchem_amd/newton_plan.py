@@ -327,7 +327,7 @@ def lds_bytes(tables, staged: bool = True) -> int:
         gj = (2 * (min(T, 128) // 16 + 1) + 1) * 16 * 17
         b = max(b, (npart if T <= 128 else 64 * 130) + nsp, tail, gj)
     from .params import NPARAM
-    return 8 * (b + ((tables.neq + 4 + 7) & ~7) + 3 * npad + 144 + 40 + NPARAM)   # + reduction slots, scalars, parameters
+    return 8 * (b + ((tables.neq + 4 + 7) & ~7) + 3 * npad + 160 + 40 + NPARAM)   # + reduction slots, scalars, parameters
 
 
 def schur_sources(tables) -> int:
