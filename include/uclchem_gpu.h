@@ -218,7 +218,8 @@ int ucg_solve_batch_device_noalloc(int handle, int n, const double *params, cons
 
 /* Stop every solve launched on a handle before this call (ucg_solve_batch_device launches,
  * including ones queued behind other work, and the handle's request queues): workgroups
- * finish their current integrator step and take no further points; unfinished points
+ * stop at the latest 16 integrator steps later (of 0.03 to 0.1 ms; the dense form and plans run
+ * from the workspace: after the current step) and take no further points; unfinished points
  * report UCG_E_CANCELLED and a stopped queue's unrun requests fail ucg_queue_test.
  * Launches issued after the call are not affected.  Callable from another host thread
  * while the solves run (not concurrently with ucg_network_free of the same handle).  No

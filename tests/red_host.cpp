@@ -5,6 +5,11 @@
 // Recorder computes as HostOps does and logs what the kernel's Ops does in the same call: a
 // reduction is a write to its buffer, a barrier, and reads of it; the other calls have the barriers
 // listed here at least (a barrier more in the kernel would only separate uses further).
+#include <pthread.h>
+
+#include <atomic>
+#include <thread>
+
 #include "bdf_host.cpp"
 
 #include "../uclchem_amd/csrc/ucg_reduce.h"
@@ -114,5 +119,30 @@ int red_host_run(int problem, int ncalls, const double *tout, double rtol, doubl
     out[1] = o.reductions;
     out[2] = o.order_after_correction;
     return r;
+}
+
+// `threads` threads poll a cancel word that answers 1 from its `raised`-th reading on, `calls`
+// times each, every `every`-th call.  seen [threads][calls]: what each poll returned; returns the
+// number of readings of the word.
+int red_host_cancel(int threads, int calls, int every, int raised, int *seen)
+{
+    pthread_barrier_t bar;
+    pthread_barrier_init(&bar, nullptr, threads);
+    std::atomic<int> readings{0};
+    double flag = 0.0;
+    std::vector<std::thread> team;
+    for (int w = 0; w < threads; w++)
+        team.emplace_back([&, w] {
+            int n = 0;
+            for (int c = 0; c < calls; c++) {
+                seen[w * calls + c] = ucg::cancel_poll(
+                    n, every, w == 0, flag, [&] { return ++readings >= raised; },
+                    [&] { pthread_barrier_wait(&bar); });
+                pthread_barrier_wait(&bar);   // a step has barriers
+            }
+        });
+    for (auto &t : team) t.join();
+    pthread_barrier_destroy(&bar);
+    return readings;
 }
 }

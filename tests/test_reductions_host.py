@@ -23,10 +23,12 @@ def lib(tmp_path_factory):
     if cxx is None:
         pytest.skip("g++ not available")
     out = str(tmp_path_factory.mktemp("red_host") / "libredhost.so")
-    subprocess.check_call([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-o", out, os.path.join(HERE, "red_host.cpp")])
+    subprocess.check_call([cxx, "-O2", "-std=c++17", "-shared", "-fPIC", "-pthread", "-o", out,
+                           os.path.join(HERE, "red_host.cpp")])
     lib = ctypes.CDLL(out)
     lib.red_host_run.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_double, ctypes.c_double,
                                  ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p]
+    lib.red_host_cancel.argtypes = [ctypes.c_int] * 4 + [ctypes.c_void_p]
     return lib
 
 
@@ -40,3 +42,19 @@ def test_no_buffer_is_reused_without_a_barrier(lib, problem, rtol, mxstep):
     assert reductions > 20
     assert after_correction > 0      # the path without a barrier is taken
     assert hazards == 0
+
+
+@pytest.mark.parametrize("every", [1, 16])
+@pytest.mark.parametrize("raised", [1, 2, 3])
+def test_every_thread_gets_the_same_answer_to_a_cancel(lib, every, raised):
+    """The word is raised between two readings; the threads of a workgroup must agree in every call
+    (they meet barriers in what follows), and only one of them reads it."""
+    threads, calls = 8, 64
+    seen = np.zeros((threads, calls), dtype=np.int32)
+    readings = lib.red_host_cancel(threads, calls, every, raised, seen.ctypes.data)
+    assert np.all(seen == seen[0])
+    assert readings == calls // every
+    first = (raised - 1) * every
+    want = np.zeros(calls, dtype=np.int32)
+    want[first::every] = 1
+    assert np.array_equal(seen[0], want)

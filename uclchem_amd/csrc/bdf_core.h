@@ -24,7 +24,7 @@
 //   2 success, -1 step limit, -2 tolerance too small, -4 repeated error-test
 //   failures, -5 repeated convergence failures, -3 illegal input,
 //   -6 singular/invalid Newton matrix or non-finite state, -7 cancelled by the caller
-//   (Ops::cancelled(), asked once per step).
+//   (Ops::cancelled(), called once per step).
 // On a negative return the state is the last accepted step (t = tn, y = zn[0]).
 #pragma once
 

@@ -1,4 +1,5 @@
-// Buffers of the solve kernel's workgroup reductions.
+// What the waves of a solve workgroup decide together: the buffers of their reductions, and how
+// they learn of a cancel.
 //
 // A reduction has one barrier: each wave writes its total to its slot of a buffer, a barrier
 // follows, every wave adds up all slots.  A wave may still be reading after the barrier while
@@ -7,6 +8,7 @@
 // the next; the reductions that can meet on such a path have buffers of their own
 // (tests/red_host.cpp follows the control code and checks every pair).
 #pragma once
+#include "bdf_core.h"
 
 namespace ucg {
 
@@ -24,5 +26,18 @@ struct OpsBuffers {
     static constexpr int first_step = RED_HIST;  // hub_inverse
     static constexpr int ydd = RED_CORR;         // ydd_norm
 };
+
+// Whether the caller has cancelled the launch, asked every `every`-th call (a power of two).  The
+// host may raise the word at any moment, so one thread asks and all take its answer behind the
+// barrier: were every wave to ask, some would leave the step loop and others go on into its
+// barriers.  `flag` is shared by the threads; at least one more barrier lies between two askings.
+template <class Flag, class Ask, class Barrier>
+BDF_HD bool cancel_poll(int &calls, int every, bool asks, Flag &flag, Ask ask, Barrier barrier)
+{
+    if ((calls++ & (every - 1)) != 0) return false;
+    if (asks) flag = ask() ? 1.0 : 0.0;
+    barrier();
+    return bdf_uni(flag) != 0.0;
+}
 
 }  // namespace ucg

@@ -137,6 +137,7 @@ __device__ __forceinline__ double wave_max0(double v)   // v >= 0
 // Workgroup reductions with one barrier: each wave's total goes to its slot of buffer `id`
 // (ucg_reduce.h says when two may share one), every wave adds all of them.
 constexpr int RED_FLAGS = 16;                                   // red[0..15]: flags and small scratch
+constexpr int RED_CANCEL = 10;                                  // the flag of cancel_poll
 constexpr int RED_LEN = RED_FLAGS + RED_NBUF * 2 * NWAVE;
 __device__ __forceinline__ double block_sum(double v, LDS double *red, int id)
 {
@@ -2518,9 +2519,14 @@ struct GpuOps {
     const int *cancel = nullptr;  // highest cancelled launch generation, raised by the host while kernels run
     int gen = 0;                  // this launch's generation
     int polls = 0;
-    // the cancel word is in memory shared with the host (a load from it takes microseconds):
-    // read it at every 16th step
-    __device__ __forceinline__ bool cancelled() { return (polls++ & 15) == 0 && cancel_requested(cancel, gen); }
+    // the load of the cancel word bypasses the caches and takes microseconds: a staged plan, whose
+    // steps take 33 to 112 us, reads it at every 16th step, the slower forms at every step
+    __device__ __forceinline__ bool cancelled()
+    {
+        return cancel_poll(
+            polls, staged ? 16 : 1, tid() == 0, L.red[RED_CANCEL], [&] { return cancel_requested(cancel, gen); },
+            [] { __syncthreads(); });
+    }
 
     __device__ GpuOps(const DevNet *np_, Lds &l_, LUT *m_)
         : N(*(const CST DevNet *)np_), Np(np_), L(l_), M(m_), neq(((const CST DevNet *)np_)->neq)
