@@ -309,7 +309,7 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
     // right-hand-side sums of the replaced rows: entries of their L21 rows on the permuted
     // right-hand side itself when all those rows lie in the tail
     const int NB = d->special_species[24], NS = d->special_species[23], NE = d->special_species[21];
-    const bool charge = d->nion > 0 && NE < d->nspec;
+    const bool charge = NE < d->nspec;   // as the device decides: with no positive ion the sum is empty
     std::vector<std::pair<int, std::vector<int>>> sums(3);
     sums[0].first = d->nw_inv[NB];
     for (int q = 0; q < d->nbulkl; q++) sums[0].second.push_back(d->nw_inv[d->bulk_list[q]]);
