@@ -166,6 +166,11 @@ int ucg_network_load(const ucg_network_desc *desc, int *handle);
 int ucg_network_load_file(const char *path, int *handle);
 int ucg_network_free(int handle);
 
+/* How solves with the network's sparse plan run: form 0: from the workspace, 1: staged in LDS
+ * and matrix-core registers, 2: staged with a wide tail (129..256 rows); lds: bytes of LDS a
+ * solve workgroup takes (the dense form takes the same). */
+int ucg_network_plan(int handle, int *form, int *lds);
+
 /* Full single-point models for a batch of independent grid points.
  *   params  [n][UCG_NPARAM]; y_init [n][neq] or NULL for UCLCHEM's elemental start
  *   y_out   [n][neq] final state (abundances + density)

@@ -10,7 +10,8 @@ extern "C" {
 
 // Programs for `nwave` waves and at most `max_tail` tail rows (twice that as a wide tail).
 // out: ok, wide, presum, sparse rows, tail rows, working slots, then {row, first, end} of the three
-// sums, then the most slices a wave has in the entry program.  Returns 0, or -1 if the planner threw.
+// sums, then the most slices a wave has in the entry and in the elimination program.  Returns 0, or
+// -1 if the planner threw.
 int plan_host(const ucg_network_desc *d, int nwave, int max_tail, int *out)
 {
     std::vector<int> off((size_t)d->nreac + 1, 0);
@@ -20,9 +21,12 @@ int plan_host(const ucg_network_desc *d, int nwave, int max_tail, int *out)
         const int head[6] = {S.ok, S.wide, S.presum, S.ns, S.t, S.n_slots};
         for (int k = 0; k < 6; k++) out[k] = head[k];
         for (int k = 0; k < 9; k++) out[6 + k] = k < (int)S.sum_rows.size() ? S.sum_rows[k] : -1;
-        out[15] = 0;
-        for (size_t w = 1; w < S.entries.list_ptr.size(); w++)
-            out[15] = std::max(out[15], (int)(S.entries.list_ptr[w] - S.entries.list_ptr[w - 1]));
+        const ucg::Program *list[2] = {&S.entries, &S.elim};
+        for (int k = 0; k < 2; k++) {
+            out[15 + k] = 0;
+            for (size_t w = 1; w < list[k]->list_ptr.size(); w++)
+                out[15 + k] = std::max(out[15 + k], list[k]->list_ptr[w] - list[k]->list_ptr[w - 1]);
+        }
     } catch (const std::exception &) {
         return -1;
     }

@@ -35,10 +35,10 @@ def plan(tmp_path_factory):
             setattr(d, k, v.ctypes.data)
         d.special_species[:] = [int(x) for x in ssp]
         d.special_reactions[:] = [int(x) for x in srx]
-        res = np.zeros(16, dtype=np.int32)
+        res = np.zeros(17, dtype=np.int32)
         assert lib.plan_host(ctypes.byref(d), 8, 128, res.ctypes.data_as(ctypes.c_void_p)) == 0
         return dict(ok=res[0], wide=res[1], presum=res[2], ns=res[3], tail=res[4], slots=res[5],
-                    sums=res[6:15].reshape(3, 3), entry_slices=res[15])
+                    sums=res[6:15].reshape(3, 3), entry_slices=res[15], pivot_slices=res[16])
     return run
 
 
@@ -66,3 +66,17 @@ def test_sum_rows_of_a_network_without_positive_ions(plan, name, tail):
     assert np.all((without["sums"][:, 0] >= 0) & (without["sums"][:, 0] < rows))
     assert np.array_equal(without["sums"][:, 0], with_ions["sums"][:, 0])
     assert without["sums"][2, 1] == without["sums"][2, 2]      # nothing to add
+
+
+def test_elimination_lists_longer_than_a_wave(plan):
+    """A wave holds 64 slice descriptors at a time; the plan that test_gpu_plan_forms runs for longer
+    lists has them."""
+    import copy
+    from uclchem_amd import makerates_hip as mh
+    from uclchem_amd import newton_plan
+    from uclchem_amd import synthetic as sy
+    sp, re = sy.synthetic_species_and_reactions(140, 700)
+    t = mh.build_tables(sp, re, "synthetic_140_700")
+    t.arrays = {**t.arrays, **newton_plan.build_plan(t, split=t.neq + 2)}
+    p = plan(t)
+    assert p["ok"] and p["tail"] == 0 and p["pivot_slices"] > 64

@@ -1047,6 +1047,17 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
     return 0;
 }
 
+int ucg_network_plan(int handle, int *form, int *lds)
+{
+    std::lock_guard<std::mutex> lk(g_mu);
+    const NetHandle *h = get(handle);
+    if (!h) return fail(UCG_E_HANDLE, "bad network handle");
+    if (!form || !lds) return fail(UCG_E_ARG, "null argument");
+    *form = h->dev.nw_stage;
+    *lds = (int)lds_bytes(h->dev);
+    return 0;
+}
+
 int ucg_network_free(int handle)
 {
     std::lock_guard<std::mutex> lk(g_mu);

@@ -132,6 +132,16 @@ class Network:
         """Stop running device solves on this network (unfinished points: CANCELLED)."""
         _check(lib().ucg_cancel(ctypes.c_int(self.handle)), "ucg_cancel")
 
+    WORKSPACE, STAGED, STAGED_WIDE = 0, 1, 2
+
+    def plan_form(self) -> tuple:
+        """(form, LDS bytes a solve workgroup takes): how solves with the sparse plan run, from the
+        WORKSPACE, STAGED in LDS or STAGED_WIDE (a dense tail of 129..256 rows)."""
+        form, lds = ctypes.c_int(-1), ctypes.c_int(0)
+        _check(lib().ucg_network_plan(ctypes.c_int(self.handle), ctypes.byref(form), ctypes.byref(lds)),
+               "ucg_network_plan")
+        return form.value, lds.value
+
     def set_linear_solver(self, kind: int) -> None:
         """Network.SPARSE (static-pattern plan, default) or Network.DENSE (full LU)."""
         _check(lib().ucg_set_linear_solver(ctypes.c_int(self.handle), ctypes.c_int(kind)), "ucg_set_linear_solver")
