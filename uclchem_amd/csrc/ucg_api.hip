@@ -868,15 +868,19 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
         std::vector<int> sx;
         for (size_t k = 0; k < R; k++) {
             std::vector<unsigned> f;
-            int swaps = 0;
+            int swaps = 0, divs = 0;
             for (int m = 0; m < d->nfac[k]; m++) {
                 const int c = d->fac[ucg::MAXFAC * k + m];
                 if (c == ucg::OP_SWAP && !swaps++) continue;
+                if (c == ucg::OP_DIVSM && !divs++) continue;
                 f.push_back((unsigned)(c >= 0 ? c
                                             : d->neq + (c == ucg::OP_BLR ? ucg::YX_BLR : c == ucg::OP_DIVSM ? ucg::YX_ISM : ucg::YX_TSM)));
                 if (c == ucg::FAC_D) f.back() = (unsigned)d->neq - 1;
             }
+            // last place of the last record, where the RHS looks for them
+            if (divs && swaps) f.push_back((unsigned)(d->neq + ucg::YX_ISM));
             f.resize(4 * N.rx_w, (unsigned)(d->neq + ucg::YX_ONE));
+            if (divs) f.back() = (unsigned)(d->neq + ucg::YX_ISM);
             for (int m = 0; m < 4 * N.rx_w; m++) {   // term order, as the partials are numbered
                 const int c = m < d->nfac[k] ? d->fac[ucg::MAXFAC * k + m] : ucg::OP_NONE;
                 ucg::put16(&rp[2 * k * N.rx_w], m,
@@ -884,7 +888,7 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
                                       : d->neq + (c == ucg::OP_BLR ? ucg::YX_BLR : c == ucg::OP_DIVSM ? ucg::YX_ISM
                                                   : c == ucg::OP_SWAP ? ucg::YX_TSM : ucg::YX_ONE)));
             }
-            if (swaps) {   // last place of the last record, where the RHS looks for it
+            if (swaps) {
                 f.back() = (unsigned)(d->neq + ucg::YX_TSM);
                 sx.push_back((int)k);
             }
