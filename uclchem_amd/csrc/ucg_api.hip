@@ -48,11 +48,12 @@ struct NetHandle {
     void *ws = nullptr;
     size_t ws_bytes = 0;
     int *counter = nullptr;
-    int *cancel = nullptr;              // device word: highest cancelled launch generation
+    // pinned word: highest cancelled launch generation.  The host stores to it directly: a copy on a
+    // stream of its own waited for the solve whenever the two streams shared a hardware queue
+    int *cancel = nullptr;
     int gen = 0;                        // generation of the last launch on this handle
     int cancel_sent = 0;                // highest generation written to *cancel
     ucg::DevNet *d_dev = nullptr;       // device copy of dev, the kernels' table descriptor
-    hipStream_t cancel_stream = nullptr;
     int linear_solver = UCG_LINSOL_SPARSE;
 };
 std::vector<NetHandle> g_nets;
@@ -1034,9 +1035,6 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
     if ((rc = upload(h, d->gar_params, 7 * (size_t)d->ngar, N.gar))) return rc;
     HIPCHK(hipMalloc(&h.counter, sizeof(int)));
     h.allocs.push_back(h.counter);
-    HIPCHK(hipMalloc(&h.cancel, sizeof(int)));
-    h.allocs.push_back(h.cancel);
-    HIPCHK(hipMemset(h.cancel, 0, sizeof(int)));
     hipDeviceProp_t prop;
     HIPCHK(hipGetDeviceProperties(&prop, g_device));
     if ((rc = load_staged_plan(d, h, (size_t)prop.sharedMemPerBlock))) return rc;
@@ -1047,7 +1045,8 @@ static int load_tables(const ucg_network_desc *d, NetHandle &h)
     HIPCHK(hipMalloc(&h.d_dev, sizeof(ucg::DevNet)));   // the descriptor the kernels read (final values)
     h.allocs.push_back(h.d_dev);
     HIPCHK(hipMemcpy(h.d_dev, &N, sizeof(ucg::DevNet), hipMemcpyHostToDevice));
-    HIPCHK(hipStreamCreateWithFlags(&h.cancel_stream, hipStreamNonBlocking));   // last: nothing fails after it
+    HIPCHK(hipHostMalloc((void **)&h.cancel, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));   // last: nothing fails after it
+    *h.cancel = 0;
     return 0;
 }
 
@@ -1072,7 +1071,7 @@ int ucg_network_free(int handle)
             return fail(UCG_E_ARG, "close the network's request queues first");
     for (void *p : h->allocs) (void)hipFree(p);
     if (h->ws) (void)hipFree(h->ws);
-    if (h->cancel_stream) (void)hipStreamDestroy(h->cancel_stream);
+    if (h->cancel) (void)hipHostFree(h->cancel);
     *h = NetHandle();
     return 0;
 }
@@ -1083,7 +1082,6 @@ int ucg_cancel(int handle)
     // cancel does not wait behind a host-buffer solve that holds it for its whole run
     std::lock_guard<std::mutex> ck(g_cancel_mu);
     int *word;
-    hipStream_t stream;
     int gen;
     {
         std::lock_guard<std::mutex> lk(g_mu);
@@ -1091,12 +1089,10 @@ int ucg_cancel(int handle)
         if (!h) return fail(UCG_E_HANDLE, "bad network handle");
         if (h->gen <= h->cancel_sent) return 0;   // nothing launched since the last cancel
         word = h->cancel;
-        stream = h->cancel_stream;
         gen = h->gen;
         h->cancel_sent = gen;
     }
-    HIPCHK(hipMemcpyAsync(word, &gen, sizeof(int), hipMemcpyHostToDevice, stream));
-    HIPCHK(hipStreamSynchronize(stream));
+    __atomic_store_n(word, gen, __ATOMIC_RELEASE);
     return 0;
 }
 
