@@ -55,3 +55,36 @@ def test_terms_divided_by_the_mantle(name, oracle_of):
         assert np.all(err <= nfac[m] * U * (1 + 1e-6)), (q, float((err / (nfac[m] * U)).max()))
         checked += int(m.sum())
     assert checked > 300
+
+
+def test_co_photodissociation_at_the_table_edges(tables, oracle):
+    """kc = 2e-10 (G0 / 1.7) 10^s with s a table entry: the quotient and the products by 2e-10, by the
+    shielding and by the dust's 1 (exact) round once each, the power of ten is good to 2u."""
+    from uclchem_amd import gpu
+    from uclchem_amd.params import INDEX
+    t = tables
+    net = gpu.Network(t)
+    P, PH, Y, R = _states(t, oracle, 200, 9)
+    rng = np.random.default_rng(3)
+    # shielding table: [log N(CO) 12..18][log N(H2) 18..23], the 42 entries the reference's spline sees
+    corner = {(0, 0): 0.0, (1, 0): -2.760, (0, 1): -1.676, (1, 1): -3.888}
+    want = np.zeros(len(P), dtype=LD)
+    for q in range(len(P)):
+        co, h2 = q % 2, (q // 2) % 2
+        PH[q, 3] = 0.0                                       # Av: no dust
+        PH[q, 4] = 1e19
+        Y[q, -1] = 1e4
+        Y[q, t.scalars["nh2"]] = 1e-2 if h2 else 1e-8        # N(H2) = 5e20 ... 5e14: set to the edges below
+        Y[q, t.scalars["nco"]] = 1e-3 if co else 1e-13
+        if h2:
+            PH[q, 4] = 1e22                                  # N(H2) = 5e23, beyond the last knot
+            Y[q, t.scalars["nco"]] = 1e-6 if co else 1e-16   # N(CO) = 5e19 or 5e9
+        P[q, INDEX["radfield"]] = 10 ** rng.uniform(0, 3)
+        s = corner[(co, h2)]
+        want[q] = LD(2.0e-10) * (LD(P[q, INDEX["radfield"]]) / LD(float(np.float32(1.7)))) * LD(10) ** LD(s)
+    _, rate = net.rhs(P, PH, R, Y)
+    kc = rate[:, int(t.scalars["nR_CO_hv"])]
+    err = (np.abs(kc - want) / want).astype(float)
+    print("[photo] CO at the table's corners, worst error in u by corner:",
+          [round(float(err[k::4].max() / U), 2) for k in range(4)], flush=True)
+    assert np.all(err <= 5 * U * (1 + 1e-6))

@@ -325,9 +325,9 @@ __device__ inline double co_photodiss_dev(double nh2col, double ncocol, double r
 
 // Both photodissociation rates at up to four column pairs by one wave: each row of 16 lanes takes
 // the columns its lanes were given (equal within a row) and every lane of the row returns the
-// rates.  The chain of the functions above is cut to one logarithm and one exponential: the lanes
-// of a row evaluate the two columns' logarithms and the H2 optical depth's together, then the
-// scattering terms, the H2 shielding power and the CO shielding power together; the spline knots
+// rates.  The chain of the functions above is cut to one logarithm, one exponential and one power:
+// the lanes of a row evaluate the two columns' logarithms together, then the scattering terms, then
+// the shielding powers of H2 and CO; the spline knots
 // are one apart (12..18 and 18..23), so intervals come from comparisons and the natural spline's
 // tridiagonal system has constant factors; the dust wavelength is clamped to the first knots.
 // Table entries are selected by value: chosen by computed address the tables went through scratch
@@ -358,11 +358,10 @@ __device__ __forceinline__ void photo_rates_wave(double h2col, double cocol, dou
     }
     const double sc_c = c_scat[l & 7][0], sc_k = c_scat[l & 7][1];
     const double taud = 0.5 * h2col * (double)1.5e-2f * 1.0e-2 / (1.0 / (1000.0 * 1.0e-8));
-    const double larg = l == 0 ? h2col + 1.0 : l == 1 ? cocol + 1.0 : l == 2 ? fabs(h2col) + 1.0
-                      : l == 3 ? fabs(cocol) + 1.0 : taud;
+    const double larg = l == 0 ? h2col + 1.0 : l == 1 ? cocol + 1.0 : l == 2 ? fabs(h2col) + 1.0 : fabs(cocol) + 1.0;
     const double lg = log10(larg);
     double lognh2 = row16_bcast<0>(lg), lognco = row16_bcast<1>(lg);
-    const double lw = row16_bcast<2>(lg), lu = row16_bcast<3>(lg), ltau = row16_bcast<4>(lg);
+    const double lw = row16_bcast<2>(lg), lu = row16_bcast<3>(lg);
     if (lognco < 12.0) lognco = 12.0;
     if (lognh2 < 18.0) lognh2 = 18.0;
     if (lognco > 18.0) lognco = 18.0;
@@ -428,12 +427,14 @@ __device__ __forceinline__ void photo_rates_wave(double h2col, double cocol, dou
         if (xl < 0.0) xl = 0.0;
         tl = (av / 1.086) * xl;
     }
-    // one exponential: scattering terms (lanes 0..5), H2 shielding (6), CO shielding (7)
-    constexpr double LN10 = 2.302585092994045684;
+    // one exponential: scattering terms (lanes 0..5), H2 shielding of thin columns (6); one power: H2
+    // shielding of thick ones (6), CO shielding (7).  The powers as exponentials of scaled logarithms
+    // saved 0.4 us an RHS and were less accurate (CO rate at the table's corners: errors up to 8.6
+    // units of 2^-53, 2.6 with the power)
     const double p = taud < 10.0 ? -1.25 : taud < 100.0 ? -1.15 : -1.0667;
-    const double earg = l == 6 ? (taud < 2.0 ? -0.6666667 * taud : p * ltau * LN10) : l == 7 ? s * LN10 : -(sc_k * tl);
-    const double ex = exp(earg);
-    const double term = (l < 6 && -earg >= 100.0) ? 0.0 : (l < 6 ? sc_c * ex : ex);
+    const double earg = l == 6 ? -0.6666667 * taud : -(sc_k * tl);
+    const double ex = exp(earg), pw = pow(l == 7 ? 10.0 : taud, l == 7 ? s : p);
+    const double term = l < 6 ? (-earg >= 100.0 ? 0.0 : sc_c * ex) : (l == 6 && taud < 2.0) ? ex : pw;
     const double t0 = row16_bcast<0>(term);
     double scat = row16_bcast<1>(term);
     scat = scat + row16_bcast<2>(term);
