@@ -132,7 +132,9 @@ def rates_to_dy_and_flux(physics: np.ndarray, abundances: np.ndarray, rates: np.
     a = tables.arrays
     ab = abundances.reshape(n, -1)
     # what the terms change of the surface as a whole, before the bulk<->surface transfer
-    surface = flux @ inc[:, np.asarray(a["surface_list"], dtype=int)].sum(axis=1)
+    # (species by species: summed over the terms at once, what cancels between the species comes in
+    # the order of the reactions, and the sum's relative error doubled)
+    surface = (flux @ inc[:, np.asarray(a["surface_list"], dtype=int)]).sum(axis=1)
     ysurf, ybulk = ab[:, tables.scalars["nsurface"]], ab[:, tables.scalars["nbulk"]]
     pairs = _swap_pairs(tables)
     geo = np.zeros((n, 2 * len(pairs)))
