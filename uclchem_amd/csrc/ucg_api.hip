@@ -742,21 +742,20 @@ int ucg_network_load_file(const char *path, int *handle)
     return ucg_network_load(&d, handle);
 }
 
-// The staged form of the sparse plan, when its tail fits the workgroup's registers and its working
-// set the device's LDS; otherwise the plan runs from the workspace (nw_stage = 0).
-static int load_staged_plan(const ucg_network_desc *d, NetHandle &h, size_t lds_limit)
+// Plans the staged form and takes its sizes into N, N.nw_stage among them; 0: this form cannot be
+// built or does not fit the device's LDS, and the plan runs from the workspace.
+static void size_staged_plan(const ucg_network_desc *d, ucg::DevNet &N, size_t lds_limit, bool whole_blocks,
+                             ucg::SparsePrograms &S)
 {
-    ucg::DevNet &N = h.dev;
-    N.nw_stage = 0;
     std::vector<int> foff((size_t)d->nreac + 1, 0);
     for (int k = 0; k < d->nreac; k++) foff[k + 1] = foff[k] + d->nfac[k];
-    ucg::SparsePrograms S;
+    N.nw_stage = 0;
     try {
-        S = ucg::build_sparse_programs(d, ucg::NWAVE, ucg::GJ_MAX, foff, foff.back());
+        S = ucg::build_sparse_programs(d, ucg::NWAVE, ucg::GJ_MAX, foff, foff.back(), whole_blocks);
     } catch (const std::exception &) {   // a pattern the planner cannot follow: run the given schedule
         S.ok = false;
     }
-    if (!S.ok) return 0;
+    if (!S.ok || S.schur.size() > ucg::WIDE_PANELS) return;
     N.px = ucg::partial_slots(foff.back(), N.nswt, d->nswap, d->nsurfl);
     N.sp_ns = S.ns;
     N.sp_T = S.t;
@@ -770,13 +769,22 @@ static int load_staged_plan(const ucg_network_desc *d, NetHandle &h, size_t lds_
     // operands' place (their values wait)
     N.sp_w0 = S.wide ? std::max(0, ucg::WIDE_COLS * ucg::WIDE_LD - S.at_L) : std::max(N.px.n, S.t * S.t - S.at_L);
     N.sp_panels = (int)S.schur.size();
-    if (N.sp_panels > ucg::WIDE_PANELS) return 0;
     N.sp_presum = S.presum ? 1 : 0;
     N.nw_stage = S.wide ? 2 : 1;
-    if (lds_bytes(N) > lds_limit) {
-        N.nw_stage = 0;
-        return 0;
-    }
+    if (lds_bytes(N) > lds_limit) N.nw_stage = 0;
+}
+
+// The staged form of the sparse plan, when its tail fits the workgroup's registers and its working
+// set the device's LDS, if need be without filling the tail's last block (250/2500 network, tail of
+// 125 rows: 147 us a step in FP64 and 178 in FP32 from the workspace, 44 and 44 staged; before tails
+// took whole blocks 163 and 158, staged); otherwise the plan runs from the workspace.
+static int load_staged_plan(const ucg_network_desc *d, NetHandle &h, size_t lds_limit)
+{
+    ucg::DevNet &N = h.dev;
+    ucg::SparsePrograms S;
+    size_staged_plan(d, N, lds_limit, true, S);
+    if (N.nw_stage == 0 && S.ok && !S.wide) size_staged_plan(d, N, lds_limit, false, S);
+    if (N.nw_stage == 0) return 0;
     int rc;
     if ((rc = upload(h, S.stream.data(), S.stream.size(), N.sp_stream)) ||
         (rc = upload(h, S.part_wave.data(), S.part_wave.size(), N.sp_part_wave)) ||

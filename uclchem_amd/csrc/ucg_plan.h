@@ -234,8 +234,10 @@ struct EntryItem {
 constexpr int WIDE_ROWS = 128, WIDE_COLS = 64, WIDE_LD = 130, WIDE_PANELS = 8;
 
 // One network's tables as the planner reads them (the fields of ucg_network_desc it needs).
+// `whole_blocks`: the tail may take more rows than the plan gives it.
 template <class Desc>
-SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, const std::vector<int> &fac_off, int npart)
+SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, const std::vector<int> &fac_off, int npart,
+                                     bool whole_blocks = true)
 {
     SparsePrograms S;
     const int neq = d->neq, NN = d->nw_sizes[0], ns0 = d->nw_sizes[1], T0 = d->nw_sizes[2], nsp0 = d->nw_sizes[3];
@@ -243,8 +245,10 @@ SparsePrograms build_sparse_programs(const Desc *d, int nwave, int max_tail, con
     S.wide = T0 > max_tail;
     if (S.wide) max_tail *= 2;
     // the tail fills whole 16-row blocks: the rows up to the next block cost its inversion nothing
-    // and leave the sparse pivots with fewer levels
-    const int T = std::min(std::min((T0 + 15) / 16 * 16, max_tail), NN), ns = NN - T;
+    // and leave the sparse pivots with fewer levels.  They cost LDS, though: up to 15 rows and columns
+    // of up to 128 doubles, 13.8 KB with the default network's tail, so that a plan which fits
+    // without them is built without them if it does not fit with them.
+    const int T = whole_blocks || S.wide ? std::min(std::min((T0 + 15) / 16 * 16, max_tail), NN) : T0, ns = NN - T;
     S.ns = ns;
     S.t = T;
     if (S.wide && T % 16 != 0) return S;
