@@ -13,6 +13,7 @@
 // registers: rate and flux arrays [NREAC], the RHS input/output and solve vectors
 // [NEQ], and each thread's slice of the Nordsieck history (registers).
 #include "ucg_device.h"
+#include "ucg_recip.h"
 #include "ucg_reduce.h"
 
 namespace ucg {
@@ -1316,22 +1317,13 @@ template <int R> __device__ __forceinline__ double rows_bcast(double v)
     return __hiloint2double((int)rows_bcast32<R>((unsigned)__double2hiint(v)),
                             (int)rows_bcast32<R>((unsigned)__double2loint(v)));
 }
-// 1/x by the hardware estimate and two Newton steps
-__device__ __forceinline__ double fast_rcp(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-    r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
-    r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
-    return r;
-}
 // one Gauss-Jordan step on a 16x16 block in the tile layout
 template <int K> __device__ __forceinline__ void gj16_steps(f64x4 &d, int g, int c, bool &bad)
 {
     if constexpr (K < 16) {
         const double rowk = rows_bcast<K & 3>(d[K >> 2]);   // a(K, c)
         const double piv = row16_bcast<K>(rowk);
-        bad |= !(piv == piv) || piv == 0.0 || isinf(piv);
-        const double q = fast_rcp(piv);
+        const double q = pivot_reciprocal(piv, __builtin_amdgcn_rcp(piv), bad);
         const double rq = (c == K) ? q : rowk * q;          // row K of the result
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -2185,8 +2177,9 @@ __device__ __forceinline__ void eliminate(NetRef N, Slices<uint2, 2> &run, LDS d
             if (h & HDR_VALID) {
                 double v = W[h & HDR_INDEX] - s;
                 if (h & HDR_RECIP) {
-                    if (!(v == v) || v == 0.0 || isinf(v)) red[9] = 1.0;
-                    v = fast_rcp(v);
+                    bool bad = false;
+                    v = pivot_reciprocal(v, __builtin_amdgcn_rcp(v), bad);
+                    if (bad) red[9] = 1.0;
                 }
                 W[h & HDR_INDEX] = v;
             }
