@@ -56,3 +56,21 @@ def test_solves_with_a_partly_filled_block(edge, lu_bits):
     assert np.all(out["status"] == 0) and np.all(dense["status"] == 0)
     m = dense["y"][:, :t.nspec] > 1e-14
     assert (np.abs(out["y"] - dense["y"])[:, :t.nspec][m] / dense["y"][:, :t.nspec][m]).max() < 0.01
+
+
+@pytest.mark.parametrize("size,tail", [((150, 1500), 16), ((220, 5000), None), ((500, 6000), 300)])
+def test_workspace_form_takes_no_more_lds_than_its_arrays(size, tail):
+    """The partials with two scratch vectors, four vectors of the state's length, 40 doubles of
+    reduction slots and scalars and the parameters: what a network needs for the device to take it
+    (the limit is a CU's LDS) must not grow beyond that."""
+    from test_gpu_plan_forms import W, _with_tail
+    from uclchem_amd import gpu
+    from uclchem_amd.params import NPARAM
+    t = _network(*size)
+    if tail is not None:
+        t = _with_tail(t, tail)
+    form, lds = gpu.Network(t).plan_form()
+    assert form == W
+    pad = lambda n: (n + 7) & ~7
+    npart = int(t.arrays["nfac"].sum())
+    assert lds <= 8 * (max(t.nreac + 1, pad(npart) + 2 * pad(t.neq)) + 4 * pad(t.neq) + 40 + NPARAM)

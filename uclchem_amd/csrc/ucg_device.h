@@ -173,7 +173,7 @@ template <class Net>
 __host__ __device__ inline int flux_region_len(const Net &N)
 {
     const int npad = (N.neq + 7) & ~7, Npad = (N.nw_N + 7) & ~7;
-    const int a = N.npart_pad + 2 * npad;
+    const int a = N.npart_pad + npad;                // the partials and a scratch vector
     const int b0 = N.nreac + 1 > a ? N.nreac + 1 : a;
     const int b1 = b0 > 3 * Npad ? b0 : 3 * Npad;
     const int b = b1 > NT ? b1 : NT;                 // >= one value per thread (ordered_sum)

@@ -12,7 +12,9 @@
 
 namespace ucg {
 
-enum { RED_TS, RED_S, RED_TOTALS, RED_CHARGE, RED_EWT, RED_ACOR, RED_CORR, RED_HIST, RED_ORDER, RED_NBUF };
+// a value a wave; the reductions of two values have two buffers, one after the other
+enum { RED_TS, RED_S, RED_TOTALS, RED_TOTALS_2, RED_CHARGE, RED_EWT, RED_EWT_2, RED_ACOR, RED_CORR, RED_HIST, RED_ORDER,
+       RED_NBUF };
 
 // The integrator's reductions (bdf_core.h's Ops).
 struct OpsBuffers {

@@ -139,10 +139,10 @@ __device__ __forceinline__ double wave_max0(double v)   // v >= 0
 // (ucg_reduce.h says when two may share one), every wave adds all of them.
 constexpr int RED_FLAGS = 16;                                   // red[0..15]: flags and small scratch
 constexpr int RED_CANCEL = 10;                                  // the flag of cancel_poll
-constexpr int RED_LEN = RED_FLAGS + RED_NBUF * 2 * NWAVE;
+constexpr int RED_LEN = RED_FLAGS + RED_NBUF * NWAVE;
 __device__ __forceinline__ double block_sum(double v, LDS double *red, int id)
 {
-    LDS double *buf = red + RED_FLAGS + id * 2 * NWAVE;
+    LDS double *buf = red + RED_FLAGS + id * NWAVE;
     v = wave_sum(v);
     if ((tid() & 63) == 0) buf[tid() >> 6] = v;
     __syncthreads();
@@ -153,7 +153,7 @@ __device__ __forceinline__ double block_sum(double v, LDS double *red, int id)
 }
 __device__ __forceinline__ void block_sum2(double &a, double &b, LDS double *red, int id)
 {
-    LDS double *buf = red + RED_FLAGS + id * 2 * NWAVE;
+    LDS double *buf = red + RED_FLAGS + id * NWAVE;
     a = wave_sum(a);
     b = wave_sum(b);
     if ((tid() & 63) == 0) {
@@ -172,7 +172,7 @@ __device__ __forceinline__ void block_sum2(double &a, double &b, LDS double *red
 }
 __device__ __forceinline__ double block_max0(double v, LDS double *red, int id)   // v >= 0
 {
-    LDS double *buf = red + RED_FLAGS + id * 2 * NWAVE;
+    LDS double *buf = red + RED_FLAGS + id * NWAVE;
     v = wave_max0(v);
     if ((tid() & 63) == 0) buf[tid() >> 6] = v;
     __syncthreads();
@@ -843,7 +843,7 @@ UCG_BIG __device__ void block_newton_matrix(NetRef N, const Lds L, LUT *M, doubl
     const int neq = N.neq, ld = N.ld;
     LDS double *y = L.y, *sc = L.sc, *g = L.g;
     double *rate = L.rate;
-    LDS double *scr = L.flux + N.npart_pad;   // scratch [>= 2*neq] beside the partials
+    LDS double *scr = L.flux + N.npart_pad, *gts = L.b;   // scratch [neq]: beside the partials; a free vector
     const double D = y[neq - 1];
     const double ysur = y[N.nsurface], ybulk = y[N.nbulk];
     const double sm = fmax(1e-30, ysur), sbk = fmax(1e-30, ybulk);
@@ -879,15 +879,15 @@ UCG_BIG __device__ void block_newton_matrix(NetRef N, const Lds L, LUT *M, doubl
             u += N.sw_c[q] * w;
         }
         scr[i] = u;
-        scr[neq + i] = 0.0;
+        gts[i] = 0.0;
     }
     __syncthreads();
     if (tid() == 0) {
         for (int q = 0; q < N.nswap; q++) {
             const int k = N.swap_list[q];
-            scr[neq + N.ops[MAXOPS * k]] += rate[k] * blr;
+            gts[N.ops[MAXOPS * k]] += rate[k] * blr;
         }
-        scr[neq + N.nbulk] = (blr < 1.0 && ybulk > 1e-30) ? -TS / sbk : 0.0;
+        gts[N.nbulk] = (blr < 1.0 && ybulk > 1e-30) ? -TS / sbk : 0.0;
     }
     __syncthreads();
     for (int idx = tid(); idx < neq * (N.nbulkl + 1); idx += NT) {
@@ -895,7 +895,7 @@ UCG_BIG __device__ void block_newton_matrix(NetRef N, const Lds L, LUT *M, doubl
         const double u = scr[i];
         if (u == 0.0) continue;
         const int b = (q < N.nbulkl) ? N.bulk_list[q] : N.nbulk;
-        const double gb = scr[neq + b];
+        const double gb = gts[b];
         if (gb != 0.0) M[(size_t)b * ld + i] = (LUT)((double)M[(size_t)b * ld + i] + u * gb);
     }
     __syncthreads();
@@ -1644,7 +1644,7 @@ UCG_BIG __device__ void sparse_jacobian(NetRef N_, const Lds L, double *V)
     const int neq = N.neq;
     LDS double *y = L.y, *sc = L.sc;
     double *rate = L.rate;
-    LDS double *scr = L.flux + N.npart_pad;   // scratch [>= 2*neq] beside the partials
+    LDS double *scr = L.flux + N.npart_pad, *gts = L.b;   // scratch [neq]: beside the partials; a free vector
     const double D = y[neq - 1];
     const double ysur = y[N.nsurface], ybulk = y[N.nbulk];
     const double sm = fmax(1e-30, ysur), sbk = fmax(1e-30, ybulk);
@@ -1683,17 +1683,17 @@ UCG_BIG __device__ void sparse_jacobian(NetRef N_, const Lds L, double *V)
             u += N.sw_c[q] * w;
         }
         scr[i] = u;
-        scr[neq + i] = 0.0;
+        gts[i] = 0.0;
     }
     __syncthreads();
     // g1 = d totalSwap / dy: one BULKSWAP per bulk species, so the targets are distinct
     // (checked when the network is loaded) and the sums need no ordering
     for (int q = tid(); q < N.nswap; q += NT) {
         const int k = glb(N.swap_list)[q];
-        scr[neq + glb(N.ops)[MAXOPS * k]] += glb(rate)[k] * blr;
+        gts[glb(N.ops)[MAXOPS * k]] += glb(rate)[k] * blr;
     }
     __syncthreads();
-    if (tid() == 0) scr[neq + N.nbulk] = (blr < 1.0 && ybulk > 1e-30) ? -TS / sbk : 0.0;
+    if (tid() == 0) gts[N.nbulk] = (blr < 1.0 && ybulk > 1e-30) ? -TS / sbk : 0.0;
     __syncthreads();
     // 2. border rows and columns, constant sum rows
     for (int j = tid(); j < neq; j += NT) {
@@ -1704,7 +1704,7 @@ UCG_BIG __device__ void sparse_jacobian(NetRef N_, const Lds L, double *V)
             V[r2] = acc;
         }
         const int r1 = N.nw_s1r[j];
-        if (r1 >= 0) V[r1] = -scr[neq + j];
+        if (r1 >= 0) V[r1] = -gts[j];
         const int cc = N.nw_s1c[j];
         if (cc >= 0) V[cc] = scr[j];
     }

@@ -321,13 +321,13 @@ def lds_bytes(tables, staged: bool = True) -> int:
     N, T, nsp = int(z[0]), (int(z[2]) + 15) & ~15, int(z[3])
     npad = (tables.neq + 7) & ~7
     npart = int(a["nfac"].sum())
-    b = max(tables.nreac + 1, ((npart + 7) & ~7) + 2 * npad, 3 * ((N + 7) & ~7), 512)
+    b = max(tables.nreac + 1, ((npart + 7) & ~7) + npad, 3 * ((N + 7) & ~7), 512)
     if staged:
         tail = T * T if T <= 128 else 128 * 130
         gj = (2 * (min(T, 128) // 16 + 1) + 1) * 16 * 17
         b = max(b, (npart if T <= 128 else 64 * 130) + nsp, tail, gj)
     from .params import NPARAM
-    return 8 * (b + ((tables.neq + 4 + 7) & ~7) + 3 * npad + 160 + 40 + NPARAM)   # + reduction slots, scalars, parameters
+    return 8 * (b + ((tables.neq + 4 + 7) & ~7) + 3 * npad + 104 + 40 + NPARAM)   # + reduction slots, scalars, parameters
 
 
 def schur_sources(tables) -> int:
