@@ -179,8 +179,10 @@ int ucg_network_plan(int handle, int *form, int *lds);
  *   n_rec   [n] rows written; status [n] UCLCHEM success flag per point
  *   stats   [n][8] steps, f-evals, Newton-matrix setups, Newton iterations,
  *           convergence failures, error-test failures, intervals, integrator retries
- *   lu_bits 64: FP64 Newton-matrix factorisation; 32: FP32 factorisation with the FP64
- *           residual (every Newton iterate is re-evaluated in FP64).
+ *   lu_bits 64: FP64 factors of the Newton matrix; 32: factors stored and applied in FP32 with
+ *           the FP64 residual (every Newton iterate is re-evaluated in FP64).  A staged plan
+ *           forms and factors the matrix in FP64 either way; a plan run from the workspace and
+ *           the dense form factor it in lu_bits.
  * Returns when all points are done.  It waits for the whole device, so while a request
  * queue's kernel runs (ucg_queue_open) use ucg_solve_batch_device on a stream instead. */
 int ucg_solve_batch(int handle, int n, const double *params, const double *y_init, double *y_out,

@@ -541,7 +541,7 @@ static int check_plan(const ucg_network_desc *d)
         nph < 1 || nphs < 0 || ngs < 0)
         return bad("inconsistent sizes");
     if (T > 0 && NN - ns > ucg::NT * ucg::EPT) return bad("tail too large");
-    // the unstaged tail's blocked LU keeps its 16x16 block factors in the NEQ-long work vectors
+    // plans with a dense tail are taken from 57 equations on; no buffer here needs that any more
     if (T > 0 && ((d->neq + 7) & ~7) < 64) return bad("network too small for the dense tail");
     auto in = [](const int *a, long n, long lo, long hi) {   // every a[i] in [lo, hi)
         if (n > 0 && !a) return false;

@@ -93,6 +93,11 @@ struct DevProg {
     const uint32_t *hdr, *rec;
 };
 constexpr int NWAVE = NT / 64;
+constexpr int GJ_MAX = 16 * NWAVE;        // rows of a tail one workgroup's waves can hold
+constexpr int GJ_TILE = 16 * 17;          // LDS tile, column-major, column stride 17 (bank spread)
+// LDS doubles of the exchange buffers of a tail's inversion: two generations of inverse + panel,
+// the next pivot block
+__host__ __device__ inline int gj_stage_len(int n) { return (2 * ((n + 15) / 16 + 1) + 1) * GJ_TILE; }
 
 struct DevNet {
     int32_t nspec, neq, nreac, nice, nsurfl, nbulkl, nfp, nswap, nnz, ld;
@@ -183,7 +188,7 @@ __host__ __device__ inline int flux_region_len(const Net &N)
         const int m = WIDE_ROWS * WIDE_LD, e = c > m ? c : m;
         return b > e ? b : e;
     }
-    const int gj = (2 * ((N.sp_T + 15) / 16 + 1) + 1) * 16 * 17, tt = N.sp_T * N.sp_T;
+    const int gj = gj_stage_len(N.sp_T), tt = N.sp_T * N.sp_T;
     const int e0 = c > gj ? c : gj;
     const int e = e0 > tt ? e0 : tt;
     return b > e ? b : e;

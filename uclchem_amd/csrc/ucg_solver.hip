@@ -8,10 +8,13 @@
 // rates frozen per interval attempt, a cold-start BDF integration per interval with
 // DVODE's ITASK=1 contract, the retry policy, the 1e-30 clamp and the physics update.
 //
-// Memory layout per workgroup slot: the dense Newton matrix (column-major, leading
-// dimension ld) in HBM (FP64 or FP32, template LUT), everything else in LDS or
-// registers: rate and flux arrays [NREAC], the RHS input/output and solve vectors
-// [NEQ], and each thread's slice of the Nordsieck history (registers).
+// Memory layout.  A workgroup's slot in HBM holds the rate coefficients [NREAC] and the Newton
+// system (FP64 or FP32, template LUT): the factors of a staged plan in the order its solves read
+// them, beside the matrix entries that wait for their panel of the tail; or all values of a plan
+// that runs from the workspace, and their J-form; or the dense matrix (column-major, leading
+// dimension ld).  In LDS: a region that the fluxes, the term partials, a staged plan's elimination
+// and the solve's vectors share, the state, the RHS and two vectors of its length, reduction slots,
+// scalars and parameters.  In registers: each thread's slice of the Nordsieck history.
 #include "ucg_device.h"
 #include "ucg_recip.h"
 #include "ucg_reduce.h"
@@ -1019,6 +1022,7 @@ UCG_BIG __device__ void block_newton_matrix(NetRef N, const Lds L, LUT *M, doubl
 #define UCG_LU_NB 16
 #endif
 constexpr int LU_NB = UCG_LU_NB;
+static_assert(NT >= 2 * LU_NB * LU_NB, "the shared region holds a value a thread; the block factors need this many");
 
 // Right-looking blocked LU of the column-major n x n matrix M (unit lower L, upper U
 // stored in place).  Per block column: the 16x16 diagonal block is factored by wave 0 in
@@ -1298,12 +1302,7 @@ UCG_BIG __device__ int block_lu_tiled(MP M, int n, int ld, LDS double *red, LDS 
 // 2 n^3 FLOP at FP64 on one CU.  A sweep is 3.7 us, of which the inversion of the next pivot block
 // (16 dependent steps) is 2.4: alone it takes 1.6, but FP64 vector instructions and the FP64 MFMAs
 // of the column wave on the same SIMD share one unit.
-constexpr int GJ_MAX = 16 * NWAVE;        // rows one workgroup's waves can hold
-constexpr int GJ_TILE = 16 * 17;          // LDS tile, column-major, column stride 17 (bank spread)
 using f64x4 = __attribute__((ext_vector_type(4))) double;
-
-// LDS doubles of the exchange buffers: two generations of inverse + panel, the next pivot block
-__host__ __device__ inline int gj_stage_len(int n) { return (2 * ((n + 15) / 16 + 1) + 1) * GJ_TILE; }
 
 template <int R> __device__ __forceinline__ unsigned rows_bcast32(unsigned v)
 {   // row R of 16 lanes, to all four rows
@@ -1823,13 +1822,10 @@ UCG_BIG __device__ void sparse_form_newton(NetRef N_, const double *J, LUT *V, d
     }
 }
 
-// Crout elimination of the sparse pivots in plan phases (one thread per target entry,
-// dependencies only on earlier phases), then the trailing block (its Schur complement):
-// inverted in place by blocked Gauss-Jordan when the plan is staged, LU-factored when it
-// is not.  The sparse factors stay in the workspace in their precision (LUT); a staged
-// plan's tail, with the Schur-update sources, is worked on in LDS (region) in the same
-// precision (the FP32 form does its whole factorisation in FP32: the Newton iteration's FP64
-// residuals absorb the difference) and stored back.  stage: 512 doubles of LDS.
+// A plan run from the workspace: Crout elimination of the sparse pivots and the tail's Schur
+// update in plan phases (one thread per target entry, dependencies only on earlier phases), in
+// place and in the factors' precision (with LUT float the whole factorisation is FP32: the Newton
+// iteration's FP64 residuals absorb the difference).
 template <typename LUT, typename WP>
 __device__ __forceinline__ void crout_phases(NetRef N, WP W, LDS double *red, int nph)
 {
@@ -2400,7 +2396,10 @@ __device__ __forceinline__ void staged_solve(NetRef N_, const Lds &L, const LUT 
         apply(0, 1, x2, [&](int r, double s) { x1[r] -= s; });
     } else
     {   // four lanes a row of the tail's inverse, each every fourth column, in two chains (one chain
-        // over the columns fetched ahead took 0.3 us more a step: 43.9 against 43.5)
+        // over the columns fetched ahead took 0.3 us more a step: 43.9 against 43.5).  The last two
+        // columns of an even number go to the first chain: an order as good as pairs to the end, and
+        // as fast; the two differ in the last bits, by which a grid point of storms (3086 of the 4096)
+        // ends far from or near to the reference's answer, as it does with any change of rounding.
         double p0 = 0.0, p1 = 0.0;
 #pragma unroll
         for (int q = 0; q < TAIL_AHEAD; q += 2) {

@@ -305,51 +305,3 @@ def plan_summary(plan) -> Dict[str, int]:
     s["values"] = s["nsp"] + s["T"] * s["T"]
     s["tail_lu_mads"] = s["T"] ** 3 // 3
     return s
-
-
-LDS_BYTES_PER_CU = 160 * 1024
-
-
-def lds_bytes(tables, staged: bool = True) -> int:
-    """LDS one solve workgroup needs.  With staged=False (plans that run from the workspace, and the
-    dense form) this is the library's size: fluxes or Jacobian term partials, the NEQ-long vectors,
-    reduction slots, scalars and parameters.  For a staged plan it is an upper estimate: partials
-    and sparse factors side by side, the dense tail (a panel of it beyond 128 rows), or the exchange
-    buffers of its inversion; the library's planner gives slots only to values that meet there."""
-    a = tables.arrays
-    z = a["nw_sizes"]
-    N, T, nsp = int(z[0]), (int(z[2]) + 15) & ~15, int(z[3])
-    npad = (tables.neq + 7) & ~7
-    npart = int(a["nfac"].sum())
-    b = max(tables.nreac + 1, ((npart + 7) & ~7) + npad, 3 * ((N + 7) & ~7), 512)
-    if staged:
-        tail = T * T if T <= 128 else 128 * 130
-        gj = (2 * (min(T, 128) // 16 + 1) + 1) * 16 * 17
-        b = max(b, (npart if T <= 128 else 64 * 130) + nsp, tail, gj)
-    from .params import NPARAM
-    return 8 * (b + ((tables.neq + 4 + 7) & ~7) + 3 * npad + 104 + 40 + NPARAM)   # + reduction slots, scalars, parameters
-
-
-def schur_sources(tables) -> int:
-    """Distinct sparse factor entries the last elimination phase reads when that phase is
-    the pure Schur-complement update of the dense tail (0 otherwise); the library gathers
-    them into LDS beside the staged tail."""
-    a = tables.arrays
-    nsp, nph = int(a["nw_sizes"][3]), int(a["nw_sizes"][7])
-    ph, tp = a["nw_ph_ptr"], a["nw_tg_ptr"]
-    if nph < 2:
-        return 0
-    t0, t1 = int(ph[nph - 1]), int(ph[nph])
-    q0, q1 = int(tp[t0]), int(tp[t1])
-    if q1 <= q0 or (a["nw_tg_slot"][t0:t1] < nsp).any() or (a["nw_tg_div"][t0:t1] >= 0).any():
-        return 0
-    refs = np.concatenate([a["nw_pr_l"][q0:q1], a["nw_pr_u"][q0:q1]])
-    if (refs >= nsp).any():
-        return 0
-    return int(len(np.unique(refs)))
-
-
-def plan_is_staged(tables) -> bool:
-    """Whether the library is sure to stage this network's plan in LDS (else it may run it from the
-    workspace): the tail fits the registers of the waves that invert it (256 rows), the estimate LDS."""
-    return lds_bytes(tables, True) <= LDS_BYTES_PER_CU and int(tables.arrays["nw_sizes"][2]) <= 256
