@@ -176,7 +176,7 @@ int ucg_network_plan(int handle, int *form, int *lds);
  *   y_out   [n][neq] final state (abundances + density)
  *   rec     [n][max_rec][4+nspec] output rows (time yr, density, gasTemp, Av, abundances)
  *           like the reference's physicsarray/chemicalabunarray, or NULL with max_rec=0
- *   n_rec   [n] rows written; status [n] UCLCHEM success flag per point
+ *   n_rec   [n] rows written (rows of rec from there on are undefined); status [n] UCLCHEM success flag per point
  *   stats   [n][8] steps, f-evals, Newton-matrix setups, Newton iterations,
  *           convergence failures, error-test failures, intervals, integrator retries
  *   lu_bits 64: FP64 factors of the Newton matrix; 32: factors stored and applied in FP32 with

@@ -591,8 +591,8 @@ __device__ __forceinline__ double term_of(NetRef N, int k, double r, const LDS d
 // run the same instructions; one wave evaluates the photo rates meanwhile and one forms totalSwap
 // and the terms that carry it.  Sums: one slice program over the signed production and loss terms
 // of each species, whose records do not depend on the state.  Ice transfer and totals: one wave.
-// Bound by the LDS gathers and the latency of the three parts: 6.8 us a call (default
-// network; 6.2 with 150 species), against 17.5 for chunked sums with a second pass over the
+// Bound by the LDS gathers and the latency of the three parts: 7.0 us a call (default
+// network; 5.2 with 150 species), against 17.5 for chunked sums with a second pass over the
 // chunks, workgroup-wide reductions for each total and serial photo-rate splines.
 __device__ __forceinline__ void block_rhs(NetRef N_, const Lds L)
 {
@@ -2518,7 +2518,7 @@ struct GpuOps {
     int gen = 0;                  // this launch's generation
     int polls = 0;
     // the load of the cancel word bypasses the caches and takes microseconds: a staged plan, whose
-    // steps take 33 to 112 us, reads it at every 16th step, the slower forms at every step
+    // steps take 34 to 105 us, reads it at every 16th step, the slower forms at every step
     __device__ __forceinline__ bool cancelled()
     {
         return cancel_poll(
